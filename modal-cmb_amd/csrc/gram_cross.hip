@@ -27,9 +27,10 @@
 // primordial modes (the q3 rows of l1, l2 and the 16 l3 values staged in LDS
 // per x-chunk; the mode's pair sums of the l1, l2 rows shared by the four
 // points of a thread) and another z Q_m for the late modes; a split-K FP64
-// MFMA GEMM contracts them over the points.  GL form: M by a tiled GEMM over
-// l per (p, q), then per 64 x 64 tile of (m, n) the node sum with M staged in
-// LDS 8 nodes at a time, x outermost.
+// MFMA GEMM contracts them over the points.  GL form: M by an FP64 MFMA GEMM
+// over l per (p, q), then the node sums through the core tensor of M's
+// functions (cx_core, cx_gather), or for few modes of a wide basis per 64 x 64
+// tile of (m, n) with M staged in LDS 8 nodes at a time, x outermost.
 #include "mcmb_internal.h"
 #include "weights.h"
 #include <algorithm>
@@ -350,74 +351,317 @@ __global__ void cx_reduce(const double* __restrict__ P, int nsplit, long MN, dou
 }
 
 // ---- Gauss-Legendre form ---------------------------------------------------
+//
+// The rule is symmetric, so the tables hold the nodes mu >= 0 only (half of
+// them, padded with zero weights to SH, a multiple of 8): P_l(-mu) = (-1)^l
+// P_l(mu), and a sum over l splits into its even and odd part E, O with M(+mu)
+// = E + O, M(-mu) = E - O.  M[x][f][k], f = p Rq + q, holds +mu at k = s and
+// -mu at k = SH + s; the middle node of an odd rule sits at both with half its
+// weight.
 
-// Pt[l][s] = TTw(l) P_l(mu_s) for lmin <= l <= lmax, 0 below lmin.
-__global__ __launch_bounds__(256) void cx_legendre(const double* __restrict__ mu, int npt, int lmin, int lmax,
-                                                   const double* __restrict__ tw, double* __restrict__ Pt)
+// P[l][s] = P_l(mu_s), l <= lmax, s < SH (0 for s >= half).  One wave per 64
+// nodes; the recurrence as P_l = t + (l-1)/l (t - P_{l-2}), t = mu P_{l-1}:
+// three dependent operations per step (its coefficients formed beforehand, CK
+// at a time) instead of a division, and a smaller rounding error than the
+// three-term form, whose products are 2l times as large as P_l.  0.107 ->
+// 0.036 ms at lmax 500, 751 nodes (a serial chain: latency, not throughput).
+constexpr int CX_CK = 512;
+__global__ __launch_bounds__(64) void cx_legendre(const double* __restrict__ mu, int half, int SH, int lmax,
+                                                  double* __restrict__ P)
 {
-    const int s = blockIdx.x * 256 + threadIdx.x;
-    if (s >= npt) return;
-    const double xs = mu[s];
-    double p0 = 1.0, p1 = xs;
-    for (int l = 0; l <= lmax; ++l) {
-        double pl;
-        if (l == 0) pl = 1.0;
-        else if (l == 1) pl = xs;
-        else {
-            pl = ((2.0 * l - 1.0) * xs * p1 - (l - 1.0) * p0) / l;
+    __shared__ double cf[CX_CK];
+    const int s = blockIdx.x * 64 + threadIdx.x;
+    const double xs = s < half ? mu[s] : 0.0;
+    double p0 = 1.0, p1 = xs;   // P_{l-2}, P_{l-1}
+    if (s < SH) {
+        P[s] = s < half ? 1.0 : 0.0;
+        if (lmax >= 1) P[SH + s] = xs;
+    }
+    for (int l0 = 2; l0 <= lmax; l0 += CX_CK) {
+        const int nl = min(CX_CK, lmax - l0 + 1);
+        __syncthreads();
+        for (int e = threadIdx.x; e < nl; e += 64) cf[e] = (double)(l0 + e - 1) / (double)(l0 + e);
+        __syncthreads();
+#pragma unroll 4
+        for (int e = 0; e < nl; ++e) {
+            const double t = xs * p1, pl = fma(cf[e], t - p0, t);
             p0 = p1;
             p1 = pl;
+            if (s < SH) P[(long)(l0 + e) * SH + s] = s < half ? pl : 0.0;
         }
-        Pt[(long)l * npt + s] = l >= lmin ? tw[l] * pl : 0.0;
     }
 }
 
-// M[x][p][q][s] = sum_{l = lmin..lmax} qt[p][l][x] b_q(l) Pt[l][s]; one
-// workgroup per (64 nodes, 32 samples of x, pair (p, q)), K = l in steps of 16.
-__global__ __launch_bounds__(256) void cx_mgemm(const double* __restrict__ qt, int nlq, int nx,
-                                                const double* __restrict__ b, int ldq, int Rq,
-                                                const double* __restrict__ Pt, int npt, int lmin, int lmax, int np,
-                                                double* __restrict__ M)
+// M[x][f][.] = sum over l in [lmin, lmax] of qt[p][l][x] tw(l) b_q(l) P_l(+-mu_s):
+// one workgroup per (64 nodes, 64 samples of x, f), wave w the nodes 16w..,
+// FP64 MFMA over l in stages of 16 (8 even, 8 odd: the two parities have
+// accumulators of their own, which halves the products).  0.92 (VALU, all
+// nodes) -> 0.22 ms at lmax 500, 100 functions, 100 samples.
+__global__ __launch_bounds__(256, 2) void cx_mgemm(const double* __restrict__ qt, int nlq, int nx,
+                                                   const double* __restrict__ b, int ldq, int Rq,
+                                                   const double* __restrict__ P, const double* __restrict__ tw,
+                                                   int SH, int lmin, int lmax, double* __restrict__ M)
 {
-    __shared__ double Ps[16][64 + 1], Qs[16][32 + 1];
-    const int s0 = blockIdx.x * 64, x0 = blockIdx.y * 32;
-    const int p = blockIdx.z / Rq, q = blockIdx.z % Rq;
-    const int ts = (threadIdx.x & 15) * 4, tx = (threadIdx.x >> 4) * 2;
-    double acc[4][2] = {};
-    const double* qp = qt + (long)p * nlq * nx;
-    for (int l0 = lmin; l0 <= lmax; l0 += 16) {
-        for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-            const int l = e / 64, s = e % 64;
-            Ps[l][s] = (l0 + l <= lmax && s0 + s < npt) ? b[(long)(l0 + l) * ldq + q] * Pt[(long)(l0 + l) * npt + s0 + s]
-                                                        : 0.0;
+    // rows of 72 doubles: the four k rows of a fragment (two l apart) start 32
+    // banks apart
+    __shared__ double Qs[2][16][72], Ps[2][16][72];
+    const int s0 = blockIdx.x * 64, x0 = blockIdx.y * 64, f = blockIdx.z;
+    const int p = f / Rq, q = f % Rq;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const double* const qp = qt + (long)p * nlq * nx;
+    const int lb = lmin & ~1;
+    d4 acc[2][4];
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[u][t] = d4{0.0, 0.0, 0.0, 0.0};
+    double rq[4], rp[4];
+    const int c = tid & 63, r0 = tid >> 6;   // column, rows r0, r0 + 4, ...
+    auto gload = [&](int l0) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int l = l0 + r0 + 4 * u;
+            const bool in = l >= lmin && l <= lmax;
+            rq[u] = in && x0 + c < nx ? qp[(long)l * nx + x0 + c] : 0.0;
+            rp[u] = in && s0 + c < SH ? (tw[l] * b[(long)l * ldq + q]) * P[(long)l * SH + s0 + c] : 0.0;
         }
-        for (int e = threadIdx.x; e < 16 * 32; e += 256) {
-            const int l = e / 32, x = e % 32;
-            Qs[l][x] = (l0 + l <= lmax && x0 + x < nx) ? qp[(long)(l0 + l) * nx + x0 + x] : 0.0;
+    };
+    auto sstore = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            Qs[buf][r0 + 4 * u][c] = rq[u];
+            Ps[buf][r0 + 4 * u][c] = rp[u];
         }
-        __syncthreads();
+    };
+    gload(lb);
+    sstore(0);
+    __syncthreads();
+    int buf = 0;
+    for (int l0 = lb; l0 <= lmax; l0 += 16, buf ^= 1) {
+        const bool more = l0 + 16 <= lmax;
+        if (more) gload(l0 + 16);
 #pragma unroll
-        for (int l = 0; l < 16; ++l) {
-            double a[4], c[2];
+        for (int ks = 0; ks < 2; ++ks)
 #pragma unroll
-            for (int u = 0; u < 4; ++u) a[u] = Ps[l][ts + u];
-            c[0] = Qs[l][tx];
-            c[1] = Qs[l][tx + 1];
+            for (int u = 0; u < 2; ++u) {
+                const int r = 8 * ks + 2 * (lane >> 4) + u;
+                const double bv = Ps[buf][r][16 * wave + (lane & 15)];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                acc[u][0] += a[u] * c[0];
-                acc[u][1] += a[u] * c[1];
+                for (int t = 0; t < 4; ++t)
+                    acc[u][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(Qs[buf][r][16 * t + (lane & 15)], bv, acc[u][t], 0,
+                                                                    0, 0);
             }
-        }
+        if (more) sstore(buf ^ 1);
         __syncthreads();
     }
+    const int s = s0 + 16 * wave + (lane & 15), F = gridDim.z;
+    if (s < SH)
 #pragma unroll
-    for (int u = 0; u < 4; ++u)
+        for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int v = 0; v < 2; ++v) {
-            const int s = s0 + ts + u, x = x0 + tx + v;
-            if (s < npt && x < nx) M[(((long)x * np + p) * Rq + q) * npt + s] = acc[u][v];
+            for (int v = 0; v < 4; ++v) {
+                const int x = x0 + 16 * t + 4 * v + (lane >> 4);
+                if (x < nx) {
+                    double* const o = M + ((long)x * F + f) * (2 * SH);
+                    o[s] = acc[0][t][v] + acc[1][t][v];
+                    o[SH + s] = acc[0][t][v] - acc[1][t][v];
+                }
+            }
+}
+
+// Node sums through the core tensor.  A permanent is a sum of six products of
+// three entries M_f, M_g, M_h, and (n_late n_prim) permanents hold each such
+// triple about once: so the triples themselves are contracted,
+//   H_u[f][g][h] = sum over the unit's samples x and nodes of w M_f M_g M_h,
+// a GEMM over nodes with A = (w M_b) M_a formed in registers, and cx_gather
+// adds the six entries per (m, n).  Samples x >= 10 enter linearly, so a unit
+// is a group of them (weights c_x x^2 folded in); each sample x < 10 is a unit
+// of its own, since its rule acts on y_x.  Against the sum of permanents per
+// (m, n) (bound by its nine LDS gathers a permanent): 274 -> 1.24 + 0.09 ms at
+// 220 x 220 modes, 100 functions, 100 samples of 751 nodes: 41 TFLOP/s on the
+// matrix cores, about half of it on triples (the rest repeats triples inside
+// the diagonal tiles or pads the last tile).
+//
+// Tiles of 16 functions.  SAME (one field): f <= g <= h, tile ta of a, one b
+// in tile tb >= ta, tiles tc >= tb of c, stored tile by tile (cx_tile).
+// Otherwise the pair (a, b) is of one field and c, any tile, of the other.
+// One workgroup per (tb, ta, four tiles of c): wave w has b = 16 tb + 4w ..+3,
+// 16 accumulator tiles, per K-step of 4 nodes 16 MFMAs on 9 LDS reads.
+__host__ __device__ __forceinline__ int cx_jobs(int tb, int NTC, bool same)
+{
+    return (tb + 1) * ((NTC - (same ? tb : 0) + 3) / 4);
+}
+// tiles before the first of b-tile tb
+__host__ __device__ __forceinline__ long cx_base(int tb, int NTC, bool same)
+{
+    long o = 0;
+    for (int t = 0; t < tb; ++t) o += 16l * (t + 1) * (NTC - (same ? t : 0));
+    return o;
+}
+__device__ __forceinline__ long cx_tile(long base, int ta, int b, int tc, int NTC, bool same)
+{
+    const int tb = b >> 4, lo = same ? tb : 0;
+    return base + (long)((b & 15) * (tb + 1) + ta) * (NTC - lo) + (tc - lo);
+}
+
+// Samples of unit u: the ng groups of g samples from nm on, then the nm single ones.
+__device__ __forceinline__ int cx_unit(int u, int nm, int ng, int g, int nx, int* n)
+{
+    if (u >= ng) {
+        *n = 1;
+        return u - ng;
+    }
+    *n = min(g, nx - nm - u * g);
+    return nm + u * g;
+}
+
+template <bool SAME>
+__global__ __launch_bounds__(256, 2) void cx_core(const double* __restrict__ MA, int FA, const double* __restrict__ MC,
+                                                  int FC, int K, const double* __restrict__ wk,
+                                                  const double* __restrict__ sc, int nm, int ng, int g, int nx, int u0,
+                                                  double* __restrict__ H, long us)
+{
+    __shared__ double S[2][96][17];   // 16 a, 16 b, 64 c rows of 16 nodes
+    __shared__ double Ws[2][16];
+    const int NTC = (FC + 15) >> 4;
+    int tb = 0, job = blockIdx.x;
+    for (int nj; job >= (nj = cx_jobs(tb, NTC, SAME)); ++tb) job -= nj;
+    const int ta = job % (tb + 1), tc0 = (SAME ? tb : 0) + 4 * (job / (tb + 1)), nct = min(4, NTC - tc0);
+    int nxu;
+    const int xb = cx_unit(u0 + blockIdx.y, nm, ng, g, nx, &nxu);
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int b0 = 16 * tb + 4 * wave;
+    const bool live = b0 < FA;
+    d4 acc[4][4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) acc[r][t] = d4{0.0, 0.0, 0.0, 0.0};
+    // the six elements a thread stages: row e >> 4, node e & 15
+    const double* src[6];
+    double rs[6], rw = 0.0;
+    const int kk = tid & 15;
+#pragma unroll
+    for (int u = 0; u < 6; ++u) {
+        const int row = (tid >> 4) + 16 * u;
+        const int f = u == 0 ? 16 * ta + row : u == 1 ? 16 * tb + row - 16 : 16 * tc0 + row - 32;
+        src[u] = u < 2 ? (f < FA ? MA + ((long)xb * FA + f) * K + kk : nullptr)
+                       : (f < FC ? MC + ((long)xb * FC + f) * K + kk : nullptr);
+    }
+    const int nk = K / 16;
+    int lx = 0, lk = 0;   // sample and stage of the next load
+    auto gload = [&]() {
+        const long oa = (long)lx * FA * K + 16l * lk, oc = (long)lx * FC * K + 16l * lk;
+#pragma unroll
+        for (int u = 0; u < 6; ++u) rs[u] = src[u] ? src[u][u < 2 ? oa : oc] : 0.0;
+        if (tid < 16) rw = wk[16 * lk + kk] * sc[xb + lx];
+        if (++lk == nk) {
+            lk = 0;
+            ++lx;
         }
+    };
+    auto sstore = [&](int buf) {
+#pragma unroll
+        for (int u = 0; u < 6; ++u) S[buf][(tid >> 4) + 16 * u][kk] = rs[u];
+        if (tid < 16) Ws[buf][kk] = rw;
+    };
+    gload();
+    sstore(0);
+    __syncthreads();
+    const int nst = nxu * nk;
+    for (int st = 0; st < nst; ++st) {
+        const int buf = st & 1;
+        if (st + 1 < nst) gload();
+        if (live)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const int k = 4 * ks + (lane >> 4), col = lane & 15;
+                const double ma = S[buf][col][k], w = Ws[buf][k];
+                double mb[4], mc[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) mb[r] = ma * (S[buf][16 + 4 * wave + r][k] * w);
+#pragma unroll
+                for (int t = 0; t < 4; ++t) mc[t] = S[buf][32 + 16 * t + col][k];
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+                    if (t < nct)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r)
+                            acc[r][t] = __builtin_amdgcn_mfma_f64_16x16x4f64(mb[r], mc[t], acc[r][t], 0, 0, 0);
+            }
+        if (st + 1 < nst) sstore(buf ^ 1);
+        __syncthreads();
+    }
+    if (!live) return;
+    double* const Hu = H + (long)blockIdx.y * us;
+    const long base = cx_base(tb, NTC, SAME);
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (b0 + r < FA && t < nct) {
+                double* const o = Hu + cx_tile(base, ta, b0 + r, tc0 + t, NTC, SAME) * 256;
+#pragma unroll
+                for (int v = 0; v < 4; ++v) o[16 * (4 * v + (lane >> 4)) + (lane & 15)] = acc[r][t][v];
+            }
+}
+
+// Gamma[m][n] (+)= scale * sum over the units u0 .. u0 + nu of their part of
+// the x integral: the six entries of H_u of the matchings of m's and n's
+// indices (late slot b with index q_b reads its field's function p R + q_b);
+// of a single sample x < 10 y = x^2 (their sum), zeroed when |y| > 1e-18,
+// times c_x.  KIND 0: one field; 1: TTE, 2: TEE (the pair of H's field is T T,
+// E E).  Units are added in order.
+template <int KIND>
+__global__ __launch_bounds__(256) void cx_gather(const double* __restrict__ H, long us, int FP, int FS, int RP, int RS,
+                                                 int nm, int ng, int u0, int nu, const double* __restrict__ xv,
+                                                 const double* __restrict__ cx, const int* __restrict__ mlate, int nl,
+                                                 const int* __restrict__ mprim, int npm, double scale, int accumulate,
+                                                 double* __restrict__ out)
+{
+    __shared__ long base[64];
+    const int NTC = (FS + 15) >> 4, NTB = (FP + 15) >> 4;
+    if (threadIdx.x < NTB) base[threadIdx.x] = cx_base(threadIdx.x, NTC, KIND == 0);
+    __syncthreads();
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (long)nl * npm) return;
+    const int qm = mlate[e / npm], pn = mprim[e % npm];
+    const int q[3] = {qm & 255, (qm >> 8) & 255, (qm >> 16) & 255};
+    const int p[3] = {pn & 255, (pn >> 8) & 255, (pn >> 16) & 255};
+    constexpr int P6[6][3] = {{0, 1, 2}, {0, 2, 1}, {1, 0, 2}, {1, 2, 0}, {2, 0, 1}, {2, 1, 0}};
+    long at[6];
+#pragma unroll
+    for (int j = 0; j < 6; ++j) {
+        int a, b, c;
+        if (KIND == 0) {
+            const int u = p[P6[j][0]] * RP + q[0], v = p[P6[j][1]] * RP + q[1], w = p[P6[j][2]] * RP + q[2];
+            a = min(u, min(v, w));
+            c = max(u, max(v, w));
+            b = u + v + w - a - c;
+        } else {
+            const int s0 = KIND == 1 ? 0 : 1, s1 = KIND == 1 ? 1 : 2, s2 = KIND == 1 ? 2 : 0;
+            const int u = p[P6[j][s0]] * RP + q[s0], v = p[P6[j][s1]] * RP + q[s1];
+            a = min(u, v);
+            b = max(u, v);
+            c = p[P6[j][s2]] * RS + q[s2];
+        }
+        at[j] = cx_tile(base[b >> 4], a >> 4, b, c >> 4, NTC, KIND == 0) * 256 + 16 * (a & 15) + (c & 15);
+    }
+    double tot = accumulate ? out[e] : 0.0, sum = 0.0;
+    for (int k = 0; k < nu; ++k) {
+        const double* const h = H + (long)k * us;
+        double t = 0.0;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) t += h[at[j]];
+        if (u0 + k >= ng) {
+            const int x = u0 + k - ng;
+            t *= xv[x] * xv[x];
+            if (fabs(t) > 1e-18) t = 0.0;
+            t *= cx[x];
+        }
+        sum += t;
+    }
+    out[e] = tot + scale * sum;
 }
 
 // Gamma[m][n] for late modes m (rows, q indices) and primordial modes n
@@ -883,52 +1127,116 @@ static int cross_gl_launch(mcmb_ctx* c, int pol, int spline, int npt, double* ds
             }
         }
     }
-    DevBuf d_mu, d_w, d_cw, d_tw[2], d_Pt[2], d_M[2];
-    MCMB_TRY(d_mu.alloc(sizeof(double) * npt));
-    MCMB_TRY(d_w.alloc(sizeof(double) * npt));
-    MCMB_TRY(d_cw.alloc(sizeof(double) * nx));
-    MCMB_HIP(hipMemcpyAsync(d_mu.p, mu, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
-    MCMB_HIP(hipMemcpyAsync(d_w.p, w, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
-    MCMB_HIP(hipMemcpyAsync(d_cw.p, cw.data(), sizeof(double) * nx, hipMemcpyHostToDevice, c->stream));
-    for (int f = 0; f < 2; ++f) {
-        if (R[f] == 0) continue;
-        MCMB_TRY(d_tw[f].alloc(sizeof(double) * tw[f].size()));
-        MCMB_TRY(d_Pt[f].alloc(sizeof(double) * (size_t)(hi[f] + 1) * npt));
-        MCMB_TRY(d_M[f].alloc(sizeof(double) * (size_t)nx * np * R[f] * npt));
-        MCMB_HIP(hipMemcpyAsync(d_tw[f].p, tw[f].data(), sizeof(double) * tw[f].size(), hipMemcpyHostToDevice,
-                                c->stream));
+    // the half table of nodes and weights, and the x weights of the samples
+    // that enter linearly (cx_core)
+    const int half = (npt + 1) / 2, SH = (half + 7) & ~7, K = 2 * SH, lmaxP = std::max(hi[0] * (R[0] > 0), hi[1] * (R[1] > 0));
+    const int nm = std::min(10, nx);
+    std::vector<double> host((size_t)3 * SH + 2 * (size_t)nx + (lmaxP + 1) * 2, 0.0);
+    double *const h_mu = host.data(), *const h_w = h_mu + SH, *const h_cw = h_w + K, *const h_sc = h_cw + nx,
+                  *const h_tw = h_sc + nx;
+    for (int s = 0; s < half; ++s) {
+        const int i = npt / 2 + s;   // the middle node of an odd rule first
+        h_mu[s] = mu[i];
+        h_w[s] = h_w[SH + s] = (npt & 1) && s == 0 ? 0.5 * w[i] : w[i];
     }
+    for (int x = 0; x < nx; ++x) {
+        h_cw[x] = cw[x];
+        h_sc[x] = x < nm ? 1.0 : cw[x] * (X.xvec[x] * X.xvec[x]);
+    }
+    for (int f = 0; f < 2; ++f)
+        if (R[f]) std::copy(tw[f].begin(), tw[f].end(), h_tw + (size_t)f * (lmaxP + 1));
+    // the field of H's pair and of its third function (one field: the same)
+    const int fp = pol == 0 || pol == 1 ? 0 : 1, fs = pol == 0 || pol == 2 ? 0 : 1;
+    const bool same = fp == fs;
+    const int F[2] = {np * R[0], np * R[1]}, NTP = (F[fp] + 15) / 16, NTS = (F[fs] + 15) / 16;
+    const long us = cx_base(NTP, NTS, same) * 256;   // H of one unit
+    long jobs = 0;
+    for (int t = 0; t < NTP; ++t) jobs += cx_jobs(t, NTS, same);
+    // The core tensor costs us multiply-adds a node on the matrix cores (about
+    // 2e13/s), the sum of permanents n_late n_prim permanents (1.3e10/s
+    // measured): the tensor wherever it is cheaper by a margin, which complete
+    // mode tables always are; few modes of a wide basis keep the permanents.
+    const bool tensor = us <= 1000l * nlate * nprim;
+    // groups of linear samples: about 1536 workgroups (three rounds of the two
+    // that a CU holds), at least one group
+    const int nlin = nx - nm;
+    const int want = (int)std::max<long>(1, (1536 + jobs - 1) / jobs - nm);
+    const int g = nlin > 0 ? (nlin + std::min(nlin, want) - 1) / std::min(nlin, want) : 1;
+    const int ng = nlin > 0 ? (nlin + g - 1) / g : 0, nunit = ng + nm;
+    // H is held for as many units at a time as 1 GiB takes (at least one)
+    const int ub = (int)std::max<long>(1, std::min<long>(nunit, ((long)1 << 27) / std::max(1l, us)));
+    size_t off[6], total = host.size();
+    for (int f = 0; f < 2; ++f) {
+        off[f] = total;
+        total += R[f] ? ((size_t)nx * F[f] * K + 1 & ~(size_t)1) : 0;
+    }
+    off[2] = total;
+    total += (size_t)(lmaxP + 1) * SH;
+    off[3] = total;
+    if (tensor) total += (size_t)ub * us;
+    MCMB_TRY(c->cx_ws.alloc(sizeof(double) * total));
+    double* const ws = c->cx_ws.as<double>();
+    double *const d_mu = ws, *const d_w = d_mu + SH, *const d_cw = d_w + K, *const d_sc = d_cw + nx,
+                  *const d_tw = d_sc + nx, *const d_P = ws + off[2], *const d_H = ws + off[3];
+    double* const d_M[2] = {ws + off[0], ws + off[1]};
+    MCMB_HIP(hipMemcpyAsync(ws, host.data(), sizeof(double) * host.size(), hipMemcpyHostToDevice, c->stream));
     MCMB_HIP(hipEventRecord(c->ev0, c->stream));
     const double* bq[2] = {L.d_q.as<double>(), E.d_q.as<double>()};
     const double* qsrc[2] = {X.d_qt.as<double>(), X.d_qc.as<double>()};
-    int launches = 0;
+    int launches = 1;
+    hipLaunchKernelGGL(cx_legendre, dim3((SH + 63) / 64), dim3(64), 0, c->stream, (const double*)d_mu, half, SH, lmaxP,
+                       d_P);
     for (int f = 0; f < 2; ++f) {
         if (R[f] == 0) continue;
-        hipLaunchKernelGGL(cx_legendre, dim3((npt + 255) / 256), dim3(256), 0, c->stream, d_mu.as<double>(), npt,
-                           lo[f], hi[f], d_tw[f].as<double>(), d_Pt[f].as<double>());
-        hipLaunchKernelGGL(cx_mgemm, dim3((npt + 63) / 64, (nx + 31) / 32, np * R[f]), dim3(256), 0, c->stream,
-                           qsrc[f], X.lq + 1, nx, bq[f], ldb[f], R[f], d_Pt[f].as<double>(), npt, lo[f], hi[f], np,
-                           d_M[f].as<double>());
-        launches += 2;
+        hipLaunchKernelGGL(cx_mgemm, dim3((SH + 63) / 64, (nx + 63) / 64, F[f]), dim3(256), 0, c->stream, qsrc[f],
+                           X.lq + 1, nx, bq[f], ldb[f], R[f], (const double*)d_P,
+                           (const double*)(d_tw + (size_t)f * (lmaxP + 1)), SH, lo[f], hi[f], d_M[f]);
+        ++launches;
     }
-    const unsigned tiles = (unsigned)(((nlate + 63) / 64) * ((nprim + 63) / 64));
     const double scale = X.dphi * X.dphi / (8.0 * M_PI);
     const int* ml = pol == 0 ? L.d_modes.as<int>() : E.d_modes[pol - 1].as<int>();
-    if (pol == 0 || pol == 3) {
-        const int f = pol == 0 ? 0 : 1;
-        hipLaunchKernelGGL(cx_gl_gamma, dim3(tiles), dim3(256), 0, c->stream, (const double*)d_M[f].as<double>(), np,
-                           R[f], nx, npt, d_w.as<double>(), X.d_x.as<double>(), d_cw.as<double>(), ml, nlate,
-                           X.d_modes.as<int>(), nprim, scale, dst);
-    } else if (pol == 1) {
-        hipLaunchKernelGGL(cx_gl_gamma_mixed<1>, dim3(tiles), dim3(256), 0, c->stream,
-                           (const double*)d_M[0].as<double>(), R[0], (const double*)d_M[1].as<double>(), R[1], np, nx,
-                           npt, d_w.as<double>(), X.d_x.as<double>(), d_cw.as<double>(), ml, nlate,
-                           X.d_modes.as<int>(), nprim, scale, dst);
+    if (tensor) {
+        const long nmn = (long)nlate * nprim;
+        MCMB_TRY(launch_guard("GL cross-Gamma core", (unsigned long long)jobs, 256));
+        MCMB_TRY(launch_guard("GL cross-Gamma", (unsigned long long)((nmn + 255) / 256), 256));
+        for (int u0 = 0; u0 < nunit; u0 += ub) {
+            const int nu = std::min(ub, nunit - u0);
+            const dim3 grid((unsigned)jobs, (unsigned)nu), gather((unsigned)((nmn + 255) / 256));
+#define CX_CORE(SAME)                                                                                             \
+    hipLaunchKernelGGL(cx_core<SAME>, grid, dim3(256), 0, c->stream, (const double*)d_M[fp], F[fp],               \
+                       (const double*)d_M[fs], F[fs], K, (const double*)d_w, (const double*)d_sc, nm, ng, g, nx, u0, \
+                       d_H, us)
+#define CX_GATHER(KIND)                                                                                           \
+    hipLaunchKernelGGL(cx_gather<KIND>, gather, dim3(256), 0, c->stream, (const double*)d_H, us, F[fp], F[fs],    \
+                       R[fp], R[fs], nm, ng, u0, nu, X.d_x.as<double>(), (const double*)d_cw, ml, nlate,          \
+                       X.d_modes.as<int>(), nprim, scale, u0 > 0 ? 1 : 0, dst)
+            if (same) {
+                CX_CORE(true);
+                CX_GATHER(0);
+            } else {
+                CX_CORE(false);
+                if (pol == 1) CX_GATHER(1);
+                else CX_GATHER(2);
+            }
+#undef CX_CORE
+#undef CX_GATHER
+            launches += 2;
+        }
     } else {
-        hipLaunchKernelGGL(cx_gl_gamma_mixed<2>, dim3(tiles), dim3(256), 0, c->stream,
-                           (const double*)d_M[0].as<double>(), R[0], (const double*)d_M[1].as<double>(), R[1], np, nx,
-                           npt, d_w.as<double>(), X.d_x.as<double>(), d_cw.as<double>(), ml, nlate,
-                           X.d_modes.as<int>(), nprim, scale, dst);
+        const unsigned tiles = (unsigned)(((nlate + 63) / 64) * ((nprim + 63) / 64));
+        if (same)
+            hipLaunchKernelGGL(cx_gl_gamma, dim3(tiles), dim3(256), 0, c->stream, (const double*)d_M[fp], np, R[fp], nx,
+                               K, (const double*)d_w, X.d_x.as<double>(), (const double*)d_cw, ml, nlate,
+                               X.d_modes.as<int>(), nprim, scale, dst);
+        else if (pol == 1)
+            hipLaunchKernelGGL(cx_gl_gamma_mixed<1>, dim3(tiles), dim3(256), 0, c->stream, (const double*)d_M[0], R[0],
+                               (const double*)d_M[1], R[1], np, nx, K, (const double*)d_w, X.d_x.as<double>(),
+                               (const double*)d_cw, ml, nlate, X.d_modes.as<int>(), nprim, scale, dst);
+        else
+            hipLaunchKernelGGL(cx_gl_gamma_mixed<2>, dim3(tiles), dim3(256), 0, c->stream, (const double*)d_M[0], R[0],
+                               (const double*)d_M[1], R[1], np, nx, K, (const double*)d_w, X.d_x.as<double>(),
+                               (const double*)d_cw, ml, nlate, X.d_modes.as<int>(), nprim, scale, dst);
+        ++launches;
     }
     MCMB_HIP(hipGetLastError());
     MCMB_HIP(hipEventRecord(c->ev1, c->stream));
@@ -936,7 +1244,8 @@ static int cross_gl_launch(mcmb_ctx* c, int pol, int spline, int npt, double* ds
     float ms = 0.f;
     MCMB_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;
-    c->last_launches = launches + 1;
+    c->last_launches = launches;
+    if (c->cx_ws.bytes > ((size_t)2 << 30)) c->cx_ws.release();   // kept between calls up to 2 GiB
     return MCMB_OK;
 }
 

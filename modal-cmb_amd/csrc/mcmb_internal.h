@@ -306,6 +306,8 @@ struct mcmb_ctx {
     mcmb::TrdWork trd;
     // the GL Gram over the compressed basis: node table and Phi
     mcmb::DevBuf gl_xw;
+    // the GL cross-Gamma: node tables, M and the core tensor
+    mcmb::DevBuf cx_ws;
     // the last Gauss-Legendre rule the Grams asked for (gl_nodes)
     std::vector<double> gl_x, gl_w;
 };

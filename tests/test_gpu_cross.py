@@ -96,6 +96,30 @@ def test_cross_gl_vs_oracle(ctx, spline, kw):
     assert relmax(G, ref) < 1e-12
 
 
+@pytest.mark.parametrize("R,npb,nx,tlmax,late,prim", [
+    (8, 9, 30, 40, None, None),      # 72 functions: five 16-function tiles, two groups of c tiles
+    (4, 4, 9, 40, None, None),       # every sample under the rule on x < 10
+    (4, 5, 10, 39, None, None),      # no linear sample; odd and even node counts
+    (3, 11, 11, 38, None, None),     # one linear sample; 33 functions
+    (8, 9, 14, 40, 3, 2),            # few modes of a wide basis: the sum of permanents
+    (1, 1, 12, 40, None, None),      # one function
+])
+def test_cross_gl_core_tensor_edges(ctx, R, npb, nx, tlmax, late, prim):
+    """The node sums through the core tensor of the (p, q) functions where its
+    tiles, sample groups and single samples end, and the permanents that few
+    modes keep.  1e-12: FP64 sums of the same terms in another order, as in
+    the tests above."""
+    c = case(tlmax=tlmax, R=R, npb=npb, nx=nx, seed=R + nx)
+    if late:
+        c["order_late"], c["order_prim"] = c["order_late"][-late:], c["order_prim"][:prim]
+    setup(ctx, c)
+    G = ctx.gamma_cross_gl(modalcmb.SPLINE_NATURAL)
+    ref = O.gamma_cross_gl(c["tlmin"], c["tlmax"], c["b"], c["order_late"], c["qt"], c["xvec"], c["order_prim"],
+                           c["cl"], c["nl"], c["bl"], c["dphi"], spline=modalcmb.SPLINE_NATURAL)
+    assert relmax(G, ref) < 1e-12
+    assert np.array_equal(G, ctx.gamma_cross_gl(modalcmb.SPLINE_NATURAL))
+
+
 def test_legacy_cross_entry_points(ctx):
     lib = modalcmb.load_library()
     c = case()
