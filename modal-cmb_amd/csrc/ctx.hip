@@ -277,6 +277,7 @@ int mcmb_destroy(mcmb_ctx* c)
     c->d_aux.release();
     tridiag_release(c);
     if (c->stage) (void)hipHostFree(c->stage);
+    if (c->gn_gate) (void)hipHostFree(c->gn_gate);
     for (int k = 0; k < 2; ++k)
         if (c->stage_ev[k]) (void)hipEventDestroy(c->stage_ev[k]);
     for (int h = 0; h < 2; ++h)

@@ -1,0 +1,89 @@
+// Double-double arithmetic (an unevaluated sum hi + lo of two doubles, about
+// 106 bits) from the error-free transformations of Dekker and Knuth.
+// Contraction is off: the error terms depend on the exact operation order.
+#pragma once
+#include <hip/hip_runtime.h>
+
+namespace mcmb {
+
+struct dd {
+    double hi, lo;
+};
+
+// s + e = a + b exactly (two_sum), for |a| >= |b| (quick_two_sum)
+__device__ __forceinline__ dd two_sum(double a, double b)
+{
+#pragma clang fp contract(off)
+    const double s = a + b, t = s - a;
+    return dd{s, (a - (s - t)) + (b - t)};
+}
+__device__ __forceinline__ dd quick_two_sum(double a, double b)
+{
+#pragma clang fp contract(off)
+    const double s = a + b;
+    return dd{s, b - (s - a)};
+}
+__device__ __forceinline__ dd two_prod(double a, double b)
+{
+#pragma clang fp contract(off)
+    const double p = a * b;
+    return dd{p, __builtin_fma(a, b, -p)};
+}
+__device__ __forceinline__ dd operator+(dd a, dd b)
+{
+#pragma clang fp contract(off)
+    const dd s = two_sum(a.hi, b.hi), t = two_sum(a.lo, b.lo);
+    const dd u = quick_two_sum(s.hi, s.lo + t.hi);
+    return quick_two_sum(u.hi, u.lo + t.lo);
+}
+__device__ __forceinline__ dd operator-(dd a) { return dd{-a.hi, -a.lo}; }
+__device__ __forceinline__ dd operator-(dd a, dd b) { return a + (-b); }
+__device__ __forceinline__ dd operator*(dd a, dd b)
+{
+#pragma clang fp contract(off)
+    const dd p = two_prod(a.hi, b.hi);
+    return quick_two_sum(p.hi, __builtin_fma(a.lo, b.hi, __builtin_fma(a.hi, b.lo, p.lo)));
+}
+__device__ __forceinline__ dd operator*(double a, dd b)
+{
+#pragma clang fp contract(off)
+    const dd p = two_prod(a, b.hi);
+    return quick_two_sum(p.hi, __builtin_fma(a, b.lo, p.lo));
+}
+__device__ __forceinline__ dd operator/(dd a, dd b)
+{
+#pragma clang fp contract(off)
+    const double q = a.hi / b.hi;
+    const dd r = a - q * b;
+    const double q2 = r.hi / b.hi;
+    const dd r2 = r - q2 * b;
+    return quick_two_sum(q, q2) + dd{r2.hi / b.hi, 0.0};
+}
+// acc += p + e with the rounding errors of the high parts collected in
+// acc.lo (compensated summation: acc is not renormalised until dd_renorm)
+__device__ __forceinline__ void dd_acc(dd& acc, double p, double e)
+{
+#pragma clang fp contract(off)
+    const dd s = two_sum(acc.hi, p);
+    acc.hi = s.hi;
+    acc.lo += s.lo + e;
+}
+// acc += a b, a double
+__device__ __forceinline__ void dd_mac(dd& acc, double a, dd b)
+{
+#pragma clang fp contract(off)
+    const double p = a * b.hi;
+    dd_acc(acc, p, __builtin_fma(a, b.lo, __builtin_fma(a, b.hi, -p)));
+}
+__device__ __forceinline__ void dd_mac(dd& acc, dd a, dd b)
+{
+#pragma clang fp contract(off)
+    const double p = a.hi * b.hi;
+    dd_acc(acc, p, __builtin_fma(a.lo, b.hi, __builtin_fma(a.hi, b.lo, __builtin_fma(a.hi, b.hi, -p))));
+}
+__device__ __forceinline__ dd dd_renorm(dd a) { return two_sum(a.hi, a.lo); }
+// (by components: a ?: of two dd selects an address, which keeps both in memory)
+__device__ __forceinline__ dd dd_sel(bool c, dd a, dd b) { return dd{c ? a.hi : b.hi, c ? a.lo : b.lo}; }
+__device__ __forceinline__ dd dd_shfl_xor(dd a, int o) { return dd{__shfl_xor(a.hi, o), __shfl_xor(a.lo, o)}; }
+
+}  // namespace mcmb

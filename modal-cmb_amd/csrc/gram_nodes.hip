@@ -1,0 +1,448 @@
+// The exact l-space Gram as a node sum over the compressed pair basis, in
+// double-double arithmetic.
+//
+// With int P_l1 P_l2 P_l3 = 2 (l1 l2 l3; 0 0 0)^2 the tetrapyd sum over the
+// basis columns (gram_sep.hip) is
+//   H[a][b][c] = (3 / 4 pi) sum_s w_s Phi_a Phi_b Phi_c(x_s),
+//   Phi_a(x)   = sum_l T[l][a] P_l(x),  T[l][a] = (2l + 1) v_l P[l][a],
+// exact with Gauss-Legendre nodes of degree 3 lmax: the selection rules of the
+// 3j symbols, which the tetrapyd's walk spells out point by point, come from
+// the orthogonality of the P_l.  The work falls from N_tet r + rows r^2
+// (lmax 2500, r = 59: 5e10 multiply-adds) to r L npt / 2 + r^3 npt / 6
+// (4.1e8), but the sum cancels: the terms the rules forbid are as large as
+// L^2 times the result, which is why the FP64 node sum (mcmb_gamma_gl) keeps
+// only ten digits.  So the nodes, P_l, Phi and the node sum are carried in
+// double-double (T, as in the tetrapyd order, is rounded once), and H is
+// rounded once at the end: at lmax 2500 it is within 2^-53 of the exact sum
+// of the rounded T.  gl_gate bounds the error for the weights at hand, and a
+// setup it does not pass takes the tetrapyd contraction.  Measured, core
+// tensor by the tetrapyd contraction -> as a node sum: lmax 2500, r = 59: 2.20
+// -> 0.29 ms; lmax 2000, r = 39: 1.22 -> 0.11 ms.
+//
+// Both parities of l are summed apart (P_l(-x) = (-1)^l P_l(x)), so the table
+// holds the nodes x >= 0 only, and the columns at +x and -x are E + O and
+// E - O.
+#include "dd.h"
+#include "mcmb_internal.h"
+#include <cmath>
+
+namespace mcmb {
+
+// cl[l] = (l - 1) / l for 2 <= l <= n
+__global__ void gl_coef(int n, dd* __restrict__ cl)
+{
+    const int l = blockIdx.x * 256 + threadIdx.x;
+    if (l <= n) cl[l] = l >= 2 ? dd{l - 1.0, 0.0} / dd{(double)l, 0.0} : dd{0.0, 0.0};
+}
+
+// Stages the coefficients l0 <= l < l0 + GN_CK of a recurrence in LDS.
+constexpr int GN_CK = 512;
+__device__ __forceinline__ int stage_coef(const dd* __restrict__ cl, int l0, int lmax, dd* sc)
+{
+    const int nl = min(GN_CK, lmax - l0 + 1);
+    __syncthreads();
+    for (int e = threadIdx.x; e < nl; e += 64) sc[e] = cl[l0 + e];
+    __syncthreads();
+    return nl;
+}
+
+// Nodes and weights of the rule of order n, x >= 0 ascending (the middle node
+// of an odd rule at s = 0 with half its weight: it is summed at +x and -x).
+// Newton's method in FP64 from the asymptotic root leaves x0 within an ulp;
+// P_n(x0) in double-double (the recurrence P_l = t + c_l (t - P_{l-2}), t = x
+// P_{l-1}) and the next Taylor term, from (1 - x^2) P'' = 2 x P' - n (n + 1)
+// P, make the step to a root good to 1e-32.  One thread per node: a serial
+// chain of n steps per evaluation (0.58 ms at 3751 nodes, once per rule).
+__global__ __launch_bounds__(64) void gl_rule(int n, int half, int SH, const dd* __restrict__ cl, dd* __restrict__ x,
+                                              dd* __restrict__ w)
+{
+#pragma clang fp contract(off)
+    __shared__ dd sc[GN_CK];
+    const int s = blockIdx.x * 64 + threadIdx.x;
+    const bool mid = (n & 1) && s == 0;
+    const int i = max(0, n - 1 - (n / 2 + s));   // from the largest root down (past half: the largest again)
+    double x0 = mid ? 0.0 : cos(M_PI * (4.0 * i + 3.0) / (4.0 * n + 2.0)) * (1.0 - (n - 1.0) / (8.0 * n * (double)n * n));
+    for (int it = 0; it < 3; ++it) {
+        double p0 = 1.0, p1 = x0;
+        for (int l0 = 2; l0 <= n; l0 += GN_CK) {
+            const int nl = stage_coef(cl, l0, n, sc);
+#pragma unroll 8
+            for (int e = 0; e < nl; ++e) {
+                const double t = x0 * p1, p = __builtin_fma(sc[e].hi, t - p0, t);
+                p0 = p1;
+                p1 = p;
+            }
+        }
+        const double step = mid ? 0.0 : p1 * (x0 * x0 - 1.0) / (n * (x0 * p1 - p0));
+        x0 -= step;
+        if (__all(fabs(step) < 1e-15)) break;
+    }
+    dd p0{1.0, 0.0}, p1{x0, 0.0};
+    for (int l0 = 2; l0 <= n; l0 += GN_CK) {
+        const int nl = stage_coef(cl, l0, n, sc);
+#pragma unroll 4
+        for (int e = 0; e < nl; ++e) {
+            const dd t = x0 * p1, p = t + sc[e] * (t - p0);
+            p0 = p1;
+            p1 = p;
+        }
+    }
+    const dd x0d{x0, 0.0}, nn{(double)n, 0.0};
+    const dd om = dd{1.0, 0.0} - two_prod(x0, x0);               // 1 - x0^2
+    const dd f1 = nn * (p0 - x0d * p1) / om;                       // P'
+    const dd f2 = (2.0 * (x0d * f1) - ((n * (n + 1.0)) * p1)) / om; // P''
+    const double u = p1.hi / f1.hi;                                // Newton step, to the second order
+    const double d = mid ? 0.0 : -u * (1.0 + 0.5 * u * (f2.hi / f1.hi));
+    const dd xr = quick_two_sum(x0, d);
+    // P' at the root: Taylor from x0 (P''' from the derivative of the equation)
+    const double f3 = (4.0 * x0 * f2.hi - ((double)n * (n + 1.0) - 2.0) * f1.hi) / om.hi;
+    const dd fr = f1 + d * f2 + dd{0.5 * d * d * f3, 0.0};
+    const dd omr = dd{1.0, 0.0} - xr * xr;
+    const dd wr = dd{mid ? 1.0 : 2.0, 0.0} / (omr * (fr * fr));
+    x[s] = dd_sel(s < half, xr, dd{0.0, 0.0});
+    w[s] = dd_sel(s < half, wr, dd{0.0, 0.0});
+}
+
+// P[l][s] = P_l(x_s), l <= lmax (0 past half); one thread per node (0.34 ms at
+// lmax 2500, a serial chain, once per rule).
+__global__ __launch_bounds__(64) void gl_ptab(int lmax, int half, int SH, const dd* __restrict__ cl,
+                                              const dd* __restrict__ x, dd* __restrict__ P)
+{
+    __shared__ dd sc[GN_CK];
+    const int s = blockIdx.x * 64 + threadIdx.x;
+    const bool in = s < half;
+    const dd zero{0.0, 0.0};
+    const dd xs = x[s];
+    dd p0{1.0, 0.0}, p1 = xs;
+    P[s] = dd_sel(in, p0, zero);
+    if (lmax >= 1) P[SH + s] = dd_sel(in, p1, zero);
+    for (int l0 = 2; l0 <= lmax; l0 += GN_CK) {
+        const int nl = stage_coef(cl, l0, lmax, sc);
+#pragma unroll 4
+        for (int e = 0; e < nl; ++e) {
+            const dd t = xs * p1, p = t + sc[e] * (t - p0);
+            p0 = p1;
+            p1 = p;
+            P[(long)(l0 + e) * SH + s] = dd_sel(in, p, zero);
+        }
+    }
+}
+
+// T[l][a] = (2l + 1) v_l P[l][a] for a < r, and the gate's column a = r, (2l +
+// 1) |v_l| max_a |P[l][a]|; 0 for lmin > l and for r < a < ldt.  One workgroup
+// per 32 l (Pc is stored by columns, T by rows).
+__global__ __launch_bounds__(256) void gl_ttab(const double* __restrict__ Pc, int nlp, int nl, int r, int lmin,
+                                               const double* __restrict__ v, int ldt, double* __restrict__ T)
+{
+    __shared__ double S[GN_RMAX][33];
+    const int l0 = blockIdx.x * 32, tl = threadIdx.x & 31;
+    for (int a = threadIdx.x >> 5; a < r; a += 8) S[a][tl] = l0 + tl < nl ? Pc[(long)a * nlp + l0 + tl] : 0.0;
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        double m = 0.0;
+        for (int a = 0; a < r; ++a) m = fmax(m, fabs(S[a][tl]));
+        S[r][tl] = m;
+    }
+    __syncthreads();
+    for (int e = threadIdx.x; e < 32 * ldt; e += 256) {
+        const int l = l0 + e / ldt, a = e % ldt;
+        if (l >= nl) break;
+        const double f = (2.0 * l + 1.0) * v[l];
+        T[(long)l * ldt + a] = (l < lmin || a > r) ? 0.0 : S[a][l - l0] * (a < r ? f : fabs(f));
+    }
+}
+
+// Phi[a][k] for CA columns from a0 on at 64 nodes: k = s is +x_s, k = SH + s
+// is -x_s.  16 waves: waves 0..7 take the even l, 8..15 the odd ones, l =
+// parity + 2 wave' + 16 i, and their sums are added pairwise in LDS in a fixed
+// order.  Lane = node; the T row is uniform (scalar loads).  11 FP64 operations
+// per (l, node, column), so it is bound by FP64 issue: 0.157 ms at 2501 l,
+// 1876 nodes, 60 columns is 20e12 operations/s, where a loop of additions or
+// fused multiply-adds alone reaches 29e12 to 32e12 on this card.  CA columns
+// share a P load.
+constexpr int GN_W = 16;
+template <int CA>
+__global__ __launch_bounds__(64 * GN_W) void gl_phi(const dd* __restrict__ P, int SH, const double* __restrict__ T,
+                                                    int ldt, int nl, int nc, dd* __restrict__ Phi)
+{
+    __shared__ dd R[GN_W / 2][CA][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // block b: node block nb and column group cg with b = 8 (ncg (nb / 8) + cg)
+    // + nb % 8, so the column groups of a node block share an XCD (b % 8) and
+    // read its slice of P from one L2
+    const int ncg = (nc + CA - 1) / CA, q8 = blockIdx.x >> 3;
+    const int nb = 8 * (q8 / ncg) + (blockIdx.x & 7), a0 = CA * (q8 % ncg);
+    if (64 * nb >= SH) return;
+    const int s = 64 * nb + lane;
+    const int par = wave >> 3, ww = wave & 7;
+    dd acc[CA];
+#pragma unroll
+    for (int k = 0; k < CA; ++k) acc[k] = dd{0.0, 0.0};
+    const dd* const p = P + s;
+#pragma unroll 4
+    for (int l = par + 2 * ww; l < nl; l += GN_W) {
+        const dd pl = p[(long)l * SH];
+        const double* const t = T + (long)l * ldt + a0;
+#pragma unroll
+        for (int k = 0; k < CA; ++k) dd_mac(acc[k], t[k], pl);
+    }
+#pragma unroll
+    for (int k = 0; k < CA; ++k) acc[k] = dd_renorm(acc[k]);
+    // 8 -> 4 -> 2 -> 1 waves per parity
+#pragma unroll
+    for (int h = 4; h >= 1; h >>= 1) {
+        if (ww >= h && ww < 2 * h)
+#pragma unroll
+            for (int k = 0; k < CA; ++k) R[par * h + ww - h][k][lane] = acc[k];
+        __syncthreads();
+        if (ww < h)
+#pragma unroll
+            for (int k = 0; k < CA; ++k) acc[k] = acc[k] + R[par * h + ww][k][lane];
+        __syncthreads();
+    }
+    if (par == 1 && ww == 0)
+#pragma unroll
+        for (int k = 0; k < CA; ++k) R[0][k][lane] = acc[k];
+    __syncthreads();
+    if (wave == 0)
+#pragma unroll
+        for (int k = 0; k < CA; ++k)
+            if (a0 + k < nc) {
+                const dd o = R[0][k][lane];
+                dd* const out = Phi + (long)(a0 + k) * 2 * SH;
+                out[s] = acc[k] + o;
+                out[SH + s] = acc[k] - o;
+            }
+}
+
+// Sum the 32 accumulators of a wave over its lanes, halving their number with
+// each exchange: lane 2 i (and 2 i + 1) ends with the total of accumulator i.
+__device__ __forceinline__ dd wave_totals(dd (&acc)[32], int lane)
+{
+#pragma unroll
+    for (int o = 32, n = 16; n >= 1; o >>= 1, n >>= 1) {
+        const bool up = lane & o;
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i < n) {
+                const dd x = acc[i], y = acc[i + n];
+                acc[i] = dd_sel(up, y, x) + dd_shfl_xor(dd_sel(up, x, y), o);
+            }
+    }
+    return acc[0] + dd_shfl_xor(acc[0], 1);
+}
+
+// H[g][a r + b] = scale sum_k w_k Phi_g Phi_a Phi_b over all K = 2 SH nodes.
+// One workgroup per job: a in a tile of four columns ta, two b of tile tb >=
+// ta, c in tile tc >= tb (a <= b <= c covers every entry; the entry is written
+// at all its orders).  Wave q takes a quarter of the 64-node steps, lane =
+// node: per step 10 columns are read for 32 products (12 operations each plus
+// the pair products: FP64 issue bounds it, the reads come from L2).  The last
+// workgroup forms the gate's two sums.
+__device__ __forceinline__ void core_job(int job, int NT, int* ta, int* tb, int* tc, int* h)
+{
+    int t = 0;
+    for (int nj; job >= (nj = 2 * (t + 1) * (NT - t)); ++t) job -= nj;
+    *tb = t;
+    *h = job & 1;
+    job >>= 1;
+    *ta = job % (t + 1);
+    *tc = t + job / (t + 1);
+}
+
+__global__ __launch_bounds__(256, 2) void gl_core_dd(const dd* __restrict__ Phi, int SH, const dd* __restrict__ w,
+                                                     int r, double scale, double* __restrict__ H, long ldh, int njobs,
+                                                     const double* __restrict__ T, int ldt, int nl,
+                                                     double* __restrict__ gate)
+{
+    __shared__ dd R[4][32];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, K = 2 * SH;
+    if (blockIdx.x == (unsigned)njobs) {
+        // gate[0] = sum_k w_k Phi_r^3, gate[1] = sum_l T[l][r]; H's padding
+        // (r^2 odd) is zeroed
+        if (ldh > (long)r * r)
+            for (int g = threadIdx.x; g < r; g += 256) H[(long)g * ldh + (long)r * r] = 0.0;
+        dd A{0.0, 0.0};
+        double S = 0.0;
+        for (int k = threadIdx.x; k < K; k += 256) {
+            const dd f = Phi[(long)r * K + k];
+            A = A + w[k < SH ? k : k - SH] * f * (f * f);
+        }
+        for (int l = threadIdx.x; l < nl; l += 256) S += T[(long)l * ldt + r];
+        for (int o = 32; o >= 1; o >>= 1) {
+            A = A + dd_shfl_xor(A, o);
+            S += __shfl_xor(S, o);
+        }
+        if (lane == 0) {
+            R[wave][0] = A;
+            R[wave][1].hi = S;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const dd a = (R[0][0] + R[1][0]) + (R[2][0] + R[3][0]);
+            gate[0] = a.hi + a.lo;
+            gate[1] = (R[0][1].hi + R[1][1].hi) + (R[2][1].hi + R[3][1].hi);
+        }
+        return;
+    }
+    int ta, tb, tc, h;
+    core_job(blockIdx.x, (r + 3) / 4, &ta, &tb, &tc, &h);
+    dd acc[32];
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc[i] = dd{0.0, 0.0};
+    // columns past r repeat the last one (their products are not stored);
+    // uniform row bases and one lane offset, the next step's columns loaded
+    // before this step's products
+    const char *fa[4], *fb[2], *fc[4];
+    auto row = [&](int f) { return reinterpret_cast<const char*>(Phi + (size_t)min(f, r - 1) * K); };
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        fa[i] = row(4 * ta + i);
+        fc[i] = row(4 * tc + i);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) fb[i] = row(4 * tb + 2 * h + i);
+    const char* const wb = reinterpret_cast<const char*>(w);
+    struct Step {
+        dd a[4], b[2], c[4], w;
+    };
+    auto load = [&](int k0, Step& S) {
+        const unsigned o = (unsigned)(k0 + lane) * (unsigned)sizeof(dd);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            S.a[i] = *reinterpret_cast<const dd*>(fa[i] + o);
+            S.c[i] = *reinterpret_cast<const dd*>(fc[i] + o);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) S.b[i] = *reinterpret_cast<const dd*>(fb[i] + o);
+        S.w = *reinterpret_cast<const dd*>(wb + (unsigned)((k0 < SH ? k0 : k0 - SH) + lane) * (unsigned)sizeof(dd));
+    };
+    Step cur, nxt;
+    const int kw = __builtin_amdgcn_readfirstlane(64 * wave);
+    load(kw < K ? kw : 0, cur);
+#pragma unroll 1
+    for (int k0 = kw; k0 < K; k0 += 256) {
+        load(k0 + 256 < K ? k0 + 256 : k0, nxt);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const dd u = cur.w * cur.b[j];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const dd t = u * cur.a[i];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) dd_mac(acc[16 * j + 4 * i + q], t, cur.c[q]);
+            }
+        }
+        cur = nxt;
+    }
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc[i] = dd_renorm(acc[i]);
+    const dd tot = wave_totals(acc, lane);
+    if (!(lane & 1)) R[wave][lane >> 1] = tot;
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        const int e = threadIdx.x;
+        const dd t = scale * ((R[0][e] + R[1][e]) + (R[2][e] + R[3][e]));
+        const double v = t.hi + t.lo;
+        const int b = 4 * tb + 2 * h + (e >> 4), a = 4 * ta + ((e >> 2) & 3), c = 4 * tc + (e & 3);
+        if (a <= b && b <= c && c < r) {
+            const int o[6][3] = {{a, b, c}, {a, c, b}, {b, a, c}, {b, c, a}, {c, a, b}, {c, b, a}};
+#pragma unroll
+            for (int p = 0; p < 6; ++p) H[(long)o[p][0] * ldh + (long)o[p][1] * r + o[p][2]] = v;
+        }
+    }
+}
+
+// The double-double rule of order npt and P_l at its nodes up to lmax, kept by
+// the context for the last (npt, lmax): they depend on nothing else.
+int gl_table(mcmb_ctx* c, int npt, int lmax)
+{
+    GlTable& G = c->glt;
+    if (G.npt == npt && G.lmax >= lmax) return MCMB_OK;
+    G.npt = 0;
+    G.half = (npt + 1) / 2;
+    G.SH = (G.half + 63) & ~63;   // whole waves of nodes, the padding with weight 0
+    const int nc = std::max(npt, lmax) + 1;
+    const size_t nx = (size_t)2 * G.SH, np = (size_t)(lmax + 1) * G.SH;
+    MCMB_TRY(G.buf.alloc(sizeof(dd) * (nx + nc + np)));
+    dd* const x = G.buf.as<dd>();
+    dd *const w = x + G.SH, *const cl = w + G.SH, *const P = cl + nc;
+    hipLaunchKernelGGL(gl_coef, dim3((nc + 255) / 256), dim3(256), 0, c->stream, nc - 1, cl);
+    hipLaunchKernelGGL(gl_rule, dim3(G.SH / 64), dim3(64), 0, c->stream, npt, G.half, G.SH, (const dd*)cl, x, w);
+    hipLaunchKernelGGL(gl_ptab, dim3(G.SH / 64), dim3(64), 0, c->stream, lmax, G.half, G.SH, (const dd*)cl,
+                       (const dd*)x, P);
+    MCMB_HIP(hipGetLastError());
+    G.w = w;
+    G.P = P;
+    G.npt = npt;
+    G.lmax = lmax;
+    return MCMB_OK;
+}
+
+// Whether the node form takes this setup's whole Gram (see the header comment;
+// the gate is checked after the sums).  Below GN_LMIN the tetrapyd contraction
+// stays the default: it takes 0.17 ms there, most of it launches, and its
+// results are the same bits for all its kernel variants.  Above GN_TABMAX the
+// table of P_l would be kept at the expense of the caller's memory.
+bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool any_lmax)
+{
+    if (L.kspace || L.uniform || L.h2mode != MCMB_H2_EXACT || L.kstep != 2) return false;
+    if (row_lo != 0 || row_hi != (int)L.rows.size()) return false;
+    if (r < 1 || r + 1 > GN_RMAX || (L.lmax <= GN_LMIN && !any_lmax)) return false;
+    const size_t half = (3 * (size_t)L.lmax / 2 + 2) / 2 + 64;
+    return sizeof(dd) * half * (L.lmax + 1) <= GN_TABMAX;
+}
+
+// H (r x ldh) of the exact tetrapyd Gram over the r columns Pc (by columns,
+// leading dimension nlp).  phase: called with the name of each part.
+int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, int nl, int r, double* H, long ldh,
+                    const std::function<int(const char*)>& phase)
+{
+    const int npt = 3 * L.lmax / 2 + 1;
+    if (!(c->glt.npt == npt && c->glt.lmax >= L.lmax)) MCMB_TRY(phase("Legendre table"));
+    MCMB_TRY(gl_table(c, npt, L.lmax));
+    const GlTable& G = c->glt;
+    const int nc = r + 1, K = 2 * G.SH;
+    // columns per thread: the most that still give about one workgroup per CU
+    int ca = 8;
+    const int nbx = G.SH / 64;
+    while (ca > 2 && nbx * ((nc + ca - 1) / ca) < 200) ca >>= 1;
+    const int ldt = (nc + 7) & ~7;
+    MCMB_TRY(c->gn_ws.alloc(sizeof(dd) * (size_t)nc * K + sizeof(double) * (size_t)nl * ldt));
+    dd* const Phi = c->gn_ws.as<dd>();
+    double* const T = reinterpret_cast<double*>(Phi + (size_t)nc * K);
+    if (!c->gn_gate) MCMB_HIP(hipHostMalloc((void**)&c->gn_gate, 2 * sizeof(double), hipHostMallocDefault));
+    MCMB_TRY(phase("basis at the nodes"));
+    hipLaunchKernelGGL(gl_ttab, dim3((nl + 31) / 32), dim3(256), 0, c->stream, Pc, nlp, nl, r, L.lmin,
+                       (const double*)L.d_v.as<double>(), ldt, T);
+    const dim3 grid(8 * ((nbx + 7) / 8) * ((nc + ca - 1) / ca)), block(64 * GN_W);
+#define GN_PHI(CA) hipLaunchKernelGGL(gl_phi<CA>, grid, block, 0, c->stream, (const dd*)G.P, G.SH, (const double*)T, ldt, nl, nc, Phi)
+    if (ca == 8) GN_PHI(8);
+    else if (ca == 4) GN_PHI(4);
+    else GN_PHI(2);
+#undef GN_PHI
+    MCMB_HIP(hipGetLastError());
+    MCMB_TRY(phase("node sum"));
+    const int NT = (r + 3) / 4;
+    int njobs = 0;
+    for (int t = 0; t < NT; ++t) njobs += 2 * (t + 1) * (NT - t);
+    hipLaunchKernelGGL(gl_core_dd, dim3(njobs + 1), dim3(256), 0, c->stream, (const dd*)Phi, G.SH, (const dd*)G.w, r,
+                       3.0 / (4.0 * M_PI), H, ldh, njobs, (const double*)T, ldt, nl, c->gn_gate);
+    MCMB_HIP(hipGetLastError());
+    return MCMB_OK;
+}
+
+// After the stream has been synchronised: whether the sums are good to FP64.
+// With m_l = max_a |P[l][a]|, every term of every entry is bounded by those of
+// sum w Phi_m^3 formed with absolute values, at most 2 S^3 (|P_l| <= 1, sum w
+// = 2); A = sum w Phi_m^3 is the tetrapyd sum of the same bound over the
+// allowed terms, the scale of H that FP64 resolves to 2^-53.  Each term
+// carries about 2^-104 times a growth of the recurrence linear in l.
+bool gl_gate(const mcmb_ctx* c, int lmax)
+{
+    const double A = c->gn_gate[0], S = c->gn_gate[1];
+    return 2.0 * S * S * S * 0x1p-104 * (lmax + 64.0) <= 0x1p-54 * A;
+}
+
+}  // namespace mcmb

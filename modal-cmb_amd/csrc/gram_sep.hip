@@ -1907,6 +1907,59 @@ static int separable_ptab(mcmb_ctx* c, int ldu)
     return MCMB_OK;
 }
 
+// H over the compressed basis (S.h, r^3 entries) back to pairs: T1[(a,b)][z] =
+// sum_g H[g][(a,b)] Ct[g][z] (into M), Y2s[a][{y,z}] = sum_b Ct[b][y]
+// T1[(a,b)][z] for y <= z (into Ys, pair order), G[x][{y,z}] = sum_a Ct[a][x]
+// Y2s[a][{y,z}] (into G): the fully symmetrised tensor over pairs.
+static int sep_expand_alloc(mcmb_ctx* c, int r, int NP, int ld)
+{
+    const long ldh = (long)r * r + ((r * r) & 1), NPP = (long)NP * (NP + 1) / 2, ldp = NPP + (NPP & 1);
+    MCMB_TRY(c->sg_M.alloc(sizeof(double) * (size_t)(ldh * ld)));
+    MCMB_TRY(c->sg_Ys.alloc(sizeof(double) * (size_t)((long)r * ldp)));
+    return c->sg_G.alloc(sizeof(double) * (size_t)((long)NP * ldp));
+}
+
+static int sep_expand(mcmb_ctx* c, const SepComp& S, int NP, int ld)
+{
+    const int r = S.r;
+    const long ldh = (long)r * r + ((r * r) & 1), NPP = (long)NP * (NP + 1) / 2, ldp = NPP + (NPP & 1);
+    const int* tb = S.tab.as<int>();
+    const double* const Ct = S.ct.as<double>();
+    double *const T1 = c->sg_M.as<double>(), *const Y2s = c->sg_Ys.as<double>(), *const G = c->sg_G.as<double>();
+    for (int k = 0; k < 3; ++k) MCMB_TRY(launch_guard("expansion", sep_blocks(S.nt[k], S.gs[k]), 256));
+    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(S.nt[0], S.gs[0])), dim3(256), 0, c->stream,
+                       (const double*)S.h.as<double>(), (int)ldh, tb, Ct, (long)ld, T1, (long)ld, r * r, NP,
+                       reinterpret_cast<const SepTask*>(tb + S.o_task[0]),
+                       reinterpret_cast<const int4*>(tb + S.o_tile[0]), S.nt[0], S.gs[0], 0);
+    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN, true>), dim3(sep_blocks(S.nt[1], S.gs[1])), dim3(256), 0,
+                       c->stream, Ct, ld, tb, (const double*)T1, (long)ld, Y2s, ldp, NP, NP,
+                       reinterpret_cast<const SepTask*>(tb + S.o_task[1]),
+                       reinterpret_cast<const int4*>(tb + S.o_tile[1]), S.nt[1], S.gs[1], 0);
+    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(S.nt[2], S.gs[2])), dim3(256), 0, c->stream,
+                       Ct, ld, tb, (const double*)Y2s, (long)ldp, G, (long)ldp, NP, (int)NPP,
+                       reinterpret_cast<const SepTask*>(tb + S.o_task[2]),
+                       reinterpret_cast<const int4*>(tb + S.o_tile[2]), S.nt[2], S.gs[2], 0);
+    MCMB_HIP(hipGetLastError());
+    return MCMB_OK;
+}
+
+// The 6-term sums of the expanded tensor by 32 x 32 tiles of Gamma, blocks of
+// 6 x 6 tiles per XCD (assembly 0.205 -> 0.146 ms at 4960 modes; 2 x 2: 0.165,
+// 4 x 4: 0.152, 8 x 8: 0.147).
+static int sep_assemble_launch(mcmb_ctx* c, int R, int n, const int* d_modes, double* d_gamma)
+{
+    constexpr int SB = 6;
+    const int NP = R * (R + 1) / 2;
+    const long NPP = (long)NP * (NP + 1) / 2, ldp = NPP + (NPP & 1);
+    const int nt = (n + 31) / 32, nbk = (nt + SB - 1) / SB;
+    const unsigned long long ntile = ((unsigned long long)nbk * (nbk + 1) / 2 + 7) / 8 * 8 * SB * SB;
+    MCMB_TRY(launch_guard("assembly", ntile, 256));
+    hipLaunchKernelGGL(sep_assemble_sym<SB>, dim3((unsigned)ntile), dim3(256), 0, c->stream,
+                       (const double*)c->sg_G.as<double>(), ldp, R, d_modes, n, nt, d_gamma);
+    MCMB_HIP(hipGetLastError());
+    return MCMB_OK;
+}
+
 // ---- Gauss-Legendre Gram over the compressed pair basis ---------------------
 //
 // The GL-factorised Gram (calculate_orthol, orthogonalisation_late.c:239-336)
@@ -2081,15 +2134,12 @@ static int gl_compressed_run(mcmb_ctx* c, const GlField3& F, int npt, const doub
     const int r = S.r;
     if (r <= 0 || r > 4 * GL_GW) return MCMB_OK;   // full rank: the direct node sum
     const long ldh = (long)r * r + ((r * r) & 1);
-    const long NPP = (long)NP * (NP + 1) / 2, ldp = NPP + (NPP & 1);
     MCMB_TRY(c->gl_xw.alloc(sizeof(double) * (2 * (size_t)npt + (size_t)r * npt + (size_t)r * S.nlp)));
     double* const dx = c->gl_xw.as<double>();
     double* const dw = dx + npt;
     double* const dphi = dw + npt;
     double* const dpw = dphi + (size_t)r * npt;
-    MCMB_TRY(c->sg_M.alloc(sizeof(double) * (size_t)(ldh * ld)));
-    MCMB_TRY(c->sg_Ys.alloc(sizeof(double) * (size_t)((long)r * ldp)));
-    MCMB_TRY(c->sg_G.alloc(sizeof(double) * (size_t)((long)NP * ldp)));
+    MCMB_TRY(sep_expand_alloc(c, r, NP, ld));
     MCMB_HIP(hipMemcpyAsync(dx, x, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
     MCMB_HIP(hipMemcpyAsync(dw, w, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
     MCMB_HIP(hipEventRecord(c->ev0, c->stream));
@@ -2103,32 +2153,8 @@ static int gl_compressed_run(mcmb_ctx* c, const GlField3& F, int npt, const doub
                        (const double*)dphi, (const double*)dphi, r, npt, (const double*)dw, r, 3.0 / (4.0 * M_PI),
                        S.h.as<double>(), ldh);
     MCMB_HIP(hipGetLastError());
-    // the expansion and the assembly of the separable Gram
-    const int* tb = S.tab.as<int>();
-    double* const T1 = c->sg_M.as<double>();
-    double* const Y2s = c->sg_Ys.as<double>();
-    double* const G = c->sg_G.as<double>();
-    MCMB_TRY(launch_guard("GL expansion", sep_blocks(S.nt[0], S.gs[0]), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(S.nt[0], S.gs[0])), dim3(256), 0, c->stream,
-                       (const double*)S.h.as<double>(), (int)ldh, tb, (const double*)S.ct.as<double>(), (long)ld, T1,
-                       (long)ld, r * r, NP, reinterpret_cast<const SepTask*>(tb + S.o_task[0]),
-                       reinterpret_cast<const int4*>(tb + S.o_tile[0]), S.nt[0], S.gs[0], 0);
-    MCMB_TRY(launch_guard("GL expansion", sep_blocks(S.nt[1], S.gs[1]), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN, true>), dim3(sep_blocks(S.nt[1], S.gs[1])), dim3(256), 0,
-                       c->stream, (const double*)S.ct.as<double>(), ld, tb, (const double*)T1, (long)ld, Y2s, ldp, NP,
-                       NP, reinterpret_cast<const SepTask*>(tb + S.o_task[1]),
-                       reinterpret_cast<const int4*>(tb + S.o_tile[1]), S.nt[1], S.gs[1], 0);
-    MCMB_TRY(launch_guard("GL expansion", sep_blocks(S.nt[2], S.gs[2]), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(S.nt[2], S.gs[2])), dim3(256), 0, c->stream,
-                       (const double*)S.ct.as<double>(), ld, tb, (const double*)Y2s, (long)ldp, G, (long)ldp, NP,
-                       (int)NPP, reinterpret_cast<const SepTask*>(tb + S.o_task[2]),
-                       reinterpret_cast<const int4*>(tb + S.o_tile[2]), S.nt[2], S.gs[2], 0);
-    constexpr int SB = 6;   // blocks of SB x SB assembly tiles per XCD
-    const int nt = (n + 31) / 32, nbk = (nt + SB - 1) / SB;
-    const unsigned long long ntile = ((unsigned long long)nbk * (nbk + 1) / 2 + 7) / 8 * 8 * SB * SB;
-    MCMB_TRY(launch_guard("GL assembly", ntile, 256));
-    hipLaunchKernelGGL(sep_assemble_sym<SB>, dim3((unsigned)ntile), dim3(256), 0, c->stream, (const double*)G, ldp, R,
-                       F.d_modes, n, nt, d_gamma);
+    MCMB_TRY(sep_expand(c, S, NP, ld));
+    MCMB_TRY(sep_assemble_launch(c, R, n, F.d_modes, d_gamma));
     MCMB_HIP(hipGetLastError());
     MCMB_HIP(hipEventRecord(c->ev1, c->stream));
     MCMB_HIP(hipStreamSynchronize(c->stream));   // x and w may live on the caller's stack
@@ -2345,6 +2371,20 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
         comp = S.r > 0;
         setup_done("basis factorisation");
     }
+    auto finish = [&](int rank) -> int {
+        if (np > 0) MCMB_HIP(hipEventRecord(c->evp[np], c->stream));
+        MCMB_HIP(hipEventRecord(c->ev1, c->stream));
+        MCMB_HIP(hipStreamSynchronize(c->stream));
+        setup_done("launch to completion");
+        setup_end(c);
+        float ms = 0.f;
+        MCMB_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
+        c->last_ms = ms;
+        c->last_launches = launches;
+        c->nphases = np;
+        c->last_rank = rank;
+        return MCMB_OK;
+    };
     const int NB = comp ? S.r : NP;
     const int ldB = NB + (NB & 1);         // even leading dimension of M, Y rows
     const L3Shape sh = sep_l3_shape(NB);
@@ -2358,7 +2398,38 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
     const int tm = small ? 64 : SG_TM, tn = small ? 64 : SG_TN;
     const int ksplit = comp ? SG_KSPLIT : 1;
     bool rowptr_ready = false;
-    MCMB_TRY(separable_plan(c, L, row_lo, row_hi, NB, ldB, gsz, tm, tn, ksplit, rowptr_ready));
+    auto plan = [&]() { return separable_plan(c, L, row_lo, row_hi, NB, ldB, gsz, tm, tn, ksplit, rowptr_ready); };
+    // The core as a node sum (gram_nodes.hip), unless a switch of the tetrapyd
+    // contraction is set or the error bound failed on this setup before.
+    // (MCMB_SEP_TABLES asks for the contraction's tables, which the node form
+    // does not read: they are built all the same, for last_setup.)
+    const char* gpath = getenv("MCMB_GRAM_PATH");
+    const bool asked = gpath && !strcmp(gpath, "nodes");
+    bool nodes = comp && (!gpath || !*gpath || asked) && c->gn_refused != L.generation &&
+                 gram_nodes_supported(L, S.r, row_lo, row_hi, asked);
+    for (const char* k : {"MCMB_SEP_L3", "MCMB_SEP_WEIGHTS", "MCMB_SEP_GROUPS", "MCMB_SEP_BLOCK_ROWS"})
+        if (getenv(k)) nodes = false;
+    if (!nodes || getenv("MCMB_SEP_TABLES")) MCMB_TRY(plan());
+    if (nodes) {
+        const int r = S.r;
+        MCMB_TRY(sep_expand_alloc(c, r, NP, ld));
+        setup_done("buffers");
+        MCMB_TRY(gram_nodes_core(c, L, S.pc.as<double>(), S.nlp, nl, r, S.h.as<double>(),
+                                 (long)r * r + ((r * r) & 1), phase));
+        MCMB_TRY(phase("expansion to pairs"));
+        MCMB_TRY(sep_expand(c, S, NP, ld));
+        MCMB_TRY(phase("assembly"));
+        MCMB_TRY(sep_assemble_launch(c, R, n, L.d_modes.as<int>(), d_gamma));
+        launches += 7;
+        MCMB_TRY(finish(r));
+        if (gl_gate(c, L.lmax)) return MCMB_OK;
+        c->gn_refused = L.generation;   // the tetrapyd contraction, here and from now on
+        np = 0;
+        launches = 0;
+        setup_begin(c);
+        MCMB_HIP(hipEventRecord(c->ev0, c->stream));
+        MCMB_TRY(plan());
+    }
     const SepPlan& P = c->sep;
 
     const long NPP = (long)NP * (NP + 1) / 2;   // unordered pairs {e, f}
@@ -2579,48 +2650,21 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
         launches += 4;
     }
     if (comp) {
-        // H over the compressed basis (r^3 entries), then back to pairs:
-        // T1[(a,b)][z] = sum_g H[g][(a,b)] Ct[g][z] (into M), Y2s[a][{y,z}] =
-        // sum_b Ct[b][y] T1[(a,b)][z] for y <= z (into Ys, pair order),
-        // G[x][{y,z}] = sum_a Ct[a][x] Y2s[a][{y,z}] (into G): the fully
-        // symmetrised tensor over pairs
         MCMB_TRY(phase("expansion to pairs"));
         const int r = NB;
-        const int* tb = S.tab.as<int>();
         const long eh = (long)r * ldh;
         MCMB_TRY(launch_guard("expansion", (unsigned long long)((eh + 255) / 256), 256));
         hipLaunchKernelGGL(sep_hfull, dim3((unsigned)((eh + 255) / 256)), dim3(256), 0, c->stream,
                            (const double*)c->sg_G.as<double>(), ldq2, (long)NB * ldq2,
                            ksplit, r, S.h.as<double>(), ldh);
-        MCMB_TRY(launch_guard("expansion", sep_blocks(S.nt[0], S.gs[0]), 256));
-        SEP_GEMMF(true, 4, SG_FM, SG_FN, S.nt[0], S.gs[0], S.h.as<double>(), ldh, tb, S.ct.as<double>(), ld, c->sg_M.as<double>(),
-                 ld, r * r, NP, tb + S.o_task[0], tb + S.o_tile[0], 0);
-        MCMB_TRY(launch_guard("expansion", sep_blocks(S.nt[1], S.gs[1]), 256));
-        hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN, true>), dim3(sep_blocks(S.nt[1], S.gs[1])), dim3(256), 0,
-                           c->stream, (const double*)S.ct.as<double>(), ld, tb, (const double*)c->sg_M.as<double>(),
-                           (long)ld, c->sg_Ys.as<double>(), ldp, NP, NP,
-                           reinterpret_cast<const SepTask*>(tb + S.o_task[1]),
-                           reinterpret_cast<const int4*>(tb + S.o_tile[1]), S.nt[1], S.gs[1], 0);
-        MCMB_TRY(launch_guard("expansion", sep_blocks(S.nt[2], S.gs[2]), 256));
-        SEP_GEMMF(true, 4, SG_FM, SG_FN, S.nt[2], S.gs[2], S.ct.as<double>(), ld, tb, c->sg_Ys.as<double>(), ldp,
-                 c->sg_G.as<double>(), ldp, NP, (int)NPP, tb + S.o_task[2], tb + S.o_tile[2], 0);
-        MCMB_HIP(hipGetLastError());
+        MCMB_TRY(sep_expand(c, S, NP, ld));
         launches += 4;
     }
 #undef SEP_GEMM
 #undef SEP_GEMMF
     MCMB_TRY(phase("assembly"));
     if (comp) {
-        // the 6-term sums straight from the expanded tensor, by 32 x 32 tiles
-        // blocks of 6 x 6 tiles per XCD (assembly 0.205 -> 0.146 ms at 4960 modes;
-        // 2 x 2: 0.165, 4 x 4: 0.152, 8 x 8: 0.147)
-        constexpr int S = 6;
-        const int nt = (n + 31) / 32, nbk = (nt + S - 1) / S;
-        const unsigned long long ntile = ((unsigned long long)nbk * (nbk + 1) / 2 + 7) / 8 * 8 * S * S;
-        MCMB_TRY(launch_guard("assembly", ntile, 256));
-        hipLaunchKernelGGL(sep_assemble_sym<S>, dim3((unsigned)ntile), dim3(256), 0, c->stream,
-                           (const double*)c->sg_G.as<double>(), ldp, R, L.d_modes.as<int>(), n, nt, d_gamma);
-        MCMB_HIP(hipGetLastError());
+        MCMB_TRY(sep_assemble_launch(c, R, n, L.d_modes.as<int>(), d_gamma));
         ++launches;
     } else {
         // Gs from G2, then the 6-term sums
@@ -2636,18 +2680,7 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
         MCMB_HIP(hipGetLastError());
         launches += 2;
     }
-    if (np > 0) MCMB_HIP(hipEventRecord(c->evp[np], c->stream));
-    MCMB_HIP(hipEventRecord(c->ev1, c->stream));
-    MCMB_HIP(hipStreamSynchronize(c->stream));
-    setup_done("launch to completion");
-    setup_end(c);
-    float ms = 0.f;
-    MCMB_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
-    c->last_ms = ms;
-    c->last_launches = launches;
-    c->nphases = np;
-    c->last_rank = comp ? NB : 0;
-    return MCMB_OK;
+    return finish(comp ? NB : 0);
 }
 
 }  // namespace mcmb

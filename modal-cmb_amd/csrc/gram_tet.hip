@@ -338,9 +338,11 @@ int gram_tet_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gamma, in
     c->last_rank = -1;
     // FP64: the separable contraction wherever the basis width allows it,
     // else the factored one, else the direct point-by-point contraction below.
-    // MCMB_GRAM_PATH = separable | factored | direct selects one explicitly.
+    // MCMB_GRAM_PATH = separable | nodes | factored | direct selects one
+    // explicitly (nodes: the separable order's compressed basis with its core
+    // as a node sum, gram_nodes.hip, which is the default above GN_LMIN).
     const char* path = getenv("MCMB_GRAM_PATH");
-    const bool want_sep = !path || !*path || !strcmp(path, "separable");
+    const bool want_sep = !path || !*path || !strcmp(path, "separable") || !strcmp(path, "nodes");
     const bool want_fac = !path || !*path || !strcmp(path, "factored");
     if (want_sep && gram_separable_supported(L, precision))
         return gram_separable_launch(c, L, precision, d_gamma, row_lo, row_hi);

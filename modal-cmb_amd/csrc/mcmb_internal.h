@@ -5,6 +5,7 @@
 #include <chrono>
 #include <cstdint>
 #include <cstdlib>
+#include <functional>
 #include <string>
 #include <thread>
 #include <vector>
@@ -211,6 +212,18 @@ struct PolSet {
 // MCMB_SPLINE_TRAPEZIUM) on the increasing grid x.
 int spline_weights(const std::vector<double>& x, int kind, std::vector<double>& cw);
 
+// Double-double Gauss-Legendre rule (weights w of the nodes x >= 0) and P_l at
+// its nodes, P[l][SH] (gram_nodes.hip), for the last (npt, lmax) asked for.
+struct dd;
+struct GlTable {
+    int npt = 0, lmax = -1, half = 0, SH = 0;
+    DevBuf buf;
+    dd *w = nullptr, *P = nullptr;
+};
+constexpr int GN_RMAX = 64;                    // columns of the node form, the gate's included
+constexpr int GN_LMIN = 512;                   // the node form takes lmax above this
+constexpr size_t GN_TABMAX = (size_t)1 << 30;  // bytes of the table of P_l
+
 constexpr int MAX_PHASES = 10;
 // Per-batch slots of the pinned staging used by the projection's transfers.
 constexpr int PSLOTS = 8;
@@ -306,6 +319,12 @@ struct mcmb_ctx {
     mcmb::TrdWork trd;
     // the GL Gram over the compressed basis: node table and Phi
     mcmb::DevBuf gl_xw;
+    // the node form of the tetrapyd Gram: rule and Legendre table, work space,
+    // the gate's two sums (pinned), and the setup that did not pass it
+    mcmb::GlTable glt;
+    mcmb::DevBuf gn_ws;
+    double* gn_gate = nullptr;
+    long gn_refused = -1;
     // the GL cross-Gamma: node tables, M and the core tensor
     mcmb::DevBuf cx_ws;
     // the last Gauss-Legendre rule the Grams asked for (gl_nodes)
@@ -413,6 +432,14 @@ bool gram_factored_supported(const PointSet& P, int precision);
 int gram_factored_launch(mcmb_ctx* ctx, PointSet& P, int precision, double* d_gamma, int row_lo, int row_hi);
 // Separable Gram (contractions over l3, then l2, then l1 of the pair products):
 // whether it handles this basis width and precision, and the launch.
+// The node form of the exact l-space Gram over a compressed basis
+// (gram_nodes.hip): whether it takes the setup, the core tensor H, and after
+// the stream is synchronised whether its error bound holds.
+// (any_lmax: also up to GN_LMIN)
+bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool any_lmax);
+int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, int nl, int r, double* H, long ldh,
+                    const std::function<int(const char*)>& phase);
+bool gl_gate(const mcmb_ctx* c, int lmax);
 bool gram_separable_supported(const PointSet& P, int precision);
 int gram_separable_launch(mcmb_ctx* ctx, PointSet& P, int precision, double* d_gamma, int row_lo, int row_hi);
 }  // namespace mcmb

@@ -548,3 +548,64 @@ def test_separable_device_row_groups_equal_host(ctx, lmax, R, block_rows, weight
     assert np.array_equal(Gd, Gh)
     names = [n for n, _ in ctx.last_setup()]
     assert "row groups and tables (host)" in names
+
+
+@pytest.mark.parametrize("lmin,L,R", [(2, 24, 8), (0, 97, 9), (3, 131, 12), (2, 161, 32), (2, 600, 10), (2, 777, 8)])
+def test_node_form_vs_separable(ctx, lmin, L, R):
+    """The node form of the compressed core (the default above lmax 512)
+    against the tetrapyd contraction it replaces there and, where that is
+    quick, the oracle's direct sum: both are FP64 roundings of one sum (1e-13
+    as the contraction orders above).  Odd and even lmax and node counts, 15 to
+    63 columns (column tiles of 4, node blocks of 64)."""
+    ws = W.lspace(L, R, True, lmin=lmin)
+    ctx.lspace_set(lmin, L, ws["q"], ws["v"], ws["order"])
+    G = _gram_paths(ctx, modalcmb.FP64, ("separable", "nodes"))
+    assert ctx.last_basis_rank() == 2 * R - 1
+    assert "node sum" in [p for p, _ in ctx.last_phases()]
+    assert rel_elem(G["nodes"], G["separable"]) < 1e-13
+    assert np.array_equal(G["nodes"], G["nodes"].T)
+    if L < 200:
+        assert rel_elem(G["nodes"], O.gamma_tet(lmin, L, ws["q"], ws["v"], ws["order"])) < 1e-12
+    D = ctx.gamma_tet(modalcmb.FP64)
+    assert np.array_equal(D, G["nodes" if L > 512 else "separable"])
+
+
+def test_node_form_gate(ctx):
+    """Weights whose forbidden multipole triples outweigh the allowed ones by
+    more than double-double resolves (odd l 24 decades above even l: no triple
+    of three odd l has an even sum) take the tetrapyd contraction, bit for
+    bit; so do weights that are not finite.  Zero weights give zero."""
+    L, R = 600, 8
+    ws = W.lspace(L, R)
+    v = ws["v"].copy()
+    v[1::2] *= 1e24
+    ctx.lspace_set(2, L, ws["q"], v, ws["order"])
+    D = ctx.gamma_tet(modalcmb.FP64)
+    assert "node sum" not in [p for p, _ in ctx.last_phases()]
+    assert np.array_equal(D, _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"])
+    v = ws["v"].copy()
+    v[7] = np.inf
+    ctx.lspace_set(2, L, ws["q"], v, ws["order"])
+    D = ctx.gamma_tet(modalcmb.FP64)
+    assert np.array_equal(D, _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"], equal_nan=True)
+    ctx.lspace_set(2, L, ws["q"], np.zeros(L + 1), ws["order"])
+    assert not ctx.gamma_tet(modalcmb.FP64).any()
+    ctx.lspace_set(2, L, ws["q"], ws["v"], ws["order"])
+    ctx.gamma_tet(modalcmb.FP64)
+    assert "node sum" in [p for p, _ in ctx.last_phases()]
+
+
+def test_separable_device_row_groups_equal_host_lmax2500(ctx):
+    """As test_separable_device_row_groups_equal_host at a size where the
+    default is the node form, which reads no row groups: the tetrapyd
+    contraction by name."""
+    ws = W.lspace(2500, 30, True)
+    ctx.lspace_set(2, 2500, ws["q"], ws["v"], ws["order"])
+    Gd = _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"]
+    os.environ["MCMB_SEP_TABLES"] = "host"
+    try:
+        ctx.lspace_set(2, 2500, ws["q"], ws["v"], ws["order"])      # a new setup: tables rebuilt on the host
+        Gh = _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"]
+    finally:
+        del os.environ["MCMB_SEP_TABLES"]
+    assert np.array_equal(Gd, Gh)
