@@ -22,9 +22,11 @@
 // Both parities of l are summed apart (P_l(-x) = (-1)^l P_l(x)), so the table
 // holds the nodes x >= 0 only, and the columns at +x and -x are E + O and
 // E - O.
+#include "core_tensor.h"
 #include "dd.h"
 #include "mcmb_internal.h"
 #include <cmath>
+#include <vector>
 
 namespace mcmb {
 
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(64) void gl_ptab(int lmax, int half, int SH, const 
 __global__ __launch_bounds__(256) void gl_ttab(const double* __restrict__ Pc, int nlp, int nl, int r, int lmin,
                                                const double* __restrict__ v, int ldt, double* __restrict__ T)
 {
-    __shared__ double S[GN_RMAX][33];
+    __shared__ double S[GN_RMAX + 1][33];
     const int l0 = blockIdx.x * 32, tl = threadIdx.x & 31;
     for (int a = threadIdx.x >> 5; a < r; a += 8) S[a][tl] = l0 + tl < nl ? Pc[(long)a * nlp + l0 + tl] : 0.0;
     __syncthreads();
@@ -443,6 +445,214 @@ bool gl_gate(const mcmb_ctx* c, int lmax)
 {
     const double A = c->gn_gate[0], S = c->gn_gate[1];
     return 2.0 * S * S * S * 0x1p-104 * (lmax + 64.0) <= 0x1p-54 * A;
+}
+
+// ---- the FP64 node sum (mcmb_gamma_gl, mcmb_gamma_gl_pol) over compressed bases ----
+//
+// The Gauss-Legendre Gram keeps its FP64 nodes and recurrence (its results are
+// those of the direct node sum to rounding).  P_l at the nodes x >= 0 depends
+// on (npt, lmax) alone and is kept with the context; Phi is then a GEMM on the
+// matrix cores instead of a recurrence per column group (lmax 2000, r = 39:
+// 0.356 -> 0.035 ms, bound by its loads' latency: 94 workgroups), and the core
+// tensor is cx_core's (0.072 -> 0.038 ms with gl_hsum).
+
+// P[l][s] = P_l(x_s) by the three-term recurrence of the direct node sum, l <=
+// lmax; 0 past half.  One thread per node, a serial chain.
+__global__ __launch_bounds__(64) void gl_ptab64(int lmax, int half, int SH, const double* __restrict__ x,
+                                                double* __restrict__ P)
+{
+    const int s = blockIdx.x * 64 + threadIdx.x;
+    const bool in = s < half;
+    const double xs = x[s];
+    double p0 = 1.0, p1 = xs;   // P_{l-2}, P_{l-1}
+    P[s] = in ? 1.0 : 0.0;
+    if (lmax >= 1) P[SH + s] = in ? xs : 0.0;
+    for (int l = 2; l <= lmax; ++l) {
+        const double pl = ((2.0 * l - 1.0) * xs * p1 - (l - 1.0) * p0) / l;
+        p0 = p1;
+        p1 = pl;
+        P[(long)l * SH + s] = in ? pl : 0.0;
+    }
+}
+
+// Phi[k / 64][a][k % 64] = sum_l T[l][a] P_l(+-x_s), a < r (k = s: +x_s, SH + s:
+// -x_s): one workgroup per 16 nodes, FP64 MFMA with up to four 16-column tiles;
+// waves 0..7 take the even l, 8..15 the odd ones, 4 of a parity per step, and
+// their sums are added pairwise in LDS in a fixed order.
+__global__ __launch_bounds__(1024) void gl_phi64(const double* __restrict__ P, int SH, const double* __restrict__ T,
+                                                 int ldt, int nl, int r, double* __restrict__ Phi)
+{
+    __shared__ d4 R[8][4][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int par = wave >> 3, ww = wave & 7, col = lane & 15, nct = (r + 15) >> 4;
+    const double* const p = P + 16 * blockIdx.x + col;
+    d4 acc[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) acc[t] = d4{0.0, 0.0, 0.0, 0.0};
+    for (int l0 = par + 8 * ww; l0 < nl; l0 += 64) {
+        const int l = l0 + 2 * (lane >> 4), lc = min(l, nl - 1);
+        const double pv = l < nl ? p[(long)lc * SH] : 0.0;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+            if (t < nct)
+                acc[t] = __builtin_amdgcn_mfma_f64_16x16x4f64(T[(long)lc * ldt + 16 * t + col], pv, acc[t], 0, 0, 0);
+    }
+#pragma unroll
+    for (int h = 4; h >= 1; h >>= 1) {
+        if (ww >= h && ww < 2 * h)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) R[par * h + ww - h][t][lane] = acc[t];
+        __syncthreads();
+        if (ww < h)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) acc[t] += R[par * h + ww][t][lane];
+        __syncthreads();
+    }
+    if (par == 1 && ww == 0)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) R[0][t][lane] = acc[t];
+    __syncthreads();
+    if (wave == 0) {
+        const int s = 16 * blockIdx.x + col, km = SH + s;
+        double* const fp = Phi + (long)(s >> 6) * r * 64 + (s & 63);
+        double* const fm = Phi + (long)(km >> 6) * r * 64 + (km & 63);
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const d4 o = R[0][t][lane];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                const int a = 16 * t + 4 * v + (lane >> 4);
+                if (a < r) {
+                    fp[64 * a] = acc[t][v] + o[v];
+                    fm[64 * a] = acc[t][v] - o[v];
+                }
+            }
+        }
+    }
+}
+
+// The core H from the units' tile tensors (cx_core), added in order: H[g][a r
+// + b] of one field, or H[b][g rP + a] with (a, b) of the pair's field.
+template <bool SAME>
+__global__ __launch_bounds__(256) void gl_hsum(const double* __restrict__ Hu, long us, int nu, int rP, int rS,
+                                               double scale, double* __restrict__ H, long ldh)
+{
+    __shared__ long base[8];
+    const int NTC = (rS + 15) >> 4, NTB = (rP + 15) >> 4;
+    if (threadIdx.x < NTB) base[threadIdx.x] = cx_base(threadIdx.x, NTC, SAME);
+    __syncthreads();
+    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    if (e >= (long)rP * ldh) return;
+    const int x = (int)(e / ldh), rem = (int)(e % ldh), y = rem / rP, z = rem % rP;
+    if (rem >= (SAME ? rP : rS) * rP) {
+        H[e] = 0.0;
+        return;
+    }
+    int a, b, c;
+    if (SAME) {
+        a = min(x, min(y, z));
+        c = max(x, max(y, z));
+        b = x + y + z - a - c;
+    } else {
+        a = min(x, z);
+        b = max(x, z);
+        c = y;
+    }
+    const double* const h = Hu + cx_tile(base[b >> 4], a >> 4, b, c >> 4, NTC, SAME) * 256 + 16 * (a & 15) + (c & 15);
+    double t = 0.0;
+    for (int u = 0; u < nu; ++u) t += h[(long)u * us];
+    H[e] = scale * t;
+}
+
+// The FP64 rule's nodes x >= 0 and weights (the middle node of an odd rule
+// with half its weight, at +x and -x), and P_l at the nodes up to lmax.
+int gl_half_table(mcmb_ctx* c, int npt, int lmax, const double* x, const double* w)
+{
+    GlHalf& G = c->glh;
+    if (G.npt == npt && G.lmax >= lmax) return MCMB_OK;
+    G.npt = 0;
+    const int half = (npt + 1) / 2, SH = (half + 63) & ~63;
+    MCMB_TRY(G.buf.alloc(sizeof(double) * ((size_t)3 * SH + (size_t)(lmax + 1) * SH)));
+    std::vector<double> h((size_t)3 * SH, 0.0);
+    for (int s = 0; s < half; ++s) {
+        const int i = npt / 2 + s;
+        h[s] = x[i];
+        h[SH + s] = h[2 * SH + s] = (npt & 1) && s == 0 ? 0.5 * w[i] : w[i];
+    }
+    double* const d = G.buf.as<double>();
+    MCMB_HIP(hipMemcpyAsync(d, h.data(), sizeof(double) * h.size(), hipMemcpyHostToDevice, c->stream));
+    hipLaunchKernelGGL(gl_ptab64, dim3(SH / 64), dim3(64), 0, c->stream, lmax, half, SH, (const double*)d, d + 3 * SH);
+    MCMB_HIP(hipGetLastError());
+    MCMB_HIP(hipStreamSynchronize(c->stream));   // h
+    G.w = d + SH;
+    G.P = d + 3 * SH;
+    G.SH = SH;
+    G.npt = npt;
+    G.lmax = lmax;
+    return MCMB_OK;
+}
+
+// Doubles of T and of Phi for r columns over nl multipoles.
+static int gl_ldt(int r) { return std::max(16 * ((r + 15) / 16), (r + 8) & ~7); }
+size_t gl_phi64_size(const mcmb_ctx* c, int nl, int r) { return (size_t)nl * gl_ldt(r) + (size_t)2 * c->glh.SH * r; }
+
+// Phi of r compressed columns Pc (by columns) with per-leg weight v into the
+// second part of ws (gl_phi64_size doubles); *phi points there.
+int gl_phi64_launch(mcmb_ctx* c, const double* Pc, int nlp, int nl, int r, int lmin, const double* v, double* ws,
+                    double** phi)
+{
+    const GlHalf& G = c->glh;
+    const int ldt = gl_ldt(r);
+    *phi = ws + (size_t)nl * ldt;
+    hipLaunchKernelGGL(gl_ttab, dim3((nl + 31) / 32), dim3(256), 0, c->stream, Pc, nlp, nl, r, lmin, v, ldt, ws);
+    hipLaunchKernelGGL(gl_phi64, dim3(G.SH / 16), dim3(1024), 0, c->stream, (const double*)G.P, G.SH, (const double*)ws,
+                       ldt, nl, r, *phi);
+    MCMB_HIP(hipGetLastError());
+    return MCMB_OK;
+}
+
+// Units of the core: chunks of 64 nodes, grouped to about 512 workgroups.
+static void gl_units(const mcmb_ctx* c, int rP, int rS, bool same, long* jobs, int* g, int* ng, long* us)
+{
+    const int NTB = (rP + 15) / 16, NTC = (rS + 15) / 16, nch = 2 * c->glh.SH / 64;
+    *jobs = 0;
+    for (int t = 0; t < NTB; ++t) *jobs += cx_jobs(t, NTC, same);
+    const int want = (int)std::min<long>(nch, (511 + *jobs) / *jobs);
+    *g = (nch + want - 1) / want;
+    *ng = (nch + *g - 1) / *g;
+    *us = cx_base(NTB, NTC, same) * 256;
+}
+size_t gl_core64_size(const mcmb_ctx* c, int rP, int rS, bool same)
+{
+    long jobs, us;
+    int g, ng;
+    gl_units(c, rP, rS, same, &jobs, &g, &ng, &us);
+    return (size_t)ng * us;
+}
+
+// H (rP x ldh) = scale sum_k w_k Phi Phi Phi from phP (and phS unless it is the
+// same field); ws: gl_core64_size doubles.
+int gl_core64_launch(mcmb_ctx* c, const double* phP, int rP, const double* phS, int rS, double scale, double* ws,
+                     double* H, long ldh)
+{
+    const bool same = phP == phS;
+    long jobs, us;
+    int g, ng;
+    gl_units(c, rP, rS, same, &jobs, &g, &ng, &us);
+    const int nch = 2 * c->glh.SH / 64;
+    const dim3 grid((unsigned)jobs, ng), hgrid((unsigned)(((long)rP * ldh + 255) / 256));
+#define GL_CORE64(SAME)                                                                                          \
+    do {                                                                                                         \
+        hipLaunchKernelGGL(cx_core<SAME>, grid, dim3(256), 0, c->stream, phP, rP, phS, rS, 64,                   \
+                           (const double*)c->glh.w, 64l, (const double*)nullptr, 0, ng, g, nch, 0, ws, us);      \
+        hipLaunchKernelGGL(gl_hsum<SAME>, hgrid, dim3(256), 0, c->stream, (const double*)ws, us, ng, rP, rS, scale, H, \
+                           ldh);                                                                                 \
+    } while (0)
+    if (same) GL_CORE64(true);
+    else GL_CORE64(false);
+#undef GL_CORE64
+    MCMB_HIP(hipGetLastError());
+    return MCMB_OK;
 }
 
 }  // namespace mcmb

@@ -1972,112 +1972,7 @@ static int sep_assemble_launch(mcmb_ctx* c, int R, int n, const int* d_modes, do
 // and assembled exactly as the separable Gram's core (whose assembly takes
 // 1/36 of the six matchings: 36 / (48 pi) = 3 / (4 pi)).
 
-// The compressed basis with the GL weight folded in, Pw[a][l] = P[l][a]
-// (2l + 1) v_l (0 below lmin).
-__global__ void sep_gl_tabs(const double* __restrict__ Pc, int nlp, int nl, int r, int lmin,
-                            const double* __restrict__ v, double* __restrict__ Pw)
-{
-    const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e < (long)r * nlp) {
-        const int l = (int)(e % nlp);
-        Pw[e] = (l < nl && l >= lmin) ? Pc[e] * ((2.0 * l + 1.0) * v[l]) : 0.0;
-    }
-}
-
-// Phi[a][s] (row stride npt) for a < r: thread (node s, group of GL_AG
-// columns) runs the Legendre recurrence over l and accumulates its columns
-// (the column group is uniform over the wave, so its table reads are scalar).
-// The recurrence keeps its division by l: with rounded coefficients (2l -
-// 1)/l, (l - 1)/l it ran 10% faster but moved the lmax-500 Gram by 3e-12.
-constexpr int GL_AG = 4;
-__global__ __launch_bounds__(256) void sep_gl_phi(const double* __restrict__ Pw, int nlp, int nl, int r,
-                                                  const double* __restrict__ x, int npt, double* __restrict__ Phi)
-{
-    const int s = blockIdx.x * 64 + (threadIdx.x & 63);
-    const int a0 = __builtin_amdgcn_readfirstlane(GL_AG * (blockIdx.y * 4 + (threadIdx.x >> 6)));
-    if (a0 >= r) return;   // the whole wave
-    const double xs = s < npt ? x[s] : 0.0;
-    double acc[GL_AG];
-    const double* pw[GL_AG];
-#pragma unroll
-    for (int k = 0; k < GL_AG; ++k) {
-        acc[k] = 0.0;
-        pw[k] = Pw + (long)min(a0 + k, r - 1) * nlp;   // columns past r repeat the last (not stored)
-    }
-    double p0 = 1.0, p1 = xs;   // P_{l-2}, P_{l-1}
-#pragma unroll
-    for (int k = 0; k < GL_AG; ++k) acc[k] = fma(pw[k][0], 1.0, acc[k]);
-    if (nl > 1)
-#pragma unroll
-        for (int k = 0; k < GL_AG; ++k) acc[k] = fma(pw[k][1], xs, acc[k]);
-    for (int l = 2; l < nl; ++l) {
-        const double pl = ((2.0 * l - 1.0) * xs * p1 - (l - 1.0) * p0) / l;
-        p0 = p1;
-        p1 = pl;
-#pragma unroll
-        for (int k = 0; k < GL_AG; ++k) acc[k] = fma(pw[k][l], pl, acc[k]);
-    }
-    if (s < npt)
-#pragma unroll
-        for (int k = 0; k < GL_AG; ++k)
-            if (a0 + k < r) Phi[(long)(a0 + k) * npt + s] = acc[k];
-}
-
-// H[g][a r + b] = H[g][b r + a] = scale sum_s w_s Phi_g(s) Phi_a(s) Phi_b(s),
-// one workgroup per a <= b: t = w Phi_a Phi_b in LDS chunks of GL_SC nodes,
-// wave q sums the columns g = q, q + 4, ... over its lanes (fixed order).
-// MIX (two fields): Phi_g from PhiG (rg columns) and the entries go to
-// H[b][g r + a] = H[a][g r + b] (the paired field's index first).
-constexpr int GL_SC = 1024;
-constexpr int GL_GW = 16;   // columns g per wave (r, rg <= 64)
-template <bool MIX>
-__global__ __launch_bounds__(256) void sep_gl_core(const double* __restrict__ Phi, const double* __restrict__ PhiG,
-                                                   int rg, int npt, const double* __restrict__ w, int r,
-                                                   double scale, double* __restrict__ H, long ldh)
-{
-    __shared__ double ts[GL_SC];
-    int a = 0, rem = blockIdx.x;   // pair (a, b), a <= b, row-major upper triangle
-    while (rem >= r - a) {
-        rem -= r - a;
-        ++a;
-    }
-    const int b = a + rem;
-    const int lane = threadIdx.x & 63, q = threadIdx.x >> 6;
-    double acc[GL_GW];
-#pragma unroll
-    for (int k = 0; k < GL_GW; ++k) acc[k] = 0.0;
-    for (int s0 = 0; s0 < npt; s0 += GL_SC) {
-        __syncthreads();
-        for (int e = threadIdx.x; e < GL_SC; e += 256) {
-            const int s = s0 + e;
-            ts[e] = s < npt ? w[s] * Phi[(long)a * npt + s] * Phi[(long)b * npt + s] : 0.0;
-        }
-        __syncthreads();
-        const int ns = min(GL_SC, npt - s0);
-#pragma unroll
-        for (int k = 0; k < GL_GW; ++k) {
-            const int g = q + 4 * k;
-            if (g < rg)
-                for (int e = lane; e < ns; e += 64) acc[k] = fma(PhiG[(long)g * npt + s0 + e], ts[e], acc[k]);
-        }
-    }
-#pragma unroll
-    for (int k = 0; k < GL_GW; ++k) {
-        const int g = q + 4 * k;
-        double t = acc[k];
-#pragma unroll
-        for (int o = 32; o >= 1; o >>= 1) t += __shfl_xor(t, o);
-        if (g < rg && lane == 0) {
-            if (MIX) {
-                H[(long)b * ldh + (long)g * r + a] = scale * t;
-                H[(long)a * ldh + (long)g * r + b] = scale * t;
-            } else {
-                H[(long)g * ldh + (long)a * r + b] = scale * t;
-                H[(long)g * ldh + (long)b * r + a] = scale * t;
-            }
-        }
-    }
-}
+constexpr int GL_RMAX = 64;   // columns of a compressed basis
 
 // One field of a compressed GL Gram whose three legs are that field: its
 // basis (the first R columns of q[l][col], nl rows from l = 0), per-leg
@@ -2094,6 +1989,14 @@ struct GlField3 {
 
 static int gl_compressed_run(mcmb_ctx* c, const GlField3& F, int npt, const double* x, const double* w,
                              double* d_gamma, bool* used);
+
+// The table of P_l is kept between calls up to GN_TABMAX.
+static void gl_half_trim(mcmb_ctx* c)
+{
+    if (c->glh.buf.bytes <= GN_TABMAX) return;
+    c->glh.buf.release();
+    c->glh.npt = 0;
+}
 
 int gram_gl_compressed(mcmb_ctx* c, int npt, const double* x, const double* w, double* d_gamma, bool* used)
 {
@@ -2132,32 +2035,22 @@ static int gl_compressed_run(mcmb_ctx* c, const GlField3& F, int npt, const doub
     MCMB_TRY(separable_compress(c, *F.S, F.B, nl, NP, ld, pxy));
     const SepComp& S = *F.S;
     const int r = S.r;
-    if (r <= 0 || r > 4 * GL_GW) return MCMB_OK;   // full rank: the direct node sum
+    if (r <= 0 || r > GL_RMAX) return MCMB_OK;   // full rank: the direct node sum
     const long ldh = (long)r * r + ((r * r) & 1);
-    MCMB_TRY(c->gl_xw.alloc(sizeof(double) * (2 * (size_t)npt + (size_t)r * npt + (size_t)r * S.nlp)));
-    double* const dx = c->gl_xw.as<double>();
-    double* const dw = dx + npt;
-    double* const dphi = dw + npt;
-    double* const dpw = dphi + (size_t)r * npt;
+    MCMB_TRY(gl_half_table(c, npt, nl - 1, x, w));
+    const size_t np = gl_phi64_size(c, nl, r);
+    MCMB_TRY(c->gl_ws.alloc(sizeof(double) * (np + gl_core64_size(c, r, r, true))));
     MCMB_TRY(sep_expand_alloc(c, r, NP, ld));
-    MCMB_HIP(hipMemcpyAsync(dx, x, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
-    MCMB_HIP(hipMemcpyAsync(dw, w, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
+    double *const ws = c->gl_ws.as<double>(), *phi;
     MCMB_HIP(hipEventRecord(c->ev0, c->stream));
-    const long ntab = (long)r * S.nlp;
-    hipLaunchKernelGGL(sep_gl_tabs, dim3((unsigned)((ntab + 255) / 256)), dim3(256), 0, c->stream,
-                       (const double*)S.pc.as<double>(), S.nlp, nl, r, F.lmin, F.d_v, dpw);
-    hipLaunchKernelGGL(sep_gl_phi, dim3((unsigned)((npt + 63) / 64), (unsigned)((r + 4 * GL_AG - 1) / (4 * GL_AG))),
-                       dim3(256), 0, c->stream, (const double*)dpw, S.nlp, nl, r, (const double*)dx, npt, dphi);
-    MCMB_HIP(hipMemsetAsync(S.h.p, 0, sizeof(double) * (size_t)r * ldh, c->stream));
-    hipLaunchKernelGGL(sep_gl_core<false>, dim3((unsigned)(r * (r + 1) / 2)), dim3(256), 0, c->stream,
-                       (const double*)dphi, (const double*)dphi, r, npt, (const double*)dw, r, 3.0 / (4.0 * M_PI),
-                       S.h.as<double>(), ldh);
-    MCMB_HIP(hipGetLastError());
+    MCMB_TRY(gl_phi64_launch(c, S.pc.as<double>(), S.nlp, nl, r, F.lmin, F.d_v, ws, &phi));
+    MCMB_TRY(gl_core64_launch(c, phi, r, phi, r, 3.0 / (4.0 * M_PI), ws + np, S.h.as<double>(), ldh));
     MCMB_TRY(sep_expand(c, S, NP, ld));
     MCMB_TRY(sep_assemble_launch(c, R, n, F.d_modes, d_gamma));
     MCMB_HIP(hipGetLastError());
     MCMB_HIP(hipEventRecord(c->ev1, c->stream));
-    MCMB_HIP(hipStreamSynchronize(c->stream));   // x and w may live on the caller's stack
+    MCMB_HIP(hipStreamSynchronize(c->stream));
+    gl_half_trim(c);
     float ms = 0.f;
     MCMB_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;
@@ -2205,7 +2098,7 @@ int gram_gl_mixed_compressed(mcmb_ctx* c, int pol, int RT, int RE, int npt, cons
     const SepComp& ST = c->sepc_pt;
     const SepComp& SE = c->sepc_e;
     const int rT = ST.r, rE = SE.r;
-    if (rT <= 0 || rT > 4 * GL_GW || rE <= 0 || rE > 4 * GL_GW) return MCMB_OK;   // the direct node sum
+    if (rT <= 0 || rT > GL_RMAX || rE <= 0 || rE > GL_RMAX) return MCMB_OK;   // the direct node sum
     // P: the field on two legs, S: the other
     const bool tte = pol == 1;
     const SepComp& SP = tte ? ST : SE;
@@ -2214,17 +2107,12 @@ int gram_gl_mixed_compressed(mcmb_ctx* c, int pol, int RT, int RE, int npt, cons
     const int ldP = tte ? ldT : ldE, ldS = tte ? ldE : ldT;
     const long NQ = (long)NPP_ * (NPP_ + 1) / 2, ldq = NQ + (NQ & 1);   // pair pairs of P
     const long ldh = (long)rS * rP + (((long)rS * rP) & 1);
-    // device work: x, w, Phi^T, Phi^E, the two weighted tables, H
-    const size_t nd = 2 * (size_t)npt + (size_t)(rT + rE) * npt + (size_t)rT * ST.nlp + (size_t)rE * SE.nlp +
-                      (size_t)rP * ldh;
-    MCMB_TRY(c->gl_xw.alloc(sizeof(double) * nd));
-    double* const dx = c->gl_xw.as<double>();
-    double* const dw = dx + npt;
-    double* const phT = dw + npt;
-    double* const phE = phT + (size_t)rT * npt;
-    double* const pwT = phE + (size_t)rE * npt;
-    double* const pwE = pwT + (size_t)rT * ST.nlp;
-    double* const H = pwE + (size_t)rE * SE.nlp;
+    // device work: T and Phi of either field, the core's units, H
+    MCMB_TRY(gl_half_table(c, npt, std::max(nlT, nlE) - 1, x, w));
+    const size_t npT = gl_phi64_size(c, nlT, rT), npE = gl_phi64_size(c, nlE, rE),
+                 nco = gl_core64_size(c, rP, rS, false);
+    MCMB_TRY(c->gl_ws.alloc(sizeof(double) * (npT + npE + nco + (size_t)rP * ldh)));
+    double *const wsT = c->gl_ws.as<double>(), *const wsE = wsT + npT, *const wsC = wsE + npE, *const H = wsC + nco;
     MCMB_TRY(c->sg_M.alloc(sizeof(double) * (size_t)((long)rS * rP * ldP)));
     MCMB_TRY(c->sg_Ys.alloc(sizeof(double) * (size_t)((long)rS * ldq)));
     MCMB_TRY(c->sg_G.alloc(sizeof(double) * (size_t)((long)NPS * ldq)));
@@ -2248,32 +2136,12 @@ int gram_gl_mixed_compressed(mcmb_ctx* c, int pol, int RT, int RE, int npt, cons
     MCMB_TRY(c->gl_tab.alloc(sizeof(int) * buf.size()));
     const int* tb = c->gl_tab.as<int>();
     MCMB_HIP(hipMemcpyAsync(c->gl_tab.p, buf.data(), sizeof(int) * buf.size(), hipMemcpyHostToDevice, c->stream));
-    MCMB_HIP(hipMemcpyAsync(dx, x, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
-    MCMB_HIP(hipMemcpyAsync(dw, w, sizeof(double) * npt, hipMemcpyHostToDevice, c->stream));
     MCMB_HIP(hipEventRecord(c->ev0, c->stream));
-    // the compressed bases at the nodes
-    struct Fd {
-        const SepComp* S;
-        int nl, lmin;
-        const double* v;
-        double *pw, *ph;
-    };
-    const Fd fd[2] = {{&ST, nlT, L.lmin, L.d_v.as<double>(), pwT, phT}, {&SE, nlE, E.lmin, E.d_v.as<double>(), pwE, phE}};
-    for (const Fd& f : fd) {
-        const int r = f.S->r;
-        const long ntab = (long)r * f.S->nlp;
-        hipLaunchKernelGGL(sep_gl_tabs, dim3((unsigned)((ntab + 255) / 256)), dim3(256), 0, c->stream,
-                           (const double*)f.S->pc.as<double>(), f.S->nlp, f.nl, r, f.lmin, f.v, f.pw);
-        hipLaunchKernelGGL(sep_gl_phi, dim3((unsigned)((npt + 63) / 64), (unsigned)((r + 4 * GL_AG - 1) / (4 * GL_AG))),
-                           dim3(256), 0, c->stream, (const double*)f.pw, f.S->nlp, f.nl, r, (const double*)dx, npt,
-                           f.ph);
-    }
-    const double* const phP = tte ? phT : phE;
-    const double* const phS = tte ? phE : phT;
-    MCMB_HIP(hipMemsetAsync(H, 0, sizeof(double) * (size_t)rP * ldh, c->stream));
-    hipLaunchKernelGGL(sep_gl_core<true>, dim3((unsigned)(rP * (rP + 1) / 2)), dim3(256), 0, c->stream, phP, phS, rS,
-                       npt, (const double*)dw, rP, 1.0 / (16.0 * M_PI), H, ldh);
-    MCMB_HIP(hipGetLastError());
+    // the compressed bases at the nodes, and the core
+    double *phT, *phE;
+    MCMB_TRY(gl_phi64_launch(c, ST.pc.as<double>(), ST.nlp, nlT, rT, L.lmin, L.d_v.as<double>(), wsT, &phT));
+    MCMB_TRY(gl_phi64_launch(c, SE.pc.as<double>(), SE.nlp, nlE, rE, E.lmin, E.d_v.as<double>(), wsE, &phE));
+    MCMB_TRY(gl_core64_launch(c, tte ? phT : phE, rP, tte ? phE : phT, rS, 1.0 / (16.0 * M_PI), wsC, H, ldh));
     double* const T1 = c->sg_M.as<double>();
     double* const Y = c->sg_Ys.as<double>();
     double* const K = c->sg_G.as<double>();
@@ -2307,7 +2175,8 @@ int gram_gl_mixed_compressed(mcmb_ctx* c, int pol, int RT, int RE, int npt, cons
                            (const double*)K, ldq, RT, RE, E.d_modes[1].as<int>(), n, nt, d_gamma);
     MCMB_HIP(hipGetLastError());
     MCMB_HIP(hipEventRecord(c->ev1, c->stream));
-    MCMB_HIP(hipStreamSynchronize(c->stream));   // x, w and the tables may live on the host stack
+    MCMB_HIP(hipStreamSynchronize(c->stream));   // the tables live on the host stack
+    gl_half_trim(c);
     float ms = 0.f;
     MCMB_HIP(hipEventElapsedTime(&ms, c->ev0, c->ev1));
     c->last_ms = ms;

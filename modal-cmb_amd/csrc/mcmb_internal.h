@@ -220,6 +220,13 @@ struct GlTable {
     DevBuf buf;
     dd *w = nullptr, *P = nullptr;
 };
+// FP64 half rule (weights at +x, then at -x) and P_l at its nodes, P[l][SH],
+// of the Gauss-Legendre Gram over compressed bases, for the last (npt, lmax).
+struct GlHalf {
+    int npt = 0, lmax = -1, SH = 0;
+    DevBuf buf;
+    double *w = nullptr, *P = nullptr;
+};
 constexpr int GN_RMAX = 64;                    // columns of the node form, the gate's included
 constexpr int GN_LMIN = 512;                   // the node form takes lmax above this
 constexpr size_t GN_TABMAX = (size_t)1 << 30;  // bytes of the table of P_l
@@ -317,11 +324,12 @@ struct mcmb_ctx {
     // step (rocsolver_dstedc), created on first use
     void* rb_handle = nullptr;
     mcmb::TrdWork trd;
-    // the GL Gram over the compressed basis: node table and Phi
-    mcmb::DevBuf gl_xw;
+    // the GL Gram over compressed bases: T, Phi and the core's units
+    mcmb::DevBuf gl_ws;
     // the node form of the tetrapyd Gram: rule and Legendre table, work space,
     // the gate's two sums (pinned), and the setup that did not pass it
     mcmb::GlTable glt;
+    mcmb::GlHalf glh;
     mcmb::DevBuf gn_ws;
     double* gn_gate = nullptr;
     long gn_refused = -1;
@@ -440,6 +448,15 @@ bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool
 int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, int nl, int r, double* H, long ldh,
                     const std::function<int(const char*)>& phase);
 bool gl_gate(const mcmb_ctx* c, int lmax);
+// The FP64 node sum over compressed bases (gram_nodes.hip): the half rule's
+// table, Phi of a basis, the core tensor, and their work sizes in doubles.
+int gl_half_table(mcmb_ctx* c, int npt, int lmax, const double* x, const double* w);
+size_t gl_phi64_size(const mcmb_ctx* c, int nl, int r);
+int gl_phi64_launch(mcmb_ctx* c, const double* Pc, int nlp, int nl, int r, int lmin, const double* v, double* ws,
+                    double** phi);
+size_t gl_core64_size(const mcmb_ctx* c, int rP, int rS, bool same);
+int gl_core64_launch(mcmb_ctx* c, const double* phP, int rP, const double* phS, int rS, double scale, double* ws,
+                     double* H, long ldh);
 bool gram_separable_supported(const PointSet& P, int precision);
 int gram_separable_launch(mcmb_ctx* ctx, PointSet& P, int precision, double* d_gamma, int row_lo, int row_hi);
 }  // namespace mcmb
