@@ -6,6 +6,7 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <exception>
 
 namespace mcmb {
 
@@ -54,12 +55,11 @@ int set_device(mcmb_ctx* ctx)
     return MCMB_OK;
 }
 
-// Allocate the pinned staging halves and their events on first use.
+// Allocate the pinned staging on first use.
 int stage_ready(mcmb_ctx* c)
 {
     if (c->stage) return MCMB_OK;
     MCMB_HIP(hipHostMalloc(&c->stage, 2 * STAGE_BYTES, hipHostMallocDefault));
-    for (int k = 0; k < 2; ++k) MCMB_HIP(hipEventCreateWithFlags(&c->stage_ev[k], hipEventDisableTiming));
     return MCMB_OK;
 }
 
@@ -73,71 +73,159 @@ int copy_stream_ready(mcmb_ctx* c)
     return MCMB_OK;
 }
 
+// The staged copies cut the bytes into chunks that go round CSLOTS slots of
+// pinned memory of their own: the DMA of a chunk and the host threads' move of the
+// others overlap.  The threads live for the whole copy, each moving its stripe
+// of every chunk; progress is two counters, so no thread waits for a lock.
+// Copying a fresh 19 MB array out (its pages are touched for the first time
+// here, by all threads): 1.1 -> 0.6 ms against one pageable hipMemcpy; 1 MB
+// took 0.06 ms longer (starting the threads), hence COPY_MIN.  Below COPY_BIG
+// the slots are four of 2 MiB, since pinning costs 40 us a MiB on a context's
+// first copy; above, eight of 4 MiB in the staging (197 MB in and out twice: 24
+// ms, 31 ms through slots of 1 MiB).
+constexpr size_t COPY_BIG = 2 * STAGE_BYTES, CSTAGE_BYTES = (size_t)8 << 20;
+constexpr size_t COPY_MIN_OUT = (size_t)8 << 20, COPY_MIN_IN = (size_t)4 << 20;
+
+namespace {
+struct ChunkCrew {
+    const int nth;
+    std::vector<std::atomic<int>> done;   // threads that have moved chunk k
+    std::atomic<long> ready{0};           // chunks the threads may move
+    std::atomic<bool> stop{false};
+    std::vector<std::thread> th;
+
+    template <class F> ChunkCrew(int n, size_t nk, F move) : nth(n), done(nk)
+    {
+        for (auto& d : done) d.store(0, std::memory_order_relaxed);
+        th.reserve(n);
+        try {
+            for (int t = 0; t < n; ++t)
+                th.emplace_back([this, t, nk, move] {
+                    for (size_t k = 0; k < nk; ++k) {
+                        while (ready.load(std::memory_order_acquire) <= (long)k) {
+                            if (stop.load(std::memory_order_relaxed)) return;
+                            std::this_thread::yield();
+                        }
+                        move(t, k);
+                        done[k].fetch_add(1, std::memory_order_release);
+                    }
+                });
+        } catch (...) {   // no further thread to be had
+            join();
+            throw;
+        }
+    }
+    void join()
+    {
+        stop.store(true);
+        for (auto& x : th) x.join();
+    }
+    void wait(size_t k) const
+    {
+        while (done[k].load(std::memory_order_acquire) < nth) std::this_thread::yield();
+    }
+    ~ChunkCrew() { join(); }
+};
+}  // namespace
+
+static int staged_copy(mcmb_ctx* c, char* host, char* dev, size_t bytes, bool to_host)
+{
+    const bool big = bytes >= COPY_BIG;
+    if (big) MCMB_TRY(stage_ready(c));
+    else if (!c->copy_stage) MCMB_HIP(hipHostMalloc(&c->copy_stage, CSTAGE_BYTES, hipHostMallocDefault));
+    for (hipEvent_t& e : c->copy_ev)
+        if (!e) MCMB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    char* const stage = static_cast<char*>(big ? c->stage : c->copy_stage);
+    const size_t CSLOTS = big ? PSLOTS : 4, lag = CSLOTS / 2, slot = (big ? 2 * STAGE_BYTES : CSTAGE_BYTES) / CSLOTS,
+                 chunk = slot;
+    const size_t nk = (bytes + chunk - 1) / chunk;
+    const int nth = std::min(8, host_threads());
+    auto len = [&](size_t k) { return std::min(chunk, bytes - k * chunk); };
+    auto dma = [&](size_t k) -> int {
+        char* const sl = stage + (k % CSLOTS) * slot;
+        if (to_host) MCMB_HIP(hipMemcpyAsync(sl, dev + k * chunk, len(k), hipMemcpyDeviceToHost, c->stream));
+        else MCMB_HIP(hipMemcpyAsync(dev + k * chunk, sl, len(k), hipMemcpyHostToDevice, c->stream));
+        MCMB_HIP(hipEventRecord(c->copy_ev[k % CSLOTS], c->stream));
+        return MCMB_OK;
+    };
+    auto landed = [&](size_t k) -> int {
+        MCMB_HIP(hipEventSynchronize(c->copy_ev[k % CSLOTS]));
+        return MCMB_OK;
+    };
+    ChunkCrew crew(nth, nk, [=](int t, size_t k) {
+        const size_t n = std::min(chunk, bytes - k * chunk), a = (n * t / nth) & ~(size_t)63,
+                     b = t + 1 == nth ? n : (n * (t + 1) / nth) & ~(size_t)63;
+        char *const h = host + k * chunk + a, *const sl = stage + (k % CSLOTS) * slot + a;
+        if (to_host) memcpy(h, sl, b - a);
+        else memcpy(sl, h, b - a);
+    });
+    if (to_host) {
+        size_t issued = 0;
+        for (; issued < std::min<size_t>(nk, CSLOTS); ++issued) MCMB_TRY(dma(issued));
+        for (size_t k = 0; k < nk; ++k) {
+            MCMB_TRY(landed(k));
+            crew.ready.store((long)k + 1, std::memory_order_release);
+            // chunk k - lag's slot again: its move is most likely over
+            if (k >= lag && issued < nk) {
+                crew.wait(issued - CSLOTS);
+                MCMB_TRY(dma(issued));
+                ++issued;
+            }
+        }
+        crew.wait(nk - 1);   // (and, thread by thread, every chunk before it)
+    } else {
+        crew.ready.store((long)std::min<size_t>(nk, CSLOTS), std::memory_order_release);
+        for (size_t k = 0; k < nk; ++k) {
+            crew.wait(k);
+            MCMB_TRY(dma(k));
+            // chunk k - lag's slot is free for chunk k + lag once its DMA has read it
+            if (k >= lag && k + lag < nk) {
+                MCMB_TRY(landed(k - lag));
+                crew.ready.store((long)(k + lag) + 1, std::memory_order_release);
+            }
+        }
+        MCMB_HIP(hipStreamSynchronize(c->stream));
+    }
+    return MCMB_OK;
+}
+
+static int plain_copy(mcmb_ctx* c, void* dst, const void* src, size_t bytes, hipMemcpyKind kind)
+{
+    MCMB_HIP(hipMemcpyAsync(dst, src, bytes, kind, c->stream));
+    MCMB_HIP(hipStreamSynchronize(c->stream));
+    return MCMB_OK;
+}
+
+static bool copy_staged(size_t bytes, size_t least)
+{
+    const char* env = getenv("MCMB_HOST_COPY");
+    return bytes >= least && !(env && !strcmp(env, "direct"));
+}
+
 int copy_to_device(mcmb_ctx* c, void* dev, const void* host, size_t bytes)
 {
     if (!bytes) return MCMB_OK;
-    const char* env = getenv("MCMB_HOST_COPY");
-    if (bytes < STAGE_BYTES / 4 || (env && !strcmp(env, "direct"))) {
-        MCMB_HIP(hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, c->stream));
-        MCMB_HIP(hipStreamSynchronize(c->stream));
-        return MCMB_OK;
+    if (copy_staged(bytes, COPY_MIN_IN)) {
+        try {
+            return staged_copy(c, const_cast<char*>(static_cast<const char*>(host)), static_cast<char*>(dev), bytes, false);
+        } catch (const std::exception&) {   // no thread or memory to be had: copy without them
+            MCMB_HIP(hipStreamSynchronize(c->stream));
+        }
     }
-    MCMB_TRY(stage_ready(c));
-    char* const stage = static_cast<char*>(c->stage);
-    const char* const src = static_cast<const char*>(host);
-    char* const dst = static_cast<char*>(dev);
-    const size_t nk = (bytes + STAGE_BYTES - 1) / STAGE_BYTES;
-    const int nth = std::min(8, host_threads());
-    for (size_t k = 0; k < nk; ++k) {
-        // half k & 1 is free once the DMA of chunk k - 2 has read it
-        if (k >= 2) MCMB_HIP(hipEventSynchronize(c->stage_ev[k & 1]));
-        const size_t off = k * STAGE_BYTES, len = std::min(STAGE_BYTES, bytes - off);
-        char* half = stage + (k & 1) * STAGE_BYTES;
-        run_threads(nth, [&](int t) {
-            const size_t a = len * t / nth, b = len * (t + 1) / nth;
-            memcpy(half + a, src + off + a, b - a);
-        });
-        MCMB_HIP(hipMemcpyAsync(dst + off, half, len, hipMemcpyHostToDevice, c->stream));
-        MCMB_HIP(hipEventRecord(c->stage_ev[k & 1], c->stream));
-    }
-    MCMB_HIP(hipStreamSynchronize(c->stream));
-    return MCMB_OK;
+    return plain_copy(c, dev, host, bytes, hipMemcpyHostToDevice);
 }
 
 int copy_to_host(mcmb_ctx* c, void* host, const void* dev, size_t bytes)
 {
     if (!bytes) return MCMB_OK;
-    const char* env = getenv("MCMB_HOST_COPY");
-    if (bytes < 2 * STAGE_BYTES || (env && !strcmp(env, "direct"))) {
-        MCMB_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
-        MCMB_HIP(hipStreamSynchronize(c->stream));
-        return MCMB_OK;
+    if (copy_staged(bytes, COPY_MIN_OUT)) {
+        try {
+            return staged_copy(c, static_cast<char*>(host), const_cast<char*>(static_cast<const char*>(dev)), bytes, true);
+        } catch (const std::exception&) {
+            MCMB_HIP(hipStreamSynchronize(c->stream));
+        }
     }
-    MCMB_TRY(stage_ready(c));
-    char* const stage = static_cast<char*>(c->stage);
-    const char* const src = static_cast<const char*>(dev);
-    char* const dst = static_cast<char*>(host);
-    const size_t nk = (bytes + STAGE_BYTES - 1) / STAGE_BYTES;
-    auto issue = [&](size_t k) -> int {
-        const size_t off = k * STAGE_BYTES, len = std::min(STAGE_BYTES, bytes - off);
-        MCMB_HIP(hipMemcpyAsync(stage + (k & 1) * STAGE_BYTES, src + off, len, hipMemcpyDeviceToHost, c->stream));
-        MCMB_HIP(hipEventRecord(c->stage_ev[k & 1], c->stream));
-        return MCMB_OK;
-    };
-    const int nth = std::min(8, host_threads());
-    MCMB_TRY(issue(0));
-    for (size_t k = 0; k < nk; ++k) {
-        // half (k + 1) & 1 was emptied into host memory at step k - 1
-        if (k + 1 < nk) MCMB_TRY(issue(k + 1));
-        MCMB_HIP(hipEventSynchronize(c->stage_ev[k & 1]));
-        const size_t off = k * STAGE_BYTES, len = std::min(STAGE_BYTES, bytes - off);
-        const char* half = stage + (k & 1) * STAGE_BYTES;
-        run_threads(nth, [&](int t) {
-            const size_t a = len * t / nth, b = len * (t + 1) / nth;
-            memcpy(dst + off + a, half + a, b - a);
-        });
-    }
-    return MCMB_OK;
+    return plain_copy(c, host, dev, bytes, hipMemcpyDeviceToHost);
 }
 
 // Rows of T(lmin, lmax) in the order get_ijk_next_XXX walks them
@@ -277,9 +365,10 @@ int mcmb_destroy(mcmb_ctx* c)
     c->d_aux.release();
     tridiag_release(c);
     if (c->stage) (void)hipHostFree(c->stage);
+    if (c->copy_stage) (void)hipHostFree(c->copy_stage);
+    for (hipEvent_t e : c->copy_ev)
+        if (e) (void)hipEventDestroy(e);
     if (c->gn_gate) (void)hipHostFree(c->gn_gate);
-    for (int k = 0; k < 2; ++k)
-        if (c->stage_ev[k]) (void)hipEventDestroy(c->stage_ev[k]);
     for (int h = 0; h < 2; ++h)
         for (int k = 0; k < PSLOTS; ++k)
             if (c->slot_ev[h][k]) (void)hipEventDestroy(c->slot_ev[h][k]);

@@ -308,10 +308,13 @@ struct mcmb_ctx {
     const char* phase_names[mcmb::MAX_PHASES] = {};
     // host wall time of the parts of the last Gram call (setup and the whole
     // call), in call order
-    // pinned staging of large device -> host copies: two halves of
-    // STAGE_BYTES, allocated on first use
+    // pinned slots of the staged copies (copy_to_host, copy_to_device) and
+    // their events, made on first use
+    void* copy_stage = nullptr;
+    hipEvent_t copy_ev[mcmb::PSLOTS] = {};
+    // pinned staging of the projection's and the eigensolver's transfers, two
+    // halves of STAGE_BYTES, allocated on first use
     void* stage = nullptr;
-    hipEvent_t stage_ev[2] = {};
     // copies that overlap the context stream's work, and the events of the
     // projection's per-batch slots of the staging (made on first use)
     hipStream_t cstream = nullptr;
@@ -402,17 +405,14 @@ int gram_gl_mixed_compressed(mcmb_ctx* ctx, int pol, int RT, int RE, int npt, co
 int gl_scratch_setup(int device);
 int set_device(mcmb_ctx* ctx);
 // Copy bytes from device memory dev (written by work on the context stream)
-// to host memory, returning when the host copy is complete.  Copies of 32 MiB
-// and more go through the context's pinned staging, 16 MiB halves: the next
-// half is copied from the device while host threads move the previous one,
-// which is 3x to 4x the rate of a pageable hipMemcpy.
+// to host memory, returning when the host copy is complete.  Copies of 8 MiB
+// and more go through pinned slots of the context in chunks: host threads
+// move the chunks that have arrived while the next ones are copied.
 int copy_to_host(mcmb_ctx* ctx, void* host, const void* dev, size_t bytes);
-// The reverse, host -> device (4 MiB and more staged: host threads fill one
-// half while the other is copied to the device).
+// The reverse, host -> device (4 MiB and more in chunks).
 int copy_to_device(mcmb_ctx* ctx, void* dev, const void* host, size_t bytes);
 // The context's pinned staging (2 x STAGE_BYTES at ctx->stage), allocated on
-// first use.  Callers other than the two copies above may use it between
-// their own stream synchronisations.
+// first use, for the transfers of the projection and the eigensolver.
 constexpr size_t STAGE_BYTES = (size_t)16 << 20;
 int stage_ready(mcmb_ctx* ctx);
 // The staging, the context's copy stream (default priority) and the slot
