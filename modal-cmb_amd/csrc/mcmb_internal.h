@@ -336,6 +336,8 @@ struct mcmb_ctx {
     mcmb::DevBuf gn_ws;
     double* gn_gate = nullptr;
     long gn_refused = -1;
+    // work buffers of the Cholesky orthonormalisation and solve
+    mcmb::DevBuf la_ws;
     // the GL cross-Gamma: node tables, M and the core tensor
     mcmb::DevBuf cx_ws;
     // the last Gauss-Legendre rule the Grams asked for (gl_nodes)

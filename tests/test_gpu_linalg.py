@@ -64,6 +64,55 @@ def test_orthonormalise_inverse_is_exact_triangle(ctx):
     assert np.abs(P - np.eye(n)).max() < 1e-11
 
 
+@pytest.mark.parametrize("n", [127, 128, 129, 191, 321, 2049, 2900])
+def test_orthonormalise_block_edges(ctx, n):
+    """Sizes around the 64-column blocks, the pairs that the inverse joins (a
+    last pair without or with a short second block) and the 128-wide tiles:
+    both triangles against the matrix itself.  1e-11: rounding of n-term sums at
+    condition 1e3, as test_orthonormalise_inverse_is_exact_triangle."""
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n + 50)) * np.exp(-3.0 * np.arange(n + 50) / n)
+    G = A @ A.T + 0.05 * n * np.eye(n)
+    d = rng.uniform(0.5, 3.0, n)
+    G = G * np.outer(d, d)
+    ortho, lam, norm = ctx.orthonormalise(G)
+    F, Lam = np.tril(ortho), np.tril(lam)
+    assert np.array_equal(ortho, ortho.T) and np.array_equal(lam, lam.T)
+    assert np.abs(F @ F.T - G).max() < 1e-13 * np.abs(G).max()
+    assert np.abs(Lam @ F - np.eye(n)).max() < 1e-11
+    C = rng.standard_normal((n, 5))
+    assert np.abs(ctx.cholesky_solve(ortho, G @ C) - C).max() < 1e-10
+
+
+@pytest.mark.parametrize("bad", [0, 15, 16, 63, 64, 127, 200, 255])
+def test_not_spd_pivot_positions(ctx, bad):
+    """A dependent row at every edge of the panels and blocks is reported at its
+    own column, and a later call on a good matrix is not affected."""
+    n = 256
+    G = spd(n, 3, cond=10)
+    H = G.copy()
+    H[bad, bad] = -1.0 if bad == 0 else (H[bad, :bad] @ np.linalg.solve(H[:bad, :bad], H[:bad, bad])) * (1 - 1e-3)
+    if bad == 0:
+        with pytest.raises(modalcmb.ModalError):
+            ctx.orthonormalise(H)
+    else:
+        with pytest.raises(modalcmb.NotSPDError) as e:
+            ctx.orthonormalise(H)
+        assert f"pivot {bad})" in str(e.value)
+    ortho, _, _ = ctx.orthonormalise(G)
+    assert np.abs(np.tril(ortho) @ np.tril(ortho).T - G).max() < 1e-13 * np.abs(G).max()
+
+
+@pytest.mark.parametrize("n,nrhs", [(64, 1), (65, 4), (200, 5), (129, 128), (129, 129), (1000, 9)])
+def test_cholesky_solve_block_steps(ctx, n, nrhs):
+    """Few right-hand sides (a launch per block of 64, groups of four) and the
+    first count past them, against the matrix."""
+    G = spd(n, 4, cond=1e2)
+    ortho, _, _ = ctx.orthonormalise(G)
+    C = np.random.default_rng(n).standard_normal((n, nrhs))
+    assert np.abs(ctx.cholesky_solve(ortho, G @ C) - C).max() < 1e-11
+
+
 def test_lmax500_gram_orthonormalisation_status(ctx):
     # The lmax-500 Gram (r<=s<=t<10 Legendre modes, weight h^2/C^3) has
     # kappa(D^-1 G D^-1) ~ 1e17 > 1/eps: whether FP64 Cholesky meets a
