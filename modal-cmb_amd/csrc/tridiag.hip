@@ -9,7 +9,7 @@
 //
 // Tridiagonalisation (the lower form of LAPACK dsytrd / dlatrd, in panels of
 // TRD_NB columns).  A is kept full and symmetric, row-major; row j stands for
-// column j.  Column j = k0 + i of a panel takes three kernels:
+// column j.  Column j = k0 + i of a panel takes two kernels:
 //   trd_row   x = A[j][j..n) - sum_{p<i} (V_p[c] W_p[j] + W_p[c] V_p[j])
 //             (the panel's earlier reflectors, not yet in A), d_j = x_j, and
 //             per workgroup its part of |x_{j+2..}|^2;
@@ -18,9 +18,9 @@
 //             v = x / (x_{j+1} - beta) with v_{j+1} = 1 (tau = 0 when
 //             x_{j+2..n) = 0), e_j = beta; then y = A v over rows j+1.. and
 //             per workgroup its parts of V_p^T v, W_p^T v and y^T v;
-//   trd_symv_fin  those parts added: w = tau (y - V (W^T v) - W (V^T v)) +
-//             alpha2 v with alpha2 = -tau/2 (w^T v), kept as y, the two dot
-//             vectors and alpha2 until the next trd_row makes w final.
+//             The next trd_row (trd_wfinal after a panel's last column) adds
+//             those parts and makes w = tau (y - V (W^T v) - W (V^T v)) +
+//             alpha2 v, alpha2 = -tau/2 (w^T v), final.
 // Partial sums are added in workgroup order, so results do not depend on
 // timing, and no workgroup waits for another.  At the end of a panel the
 // trailing matrix takes A -= V W^T + W V^T on FP64 MFMA (lower tiles,
@@ -47,17 +47,15 @@ constexpr int TRD_NB = 32;           // reflectors per panel
 constexpr int TRD_MAXN = 8000;       // v of a column staged in LDS (under 64 KiB with the static part)
 constexpr int TRD_ROWT = 256;        // trd_row threads
 constexpr int TRD_SYMT = 512;        // trd_symv threads
-constexpr int TRD_SYMG = 1024;       // most trd_symv workgroups
+constexpr int TRD_SYMG = 512;        // most trd_symv workgroups (TRD_RW2 / 16, TRD_MAXN / 32)
+constexpr int TRD_RW2 = 4096;        // rows up to which a trd_symv wave takes two of them
 
 typedef double fd4 __attribute__((ext_vector_type(4)));
 
-// Device-side state of the current column and panel.
+// Device-side state of the current column.
 struct TrdState {
     double tau;
     double alpha;               // x_{j+1}
-    double c1[TRD_NB];          // V_p^T v
-    double c2[TRD_NB];          // W_p^T v
-    double alpha2[TRD_NB];      // w_p += alpha2[p] v_p, p of the panel
 };
 
 __device__ __forceinline__ double wave_sum(double v)
@@ -102,15 +100,21 @@ __device__ __forceinline__ void trd_sum_parts(int i, int nb, const double* __res
     const int q = tid >> 2, sub = tid & 3;
     double s = 0.0;
     if (q < 1 + 2 * i)
-        for (int b = sub; b < nb; b += 4) s += part[(long)q * TRD_SYMG + b];
+        for (int b0 = sub; b0 < nb; b0 += 64) {   // 16 loads in flight
+            double v[16];
+#pragma unroll
+            for (int u = 0; u < 16; ++u) v[u] = b0 + 4 * u < nb ? part[(long)q * TRD_SYMG + b0 + 4 * u] : 0.0;
+#pragma unroll
+            for (int u = 0; u < 16; ++u) s += v[u];
+        }
     s += __shfl_xor(s, 1);
     s += __shfl_xor(s, 2);
     if (q < 1 + 2 * i && sub == 0) tot[q] = s;
 }
-__device__ __forceinline__ double trd_alpha2(int i, double tau, const double* tot)
+// by one wave: alpha2 in every lane
+__device__ __forceinline__ double trd_alpha2(int i, double tau, const double* tot, int lane)
 {
-    double cc = 0.0;
-    for (int p = 0; p < i; ++p) cc = fma(tot[1 + p], tot[1 + i + p], cc);
+    const double cc = wave_sum(lane < i ? tot[1 + lane] * tot[1 + i + lane] : 0.0);
     return -0.5 * tau * (tau * (tot[0] - 2.0 * cc));
 }
 
@@ -119,7 +123,9 @@ __device__ __forceinline__ double trd_alpha2(int i, double tau, const double* to
 // x = A[j][j..) - sum_{p<i} (V_p W_p[j] + W_p V_p[j]), d_j, and each
 // workgroup's part of |x_{j+2..}|^2 (trd_symv adds them and forms the
 // reflector).
-// Vp, Wp: the panel's rows (V_p at Vp + p n, W_p at Wp + p n).
+// Vp, Wp: the panel's rows (V_p at Vp + p n, W_p at Wp + p n).  A launch per
+// column, bound by its dependent memory round trips: everything that does not
+// depend on the sums is loaded before them (7.4 -> 6.2 us at n = 2300).
 __global__ __launch_bounds__(TRD_ROWT) void trd_row(const double* __restrict__ A, int lda, int n, int j, int i,
                                                    const double* __restrict__ Vp, double* __restrict__ Wp,
                                                    const double* __restrict__ tt, double* __restrict__ xbuf,
@@ -130,7 +136,7 @@ __global__ __launch_bounds__(TRD_ROWT) void trd_row(const double* __restrict__ A
     static_assert(TRD_ROWT == 256, "trd_sum_parts takes 256 threads");
     __shared__ double sV[TRD_NB], sW[TRD_NB];
     __shared__ double tot[2 * TRD_NB + 1];
-    __shared__ double red[TRD_ROWT / 64];
+    __shared__ double red[TRD_ROWT / 64], sa2;
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const int q = i - 1;   // the column whose W becomes final here (none when i = 0)
     // this thread's column: its loads issued first, in flight during the sums below
@@ -145,26 +151,28 @@ __global__ __launch_bounds__(TRD_ROWT) void trd_row(const double* __restrict__ A
     }
     const double vq = (cin && q >= 0) ? Vp[(long)q * n + c] : 0.0;
     const double wqr = (cin && q >= 0) ? Wp[(long)q * n + c] : 0.0;
+    const double vj = tid < i ? Vp[(long)tid * n + j] : 0.0, wj = tid < i ? Wp[(long)tid * n + j] : 0.0;
+    const double tq = q >= 0 ? tt[j - 1] : 0.0;
     // column q's sums, from trd_symv's partials (the same in every workgroup)
     if (q >= 0) trd_sum_parts(q, snb, spart, tid, tot);
-    if (tid < i) sV[tid] = Vp[(long)tid * n + j];
-    if (tid < q) sW[tid] = Wp[(long)tid * n + j];
+    if (tid < i) {
+        sV[tid] = vj;
+        sW[tid] = wj;   // W_q[j] not final yet
+    }
     __syncthreads();
     const double* const c1 = tot + 1;
     const double* const c2 = tot + 1 + (q > 0 ? q : 0);
-    double tq = 0.0, a2q = 0.0;
-    if (q >= 0) {
-        tq = tt[j - 1];
-        a2q = trd_alpha2(q, tq, tot);
-    }
     if (q >= 0 && w == 0) {
-        // W_q[j] final: lane p < q adds its correction term, then the wave tree
-        double t = 0.0;
-        if (lane < q) t = Vp[(long)lane * n + j] * c2[lane] + sW[lane] * c1[lane];
-        t = wave_sum(t);
-        if (lane == 0) sW[q] = tq * (Wp[(long)q * n + j] - t) + a2q * sV[q];
+        // alpha2_q, and W_q[j] final: lane p < q adds its correction term, then the wave tree
+        const double t = wave_sum(lane < q ? sV[lane] * c2[lane] + sW[lane] * c1[lane] : 0.0);
+        const double a2 = trd_alpha2(q, tq, tot, lane);
+        if (lane == 0) {
+            sW[q] = tq * (sW[q] - t) + a2 * sV[q];
+            sa2 = a2;
+        }
     }
     __syncthreads();
+    const double a2q = q >= 0 ? sa2 : 0.0;
     if (cin) {
         // one pass over the final W_p, V_p (p < q): the row update and W_q's correction
         double corr = 0.0;
@@ -203,9 +211,12 @@ __global__ __launch_bounds__(TRD_ROWT) void trd_row(const double* __restrict__ A
 // columns j+1+peel, j+2+peel of every row (peel = (j+1) & 1) are one aligned
 // pair), stored in W_i, v stored as V_j; and the sums c1[p] = V_p^T v,
 // c2[p] = W_p^T v (p < i, lane p of each wave) and y^T v over the
-// workgroups.  The last workgroup forms alpha2 = -tau/2 w^T v with
-// w^T v = tau (y^T v - 2 c1 . c2) (w = tau (y - V c2 - W c1) is made final
-// by the next trd_row).
+// workgroups (w = tau (y - V c2 - W c1) + alpha2 v is made final by the next
+// trd_row).  Bound by latency below n of a few thousand: the loads that do not
+// need the reflector are in flight while it is formed, and two rows a wave up
+// to TRD_RW2 rows spread the matrix over twice the CUs (10.7 -> 9.4 -> 7.5 us a
+// column at n = 2300; above, four rows a wave leave half the partial sums).
+template <int RW>
 __global__ __launch_bounds__(TRD_SYMT) void trd_symv(const double* __restrict__ A, int lda, int n, int j, int i,
                                                     const double* __restrict__ xbuf, const double* __restrict__ Vp,
                                                     double* __restrict__ Wp, double* __restrict__ Vj,
@@ -213,17 +224,49 @@ __global__ __launch_bounds__(TRD_SYMT) void trd_symv(const double* __restrict__ 
                                                     double* __restrict__ tt, TrdState* __restrict__ st,
                                                     double* __restrict__ part)
 {
-    constexpr int NWV = TRD_SYMT / 64, NQ = 2 * TRD_NB + 1, RW = 4, DP = 4;
+    constexpr int NWV = TRD_SYMT / 64, NQ = 2 * TRD_NB + 1, DP = 4;
+    constexpr int XR = (TRD_MAXN + TRD_SYMT - 1) / TRD_SYMT;
     extern __shared__ double vs[];
     __shared__ double red[NWV][NQ];
     __shared__ double rs;
     const int m = n - j - 1, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    // Loads that do not depend on the reflector, before it is formed: the
+    // first steps of the wave's RW rows of A, V_p and W_p at those rows, and
+    // this thread's part of x.  (The grid has a wave for every RW rows.)
+    const int r0 = RW * (blockIdx.x * NWV + w);
+    const bool live = r0 < m;
+    const int peel = (j + 1) & 1, npair = (m - peel) >> 1, tail = (m - peel) & 1, ns = (npair + 63) >> 6;
+    const double2* Ap[RW];
+    double2 ring[DP][RW];
+    double e0[RW], e1[RW], vp[RW], wp[RW];
+#pragma unroll
+    for (int k = 0; k < RW; ++k) {
+        const int rr = min(r0 + k, m - 1), r = j + 1 + rr;
+        const double* const Ar = A + (long)r * lda + (j + 1);
+        Ap[k] = reinterpret_cast<const double2*>(Ar + peel);
+        e0[k] = live && lane == 0 && peel ? Ar[0] : 0.0;
+        e1[k] = live && lane == 0 && tail ? Ar[m - 1] : 0.0;
+        vp[k] = live && lane < i ? Vp[(long)lane * n + r] : 0.0;
+        wp[k] = live && lane < i ? Wp[(long)lane * n + r] : 0.0;
+    }
+    // steps s of the wave (t = lane + 64 s; lanes past npair read the last pair
+    // and weigh it by zero, so the loop is uniform), loaded DP steps ahead into
+    // a ring of registers (slot d holds step s0 + d)
+    if (live && ns > 0) {
+#pragma unroll
+        for (int d = 0; d < DP; ++d)
+#pragma unroll
+            for (int k = 0; k < RW; ++k) ring[d][k] = Ap[k][min(lane + 64 * d, npair - 1)];
+    }
+    double xr[XR];
+#pragma unroll
+    for (int u = 0; u < XR; ++u) xr[u] = tid + TRD_SYMT * u < m ? xbuf[j + 1 + tid + TRD_SYMT * u] : 0.0;
     if (w == 0) {
+        const double alpha = st->alpha;
         double s = 0.0;
         for (int b = lane; b < nr; b += 64) s += rpart[b];
         s = wave_sum(s);
         if (lane == 0) {
-            const double alpha = st->alpha;
             double tau = 0.0, beta = alpha, scale = 0.0;
             if (s > 0.0) {
                 beta = -copysign(sqrt(alpha * alpha + s), alpha);
@@ -240,35 +283,22 @@ __global__ __launch_bounds__(TRD_SYMT) void trd_symv(const double* __restrict__ 
     }
     __syncthreads();
     const double scale = rs;
-    for (int e = tid; e < m; e += TRD_SYMT) vs[e] = e == 0 ? 1.0 : scale * xbuf[j + 1 + e];
+#pragma unroll
+    for (int u = 0; u < XR; ++u) {
+        const int e = tid + TRD_SYMT * u;
+        if (e < m) vs[e] = e == 0 ? 1.0 : scale * xr[u];
+    }
     __syncthreads();
-    const int peel = (j + 1) & 1, npair = (m - peel) >> 1, tail = (m - peel) & 1;
     double a1 = 0.0, a2 = 0.0, yv = 0.0;   // lane p < i: V_p . v, W_p . v; lane 0: y . v
-    const int nw = gridDim.x * NWV;
-    for (int r0 = RW * (blockIdx.x * NWV + w); r0 < m; r0 += RW * nw) {
-        const double2* Ap[RW];
+    if (live) {
         double y[RW];
 #pragma unroll
         for (int k = 0; k < RW; ++k) {
-            const int rr = min(r0 + k, m - 1);
-            const double* const Ar = A + (long)(j + 1 + rr) * lda + (j + 1);
-            Ap[k] = reinterpret_cast<const double2*>(Ar + peel);
             y[k] = 0.0;
             if (lane == 0) {
-                if (peel) y[k] = Ar[0] * vs[0];
-                if (tail) y[k] = fma(Ar[m - 1], vs[m - 1], y[k]);
+                if (peel) y[k] = e0[k] * vs[0];
+                if (tail) y[k] = fma(e1[k], vs[m - 1], y[k]);
             }
-        }
-        // steps s of the wave (t = lane + 64 s; lanes past npair read the
-        // last pair and weigh it by zero, so the loop is uniform), loaded DP
-        // steps ahead into a ring of registers (slot d holds step s0 + d)
-        const int ns = (npair + 63) >> 6;
-        double2 ring[DP][RW];
-        if (ns > 0) {
-#pragma unroll
-            for (int d = 0; d < DP; ++d)
-#pragma unroll
-                for (int k = 0; k < RW; ++k) ring[d][k] = Ap[k][min(lane + 64 * d, npair - 1)];
         }
         for (int s0 = 0; s0 < ns; s0 += DP) {
 #pragma unroll
@@ -298,8 +328,8 @@ __global__ __launch_bounds__(TRD_SYMT) void trd_symv(const double* __restrict__ 
             if (rr < m) {
                 const double vr = vs[rr];
                 if (lane < i) {
-                    a1 = fma(Vp[(long)lane * n + r], vr, a1);
-                    a2 = fma(Wp[(long)lane * n + r], vr, a2);
+                    a1 = fma(vp[k], vr, a1);
+                    a2 = fma(wp[k], vr, a2);
                 }
                 if (lane == 0) {
                     Wp[(long)i * n + r] = y[k];
@@ -324,36 +354,26 @@ __global__ __launch_bounds__(TRD_SYMT) void trd_symv(const double* __restrict__ 
     }
 }
 
-// The sums of a panel's last column (the next trd_row, which adds them itself
-// for the other columns, belongs to the next panel): c1, c2 and alpha2 into
-// the state for trd_wfinal.  tt: tau of the column.
-__global__ __launch_bounds__(256) void trd_symv_fin(int i, int nb, const double* __restrict__ part,
-                                                   TrdState* __restrict__ st, const double* __restrict__ tt)
+// W_q final (q = nb - 1, the panel's last column; the next trd_row, which does
+// this for the others, belongs to the next panel) on columns [c0, n), every
+// workgroup adding the column's sums itself.
+__global__ __launch_bounds__(256) void trd_wfinal(double* __restrict__ Wp, const double* __restrict__ Vp, int n, int q,
+                                                  int c0, const double* __restrict__ tt, int nb,
+                                                  const double* __restrict__ part)
 {
-    __shared__ double tot[2 * TRD_NB + 1];
+    __shared__ double tot[2 * TRD_NB + 1], sa2;
     const int tid = threadIdx.x;
-    trd_sum_parts(i, nb, part, tid, tot);
+    const double tau = tt[0];
+    trd_sum_parts(q, nb, part, tid, tot);
     __syncthreads();
-    if (tid < i) {
-        st->c1[tid] = tot[1 + tid];
-        st->c2[tid] = tot[1 + i + tid];
-    }
-    if (tid == 0) st->alpha2[i] = trd_alpha2(i, tt[0], tot);
-}
-
-// W_q final (q = nb - 1, the panel's last column) on columns [c0, n).
-__global__ void trd_wfinal(double* __restrict__ Wp, const double* __restrict__ Vp, int n, int q, int c0,
-                           const double* __restrict__ tt, const TrdState* __restrict__ st)
-{
-    __shared__ double c1[TRD_NB], c2[TRD_NB];
-    if (threadIdx.x < q) {
-        c1[threadIdx.x] = st->c1[threadIdx.x];
-        c2[threadIdx.x] = st->c2[threadIdx.x];
+    if (tid < 64) {
+        const double a2 = trd_alpha2(q, tau, tot, tid);
+        if (tid == 0) sa2 = a2;
     }
     __syncthreads();
-    const long c = c0 + (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const long c = c0 + (long)blockIdx.x * blockDim.x + tid;
     if (c >= n) return;
-    Wp[(long)q * n + c] = trd_wfin(Vp, Wp, n, q, c, tt[0], c1, c2, st->alpha2[q]);
+    Wp[(long)q * n + c] = trd_wfin(Vp, Wp, n, q, c, tau, tot + 1, tot + 1 + q, sa2);
 }
 
 // A[k1.., k1..] -= V W^T + W V^T (nb panel rows), 64 x 64 lower tiles I >= J
@@ -433,18 +453,45 @@ __global__ void trd_lastd(const double* __restrict__ A, int lda, int n, double* 
 __global__ __launch_bounds__(1024) void trd_tmat(const double* __restrict__ V, const double* __restrict__ tt, int n,
                                                  double* __restrict__ Vt)
 {
-    __shared__ double Gs[TRD_NB][TRD_NB + 1], Ts[TRD_NB][TRD_NB + 1];
+    __shared__ double Gs[TRD_NB][TRD_NB + 1], Ts[TRD_NB][TRD_NB + 1], R[8][TRD_NB][TRD_NB + 1];
     const int k0 = blockIdx.x * TRD_NB, nb = min(TRD_NB, n - 1 - k0), c0 = k0 + 1;
-    const int tid = threadIdx.x, a = tid / TRD_NB, b = tid % TRD_NB;
-    if (a < nb && b < nb && b >= a) {
-        double s = 0.0;
-        const double* const va = V + (long)(k0 + a) * n;
-        const double* const vb = V + (long)(k0 + b) * n;
-        for (int c = k0 + b + 1; c < n; ++c) s = fma(va[c], vb[c], s);
-        Gs[a][b] = s;
+    const int tid = threadIdx.x, a = tid / TRD_NB, b = tid % TRD_NB, lane = tid & 63, w = tid >> 6;
+    // G on FP64 MFMA, the 16 waves splitting the columns; their sums are added
+    // in wave order
+    fd4 acc[2][2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int y = 0; y < 2; ++y) acc[x][y] = (fd4){0.0, 0.0, 0.0, 0.0};
+    for (int k = c0 + 4 * w; k < n; k += 64) {
+        const int c = k + (lane >> 4);
+        double v[2];
+#pragma unroll
+        for (int x = 0; x < 2; ++x) {
+            const int p = 16 * x + (lane & 15);
+            v[x] = (c < n && p < nb) ? V[(long)(k0 + p) * n + c] : 0.0;
+        }
+#pragma unroll
+        for (int x = 0; x < 2; ++x)
+#pragma unroll
+            for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(v[x], v[y], acc[x][y], 0, 0, 0);
     }
-    __syncthreads();
-    if (tid < TRD_NB * TRD_NB) Ts[a][b] = 0.0;
+    for (int h = 0; h < 2; ++h) {
+        if ((w >> 3) == h)
+#pragma unroll
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v)
+                        R[w & 7][16 * x + 4 * v + (lane >> 4)][16 * y + (lane & 15)] = acc[x][y][v];
+        __syncthreads();
+        double s = h ? Gs[a][b] : 0.0;
+        for (int k = 0; k < 8; ++k) s += R[k][a][b];
+        Gs[a][b] = s;
+        __syncthreads();
+    }
+    Ts[a][b] = 0.0;
     __syncthreads();
     if (tid < nb) {
         const int q = tid;
@@ -456,65 +503,87 @@ __global__ __launch_bounds__(1024) void trd_tmat(const double* __restrict__ V, c
         }
     }
     __syncthreads();
-    for (int c = c0 + tid; c < n; c += 1024) {
-        double s[TRD_NB];
+    // Vt = T^T V: a wave takes 16 columns at a time, K = the panel's reflectors
+    for (int cb = c0 + 16 * w; cb < n; cb += 256) {
+        const int c = cb + (lane & 15);
+        fd4 o[2] = {(fd4){0.0, 0.0, 0.0, 0.0}, (fd4){0.0, 0.0, 0.0, 0.0}};
 #pragma unroll
-        for (int p = 0; p < TRD_NB; ++p) s[p] = 0.0;
+        for (int ks = 0; ks < TRD_NB / 4; ++ks) {
+            const int q = 4 * ks + (lane >> 4);
+            const double v = (c < n && q < nb) ? V[(long)(k0 + q) * n + c] : 0.0;
 #pragma unroll
-        for (int q = 0; q < TRD_NB; ++q) {
-            const double vq = q < nb ? V[(long)(k0 + q) * n + c] : 0.0;
-#pragma unroll
-            for (int p = q; p < TRD_NB; ++p) s[p] = fma(Ts[q][p], vq, s[p]);
+            for (int x = 0; x < 2; ++x)
+                o[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(Ts[q][16 * x + (lane & 15)], v, o[x], 0, 0, 0);
         }
+        if (c < n)
 #pragma unroll
-        for (int p = 0; p < TRD_NB; ++p)
-            if (p < nb) Vt[(long)(k0 + p) * n + c] = s[p];
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int p = 16 * x + 4 * v + (lane >> 4);
+                    if (p < nb) Vt[(long)(k0 + p) * n + c] = o[x][v];
+                }
     }
 }
 
 // M[r][p] = sum_{c >= c0} E[r][c] V_p[c] for 32 rows per workgroup and the
-// panel's nb <= 32 reflectors (FP64 MFMA; the four waves split the columns c
-// and add their 32 x 32 results in LDS in wave order).
-__global__ __launch_bounds__(256) void trd_bt_proj(const double* __restrict__ E, int n, const double* __restrict__ Vp,
-                                                   int nb, int c0, double* __restrict__ M)
+// panel's nb <= 32 reflectors (FP64 MFMA; the 16 waves take 16 columns in turn
+// and their 32 x 32 results are added in LDS in wave order).  In a wave's 16
+// columns lane group q holds columns 4 q .. 4 q + 3, one per K-step, so a lane
+// reads 32 contiguous bytes of its row.  With n / 32 workgroups the chip is not
+// full, and 16 waves instead of 4 on each took it from 59 to 32 us at n = 2300.
+__global__ __launch_bounds__(1024) void trd_bt_proj(const double* __restrict__ E, int n, const double* __restrict__ Vp,
+                                                    int nb, int c0, double* __restrict__ M)
 {
-    __shared__ double R[4][32][33];
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, l16 = lane & 15, kq = lane >> 4;
+    __shared__ double R[8][32][33];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, l16 = lane & 15, kq = lane >> 4;
     const int r0 = blockIdx.x * 32;
-    const int m = n - c0, seg = ((m + 3) / 4 + 3) / 4 * 4;   // columns per wave: a quarter, a multiple of 4
-    const int ca = c0 + w * seg, cz = min(n, ca + seg);
     fd4 acc[2][2];
 #pragma unroll
     for (int x = 0; x < 2; ++x)
 #pragma unroll
         for (int y = 0; y < 2; ++y) acc[x][y] = (fd4){0.0, 0.0, 0.0, 0.0};
-    for (int k = ca; k < cz; k += 4) {
-        const int c = k + kq;
-        const bool cin = c < cz;
-        double a[2], b[2];
+    const double* er[2];
+    const double* vr[2];
 #pragma unroll
-        for (int x = 0; x < 2; ++x) {
-            const int r = r0 + 16 * x + l16, p = 16 * x + l16;
-            a[x] = (cin && r < n) ? E[(long)r * n + c] : 0.0;
-            b[x] = (cin && p < nb) ? Vp[(long)p * n + c] : 0.0;
+    for (int x = 0; x < 2; ++x) {
+        er[x] = E + (long)min(r0 + 16 * x + l16, n - 1) * n;        // (rows past n are not stored)
+        vr[x] = Vp + (long)min(16 * x + l16, nb - 1) * n;           // (nor columns past nb)
+    }
+    for (int k = c0 + 16 * w; k < n; k += 256) {
+        double a[2][4], b[2][4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int c = k + 4 * kq + u, cc = min(c, n - 1);
+#pragma unroll
+            for (int x = 0; x < 2; ++x) {
+                a[x][u] = er[x][cc];
+                b[x][u] = c < n ? vr[x][cc] : 0.0;
+            }
         }
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-            for (int y = 0; y < 2; ++y) acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x], b[y], acc[x][y], 0, 0, 0);
+            for (int x = 0; x < 2; ++x)
+#pragma unroll
+                for (int y = 0; y < 2; ++y)
+                    acc[x][y] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[x][u], b[y][u], acc[x][y], 0, 0, 0);
     }
+    double m = 0.0;
+    const int rr = tid >> 5, p = tid & 31;
+    for (int h = 0; h < 2; ++h) {
+        if ((w >> 3) == h)
 #pragma unroll
-    for (int x = 0; x < 2; ++x)
+            for (int x = 0; x < 2; ++x)
 #pragma unroll
-        for (int y = 0; y < 2; ++y)
+                for (int y = 0; y < 2; ++y)
 #pragma unroll
-            for (int v = 0; v < 4; ++v) R[w][16 * x + 4 * v + kq][16 * y + l16] = acc[x][y][v];
-    __syncthreads();
-    for (int e = threadIdx.x; e < 32 * 32; e += 256) {
-        const int rr = e >> 5, p = e & 31;
-        const int r = r0 + rr;
-        if (r < n && p < nb) M[(long)r * TRD_NB + p] = ((R[0][rr][p] + R[1][rr][p]) + R[2][rr][p]) + R[3][rr][p];
+                    for (int v = 0; v < 4; ++v) R[w & 7][16 * x + 4 * v + kq][16 * y + l16] = acc[x][y][v];
+        __syncthreads();
+        for (int k = 0; k < 8; ++k) m += R[k][rr][p];
+        __syncthreads();
     }
+    if (r0 + rr < n && p < nb) M[(long)(r0 + rr) * TRD_NB + p] = m;
 }
 
 // E[r][c] -= sum_p M[r][p] Vt_p[c] for c >= c0 (64 x 64 tiles, FP64 MFMA, K = nb).
@@ -646,26 +715,26 @@ static int trd_reduce(TrdWork& W, int n, int lda, hipStream_t st_)
             hipLaunchKernelGGL(trd_row, dim3(g1), dim3(TRD_ROWT), 0, st_, (const double*)Ad, lda, n, j, i, Vp,
                                Wp.as<double>(), (const double*)tt.as<double>(), xb.as<double>(), dd.as<double>(), sd,
                                (const double*)part.as<double>(), prev_g2, rpart.as<double>());
-            const unsigned g2 = (unsigned)std::min(TRD_SYMG, (m + 4 * (TRD_SYMT / 64) - 1) / (4 * (TRD_SYMT / 64)));
-            hipLaunchKernelGGL(trd_symv, dim3(g2), dim3(TRD_SYMT), sizeof(double) * (size_t)m, st_,
-                               (const double*)Ad, lda, n, j, i, (const double*)xb.as<double>(), Vp, Wp.as<double>(),
-                               V.as<double>() + (size_t)j * n, (const double*)rpart.as<double>(), (int)g1,
-                               ee.as<double>(), tt.as<double>(), sd, part.as<double>());
+            const int rw = m <= TRD_RW2 ? 2 : 4, rows = rw * (TRD_SYMT / 64);
+            const unsigned g2 = (unsigned)((m + rows - 1) / rows);
+#define TRD_SYMV(RW)                                                                                              \
+    hipLaunchKernelGGL(trd_symv<RW>, dim3(g2), dim3(TRD_SYMT), sizeof(double) * (size_t)m, st_, (const double*)Ad, lda, \
+                       n, j, i, (const double*)xb.as<double>(), Vp, Wp.as<double>(), V.as<double>() + (size_t)j * n, \
+                       (const double*)rpart.as<double>(), (int)g1, ee.as<double>(), tt.as<double>(), sd,          \
+                       part.as<double>())
+            if (rw == 2) TRD_SYMV(2);
+            else TRD_SYMV(4);
+#undef TRD_SYMV
             prev_g2 = (int)g2;
-            if (i == nb - 1)
-                hipLaunchKernelGGL(trd_symv_fin, dim3(1), dim3(256), 0, st_, i, (int)g2,
-                                   (const double*)part.as<double>(), sd, (const double*)(tt.as<double>() + j));
         }
         if (k1 < n) {
             hipLaunchKernelGGL(trd_wfinal, dim3((unsigned)((n - k1 + 255) / 256)), dim3(256), 0, st_,
-                               Wp.as<double>(), Vp, n, nb - 1, k1, (const double*)(tt.as<double>() + k1 - 1),
-                               (const TrdState*)sd);
+                               Wp.as<double>(), Vp, n, nb - 1, k1, (const double*)(tt.as<double>() + k1 - 1), prev_g2,
+                               (const double*)part.as<double>());
             const int T = (n - k1 + 63) / 64;
             hipLaunchKernelGGL(trd_syr2k, dim3((unsigned)(T * (T + 1) / 2)), dim3(256), 0, st_, Ad, lda, n, k1, Vp,
                                (const double*)Wp.as<double>(), nb);
         }
-        // alpha2 of the next panel starts from zero
-        MCMB_HIP(hipMemsetAsync(sd->alpha2, 0, sizeof(double) * TRD_NB, st_));
     }
     hipLaunchKernelGGL(trd_lastd, dim3(1), dim3(64), 0, st_, (const double*)Ad, lda, n, dd.as<double>());
     MCMB_HIP(hipGetLastError());
@@ -746,7 +815,7 @@ int tridiag_eigen(mcmb_ctx* c, int n, const double* d_G, int normalise, double* 
                            (const double*)tt.as<double>(), n, Vt.as<double>());
         for (int b = npan - 1; b >= 0; --b) {
             const int k0 = b * TRD_NB, nb = std::min(TRD_NB, n - 1 - k0), c0 = k0 + 1;
-            hipLaunchKernelGGL(trd_bt_proj, dim3((unsigned)((n + 31) / 32)), dim3(256), 0, c->stream,
+            hipLaunchKernelGGL(trd_bt_proj, dim3((unsigned)((n + 31) / 32)), dim3(1024), 0, c->stream,
                                (const double*)E.as<double>(), n, (const double*)(V.as<double>() + (size_t)k0 * n), nb,
                                c0, M.as<double>());
             const unsigned tiles = (unsigned)(((n + 63) / 64) * ((n - c0 + 63) / 64));
