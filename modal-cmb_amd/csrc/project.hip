@@ -10,17 +10,19 @@
 //
 // With A_ij = omega (k_i + k_j) + phi and B_k = omega k_k,
 //   sin(A + B) = sin A cos B + cos A sin B,
-// the k-sum separates:  Y[(i,j)][c,t] = sum_k W_ijk Z[k][c,t] with the four
-// column sets Z = {cos B, sin B, k cos B, k sin B} q_t(k)  -- one MFMA GEMM
-// (W resident in HBM, N^2 x N) for a batch of shapes.  Then per shape
-//   G0 = sA Yc + cA Ys                         (value,  sin(A+B))
-//   G2 = cA Yc - sA Ys                         (d/dphi, cos(A+B))
-//   G1 = (k_i + k_j) G2 + cA Yc' - sA Ys'      (d/domega, K cos(A+B))
-//   H_x[i][s][t] = sum_j q_s(j) G_x[i][j][t],  alpha_x[n] = sum_i q_r(i) H_x[i][s][t].
-// The adjoint (VJP) takes gbar = dL/dalpha, forms Hbar[i][s][t] =
-// sum_r q_r(i) Abar[r][s][t] (Abar = gbar scattered onto the canonical
-// triples), Gbar[i][j][t] = sum_s q_s(j) Hbar[i][s][t], and reduces
-// dL/dphi = sum Gbar G2, dL/domega = sum Gbar G1.
+// the k-sum separates:  Y[(i,j)][x,t] = sum_k W_ijk Z[k][x,t] with the two
+// column sets Z = {cos B, sin B} q_t(k)  -- one MFMA GEMM (W resident in HBM,
+// N^2 / 2 x N) for a batch of shapes.  Then per shape
+//   G_sin = sA Yc + cA Ys   (sin(A+B): the value)
+//   G_cos = cA Yc - sA Ys   (cos(A+B): the derivatives)
+//   H_x[i][s][t] = sum_j q_s(j) G_x[i][j][t],  A_x[r][s][t] = sum_i q_r(i) H_x[i][s][t],
+// and d/domega, which brings K = k_i + k_j + k_k, from the k_i-weighted sum
+// over i with each leg in turn on i.
+// H_x[i] is symmetric in (s, t) (W and the shape are symmetric in the legs j
+// and k), so it is formed and kept for s <= t only.
+// The adjoint (VJP) of gbar = dL/dalpha contracts it with the two derivative
+// tensors of the same k-, j- and i-sums: dL/dphi = sum_n gbar_n dalpha_n/dphi,
+// dL/domega = sum_n gbar_n dalpha_n/domega.
 #include "mcmb_internal.h"
 #include <type_traits>
 #include <cstring>
@@ -34,19 +36,13 @@ typedef double d4 __attribute__((ext_vector_type(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
 
 constexpr int PT = 128;     // GEMM tile (M and N)
+constexpr int WT = 64;      // the same of stage 1's GEMM
 constexpr int PK = 16;      // GEMM K chunk
 constexpr int PBATCH = 32;  // shapes per batch
 
 // ---- full-cube weight ------------------------------------------------------
 // W[(i*N + j)*Kp + k]; the mask compares the sorted triple exactly as the
 // oracle does: k_c <= k_a + k_b (FP64).
-// Row of the pair (i, j) in the packed i <= j order of the stage-1 product.
-__device__ __forceinline__ long pair_row(int i, int j, int N)
-{
-    const int lo = min(i, j), hi = max(i, j);
-    return (long)lo * N - (long)lo * (lo - 1) / 2 + (hi - lo);
-}
-
 template <class T>
 __global__ void proj_build_W(const double* __restrict__ kn, const double* __restrict__ kw, int N, int Kp,
                              const int2* __restrict__ rowij, long M, T* __restrict__ W)
@@ -67,7 +63,7 @@ __global__ void proj_build_W(const double* __restrict__ kn, const double* __rest
     W[e] = (T)w;
 }
 
-// The K chunks of each PT-row tile of W that hold a nonzero weight: tiles[t]
+// The K chunks of each WT-row tile of W that hold a nonzero weight: tiles[t]
 // = (first chunk, chunk count) over the tile's rows (an all-zero tile keeps
 // chunk 0).  The stage-1 GEMMs run only over those chunks: the others add
 // exact zeros.
@@ -81,7 +77,7 @@ __global__ __launch_bounds__(256) void proj_w_tiles(const T* __restrict__ W, lon
         hi = -1;
     }
     __syncthreads();
-    const long r0 = (long)blockIdx.x * PT, ne = (long)min((long)PT, M - r0) * Kp;
+    const long r0 = (long)blockIdx.x * WT, ne = (long)min((long)WT, M - r0) * Kp;
     int mlo = Kp, mhi = -1;
     for (long e = threadIdx.x; e < ne; e += 256)
         if (W[r0 * Kp + e] != (T)0) {
@@ -98,8 +94,22 @@ __global__ __launch_bounds__(256) void proj_w_tiles(const T* __restrict__ W, lon
     }
 }
 
-// Z[k][col], col = (b*2 + c)*R + t for shapes b < nb of the batch: c = 0
-// cos(omega_b k) q_t(k), c = 1 sin(omega_b k) q_t(k); Kp x ldz.
+// The R basis columns as stage 2 takes them: NT = 1 or 2 matrix tiles (R > 16)
+// of Rh columns, t = a Rh + c (a < NT, c < Rh <= 16).  A shape has the 2 NT Rh
+// columns (c, a, cos / sin) of Z and Y, so that what lane c of stage 2 needs of
+// a Y row is one vector of 2 NT elements.
+struct BasisTiles {
+    int NT, Rh, cols;   // tiles, columns of each, Z columns of a shape
+};
+__host__ __device__ __forceinline__ BasisTiles basis_tiles(int R)
+{
+    const int NT = R > 16 ? 2 : 1, Rh = (R + NT - 1) / NT;
+    return BasisTiles{NT, Rh, 2 * NT * Rh};
+}
+
+// Z[k][col], col = ((b Rh + c) NT + a) 2 + x for shapes b < nb of the batch:
+// x = 0 cos(omega_b k) q_t(k), x = 1 sin(omega_b k) q_t(k), t = a Rh + c (zero
+// past R); Kp x ldz.
 template <class T>
 __global__ void proj_build_Z(const double* __restrict__ kn, const double* __restrict__ q, int ldq, int N, int R,
                              const double* __restrict__ theta, int nb, int Kp, int ldz, T* __restrict__ Z)
@@ -108,8 +118,10 @@ __global__ void proj_build_Z(const double* __restrict__ kn, const double* __rest
     if (e >= (size_t)Kp * ldz) return;
     int k = (int)(e / ldz), col = (int)(e % ldz);
     double z = 0.0;
-    if (k < N && col < nb * 2 * R) {
-        int t = col % R, c = (col / R) % 2, b = col / (2 * R);
+    const BasisTiles bt = basis_tiles(R);
+    const int a = (col >> 1) % bt.NT, e1 = (col >> 1) / bt.NT, t = a * bt.Rh + e1 % bt.Rh, b = e1 / bt.Rh;
+    if (k < N && b < nb && t < R) {
+        const int c = col & 1;
         double om = theta[2 * b];
         double sb, cb;
         sincos(om * kn[k], &sb, &cb);
@@ -208,364 +220,346 @@ __global__ __launch_bounds__(256, 2) void proj_gemm(const T* __restrict__ A, con
             }
 }
 
-// sin and cos of omega_b k_j for the shapes of a batch: scb[b][j] = (sin, cos).
-// Stage 2 and the adjoint form sin / cos of A_ij = (omega k_i + phi) +
-// omega k_j by the angle-addition formulas from these and one sincos per
-// workgroup.
-__global__ void proj_sincos_tab(const double* __restrict__ kn, const double* __restrict__ theta, int N, int nb,
+// sin and cos of omega_b k_j for the shapes of a batch: scb[b][j] = (sin,
+// cos), zero for N <= j < Np.  Stage 2 forms sin / cos of A_ij = (omega k_i +
+// phi) + omega k_j by the angle-addition formulas from these and one sincos
+// per workgroup.
+__global__ void proj_sincos_tab(const double* __restrict__ kn, const double* __restrict__ theta, int N, int Np, int nb,
                                 double* __restrict__ scb)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nb * N) return;
-    const int b = e / N, j = e % N;
-    double sb, cb;
-    sincos(theta[2 * b] * kn[j], &sb, &cb);
+    if (e >= nb * Np) return;
+    const int b = e / Np, j = e % Np;
+    double sb = 0.0, cb = 0.0;
+    if (j < N) sincos(theta[2 * b] * kn[j], &sb, &cb);
     scb[2 * e] = sb;
     scb[2 * e + 1] = cb;
 }
 
-// ---- forward stage 2: per (shape b, i) -------------------------------------
-// H[b][x][i][s][t] = sum_j q_s(j) G_x(i, j, t) with G_x(i, j, t) = sum_k
-// W_ijk {sin, cos}(omega K + phi) q_t(k), x = 0 (sin: the value) and x = 1
-// (cos: the derivatives).  From stage 1's Yc, Ys (cos / sin omega k_k
-// columns) by angle addition: G_0 = sin A Yc + cos A Ys, G_1 = cos A Yc -
-// sin A Ys, A = omega (k_i + k_j) + phi.  Y's row of the pair (i, j) is
-// rowof[pair_row(i, j)] (stage 1 runs over W's rows in their own order).
-template <class T>
-__global__ __launch_bounds__(256) void proj_stage2(const T* __restrict__ Y, int ldy, const int* __restrict__ rowof,
-                                                   const double* __restrict__ kn,
-                                                   const double* __restrict__ q, int ldq, int N, int R,
-                                                   const double* __restrict__ theta, int nb,
-                                                   const double* __restrict__ scb, double* __restrict__ H)
+// Column of (s, t) among the pairs s <= t of R functions; the symmetric
+// planes below keep PP = the count rounded up to whole 16-column blocks.
+__host__ __device__ __forceinline__ int sym_col(int s, int t, int R)
 {
-    // one workgroup per (shape b, node i); H_x[s][t] = sum_j q_s(j) G_x[j][t]
-    // over chunks of 32 nodes j, on FP64 MFMA 16x16x4: A = Q^T (s x j), B =
-    // G_x (j x t).  Wave w owns the s tile w / 2 and the t tile w % 2 of both
-    // x (2 accumulators, the A operand shared).  The thread's 4 elements (j =
-    // j0 + tid / 32 + 8 u, t = tid % 32) of the next chunk are loaded (Y, q,
-    // sin / cos omega k_j) while the current chunk's products run.
-    __shared__ double G[2][32][32];     // [x][j in chunk][t]
-    __shared__ double Qs[32][32];       // [j in chunk][s]
-    const int b = blockIdx.x % nb, i = blockIdx.x / nb;
-    const int tid = threadIdx.x, t = tid & 31, jr = tid >> 5;
-    const int lane = tid & 63, w = tid >> 6, sm = 16 * (w >> 1), tn = 16 * (w & 1);
-    const double ki = kn[i];
-    double sa, ca;   // sin, cos of omega k_i + phi
-    sincos(theta[2 * b] * ki + theta[2 * b + 1], &sa, &ca);
-    const double* const sc = scb + 2 * (size_t)b * N;
-    d4 acc[2];
+    const int lo = s < t ? s : t, hi = s < t ? t : s;
+    return lo * (2 * R - lo - 1) / 2 + hi;
+}
+static int sym_cols(int R) { return (R * (R + 1) / 2 + 15) / 16 * 16; }
+
+// ---- stage 2: per (shape b, node i) ----------------------------------------
+// H[b][x][i][st] = sum_j q_s(j) G_x(i, j, t), s <= t, with G_x(i, j, t) =
+// sum_k W_ijk {sin, cos}(omega K + phi) q_t(k): sin for the value, cos for the
+// derivatives.  X selects the planes: 1 sin, 2 cos, 3 both (in that order).
+// From stage 1's Yc, Ys (cos / sin omega k_k columns) by angle addition:
+// G_sin = sin A Yc + cos A Ys, G_cos = cos A Yc - sin A Ys, A = omega (k_i +
+// k_j) + phi.  Y's row of the pair (i, j) is wrow[stage2_row(i, j)] (stage 1
+// runs over W's rows in their own order).
+//
+// On FP64 MFMA 16x16x4, A = Q^T (s x j), B = G_x (j x t); of the tiles of (s,
+// t) only those on and above the diagonal (NP = 3 of 4 for NT = 2).  The four
+// waves of a workgroup take every fourth K-step (4 nodes j) each and are
+// summed through LDS at the end: a lane forms the B operand of its own (j, t)
+// from its own loads, so the loop has no LDS traffic and no barrier, and the
+// loads of the next group of K-steps run under this one's products.
+//
+// What bounds it besides the products is the address unit of the CU's vector
+// loads, about 16 cycles an instruction whatever its width: with one load
+// per element of Y and q and one for the row number (7 a K-step) that unit was
+// 78% busy.  So a lane's Y, q and (sin, cos) of a K-step are one vector each
+// (the layouts of Z and of the basis table), a lane's row numbers
+// of a group lie next to each other, and the tables are padded with zeros to Np nodes so that nothing is
+// clamped or masked.
+//
+// XCD x (workgroups are dealt to the 8 XCDs in turn) takes the nodes i = x
+// mod 8, and the shapes go in groups of SG, node by node: neighbouring shapes'
+// pieces of a Y row, which share cache lines, meet in one L2, and a group's
+// part of Y is read the second time (for the pair's other node) out of cache.
+//
+// 32 shapes, 300 nodes, 30 functions, FP32 Y (347 MB; the products alone are
+// 120 us, or 60 for one plane): both planes 373 -> 200 us, cos alone (with the
+// sums that replaced the adjoint's own) 284 -> 137.  One shape of 200 nodes,
+// FP64: 14 -> 7.4.
+constexpr int SG = 4;    // shapes of a group
+// Nodes of a workgroup: two share the basis and the (sin, cos) loads and halve
+// the workgroups.  With one plane to form the address unit is the bound and
+// two are faster from S2_PAIR (shape, node) pairs on: 3200 pairs (FP64) 36.2
+// us with one, 36.8 with two; 6400 65.3, 64.6; 9600 (FP32) 157, 137.  With both
+// planes the products are (9600: 195, 199), so there it stays one.
+constexpr long S2_PAIR = 4800;
+constexpr int S2U = 2;   // K-steps a wave loads ahead
+// nodes of the padded tables: two groups of S2U K-steps past the last
+__host__ __device__ __forceinline__ int stage2_nodes(int N) { return (N + 16 * S2U - 1) / (16 * S2U) * (16 * S2U) + 32 * S2U; }
+// place of the pair (i, j) in the row table: a lane's nodes j = 16 m + r (r its own) in order of m
+static size_t stage2_row(int i, int j, int Np) { return (size_t)i * Np + (size_t)(j % 16) * (Np / 16) + j / 16; }
+
+template <class T, int X, int NT, int NI>
+__global__ __launch_bounds__(256, NI * NT == 4 ? 3 : 4) void proj_stage2(const T* __restrict__ Y, int ldy, const int* __restrict__ wrow,
+                                                      const double* __restrict__ kn, const double* __restrict__ qt,
+                                                      int N, int R, int PP, const double* __restrict__ theta, int nb,
+                                                      const double* __restrict__ scb, double* __restrict__ H)
+{
+    typedef T TV __attribute__((ext_vector_type(2 * NT)));
+    typedef double D2 __attribute__((ext_vector_type(2)));
+    typedef int I2 __attribute__((ext_vector_type(2)));
+    static_assert(S2U == 2, "a group's row numbers are one int2");
+    constexpr int NX = (X & 1) + (X >> 1), NP = NT * (NT + 1) / 2, U = S2U;
+    __shared__ double red[4][NP][256];
+    const int ni = (N + NI - 1) / NI, slot = blockIdx.x >> 3;
+    const int per = SG * ((ni + 7) / 8);   // workgroups of a whole shape group on an XCD
+    const int g0 = slot / per * SG, ns = min(SG, nb - g0), e0 = slot % per;
+    const int b = g0 + e0 % ns, i0 = NI * (8 * (e0 / ns) + (blockIdx.x & 7));   // nodes i0 .. i0 + NI - 1
+    if (i0 >= N) return;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 15,
+              kg = lane >> 4;
+    const int Np = stage2_nodes(N), Rh = (R + NT - 1) / NT;
+    double sa[NI], ca[NI];   // sin, cos of omega k_i + phi
 #pragma unroll
-    for (int x = 0; x < 2; ++x) acc[x] = (d4){0.0, 0.0, 0.0, 0.0};
-    T yv[4][2];
-    double qv[4], sv[4], cv[4];
-    // loads of chunk j0 (nodes past N repeat the last one and are zeroed in stage())
-    auto fetch = [&](int j0) {
+    for (int z = 0; z < NI; ++z)
+        sincos(theta[2 * b] * kn[min(i0 + z, N - 1)] + theta[2 * b + 1], &sa[z], &ca[z]);
+    // the wave's K-step m has the nodes j = 16 m + 4 w + kg
+    const I2* rw[NI];   // a node past N: the last one again, not stored
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int j = min(j0 + jr + 8 * u, N - 1), tt = min(t, R - 1);
-            const T* y = Y + (size_t)rowof[pair_row(i, j, N)] * ldy + (size_t)b * 2 * R + tt;
-            yv[u][0] = y[0];
-            yv[u][1] = y[R];
-            qv[u] = q[(size_t)j * ldq + tt];
-            sv[u] = sc[2 * j];
-            cv[u] = sc[2 * j + 1];
+    for (int z = 0; z < NI; ++z)
+        rw[z] = reinterpret_cast<const I2*>(wrow + (size_t)min(i0 + z, N - 1) * Np + (4 * w + kg) * (Np / 16));
+    const D2* const sc = reinterpret_cast<const D2*>(scb) + (size_t)b * Np + 4 * w + kg;
+    const double* const qj = qt + ((4 * w + kg) * 16 + c) * NT;
+    const T* const Yb = Y + (size_t)b * 2 * NT * Rh + 2 * NT * min(c, Rh - 1);   // lanes past Rh: not stored
+    d4 acc[NI][NX][NP];
+#pragma unroll
+    for (int z = 0; z < NI; ++z)
+#pragma unroll
+        for (int x = 0; x < NX; ++x)
+#pragma unroll
+            for (int p = 0; p < NP; ++p) acc[z][x][p] = (d4){0.0, 0.0, 0.0, 0.0};
+    const int ng = (N + 16 * U - 1) / (16 * U);   // groups of U K-steps a wave
+    I2 rows[NI];
+    TV yv[NI][U];
+    D2 sv[U];
+    double qv[U][NT];
+    auto load_rows = [&](int g) {
+#pragma unroll
+        for (int z = 0; z < NI; ++z) rows[z] = rw[z][g];
+    };
+    auto load = [&](int g) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int m = g * U + u;
+#pragma unroll
+            for (int z = 0; z < NI; ++z)
+                yv[z][u] = *reinterpret_cast<const TV*>(Yb + (size_t)(unsigned)rows[z][u] * (unsigned)ldy);
+            sv[u] = sc[16 * m];
+            if (NT == 2) {
+                const D2 v = *reinterpret_cast<const D2*>(qj + (size_t)m * 256 * NT);
+                qv[u][0] = v[0];
+                qv[u][NT - 1] = v[1];
+            } else
+                qv[u][0] = qj[(size_t)m * 256 * NT];
         }
     };
-    auto stage = [&](int j0) {
+    load_rows(0);
+    load(0);
+    load_rows(1);
+    for (int g = 0; g < ng; ++g) {
+        double A[U][NT], B[NI][U][NX][NT];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int jj = jr + 8 * u;
-            const bool in = j0 + jj < N && t < R;
-            const double sA = sa * cv[u] + ca * sv[u], cA = ca * cv[u] - sa * sv[u];
-            const double yc = (double)yv[u][0], ys = (double)yv[u][1];
-            const double g0 = sA * yc + cA * ys;
-            const double g1 = cA * yc - sA * ys;
-            G[0][jj][t] = in ? g0 : 0.0;
-            G[1][jj][t] = in ? g1 : 0.0;
-            Qs[jj][t] = in ? qv[u] : 0.0;
-        }
-    };
-    fetch(0);
-    for (int j0 = 0; j0 < N; j0 += 32) {
-        __syncthreads();   // the previous chunk's products are done with G and Qs
-        stage(j0);
-        __syncthreads();
-        fetch(min(j0 + 32, N - 1));
-        // 8 K-steps of 4 nodes (those past N have G = Q = 0)
+        for (int u = 0; u < U; ++u) {
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const int jj = 4 * ks + (lane >> 4);
-            const double a = Qs[jj][sm + (lane & 15)];
+            for (int a = 0; a < NT; ++a) A[u][a] = qv[u][a];
 #pragma unroll
-            for (int x = 0; x < 2; ++x)
-                acc[x] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, G[x][jj][tn + (lane & 15)], acc[x], 0, 0, 0);
-        }
-    }
-    // element v of a lane: s = sm + 4 v + lane / 16, t = tn + lane % 16
-    const int tt = tn + (lane & 15);
-    if (tt < R)
+            for (int z = 0; z < NI; ++z) {
+                const double sA = sa[z] * sv[u][1] + ca[z] * sv[u][0], cA = ca[z] * sv[u][1] - sa[z] * sv[u][0];
 #pragma unroll
-        for (int x = 0; x < 2; ++x)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int ss = sm + 4 * v + (lane >> 4);
-                if (ss < R) H[(((size_t)b * 2 + x) * N + i) * R * R + ss * R + tt] = acc[x][v];
+                for (int a = 0; a < NT; ++a) {
+                    const double yc = (double)yv[z][u][2 * a], ys = (double)yv[z][u][2 * a + 1];
+                    if (X & 1) B[z][u][0][a] = sA * yc + cA * ys;
+                    if (X & 2) B[z][u][NX - 1][a] = cA * yc - sA * ys;
+                }
             }
+        }
+        load(g + 1);
+        load_rows(g + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int z = 0; z < NI; ++z)
+#pragma unroll
+                for (int x = 0; x < NX; ++x) {
+                    int p = 0;
+#pragma unroll
+                    for (int a = 0; a < NT; ++a)
+#pragma unroll
+                        for (int t = a; t < NT; ++t, ++p)
+                            acc[z][x][p] =
+                                __builtin_amdgcn_mfma_f64_16x16x4f64(A[u][a], B[z][u][x][t], acc[z][x][p], 0, 0, 0);
+                }
+    }
+    // sum over the waves, a plane at a time; element v of a lane is row 4 v +
+    // lane / 16, column lane % 16 of its tile, and thread tid stores element
+    // (tid / 16, tid % 16).  A tile on the diagonal holds (s, t) and (t, s): of
+    // these the mean, whose stage-1 roundings are independent.
+#pragma unroll
+    for (int z = 0; z < NI; ++z)
+#pragma unroll
+        for (int x = 0; x < NX; ++x) {
+            if (x || z) __syncthreads();
+#pragma unroll
+            for (int p = 0; p < NP; ++p)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) red[w][p][64 * v + lane] = acc[z][x][p][v];
+            __syncthreads();
+            if (i0 + z >= N) continue;   // uniform over the workgroup
+            double* const h = H + (((size_t)b * NX + x) * N + i0 + z) * PP;
+            int p = 0;
+#pragma unroll
+            for (int a = 0; a < NT; ++a)
+#pragma unroll
+                for (int t = a; t < NT; ++t, ++p) {
+                    const int sc = tid >> 4, tc = tid & 15, ss = a * Rh + sc, tt = t * Rh + tc, tr = 16 * tc + sc;
+                    if (sc < Rh && tc < Rh && ss <= tt && tt < R) {
+                        double v = (red[0][p][tid] + red[1][p][tid]) + (red[2][p][tid] + red[3][p][tid]);
+                        if (a == t)
+                            v = 0.5 * (v + ((red[0][p][tr] + red[1][p][tr]) + (red[2][p][tr] + red[3][p][tr])));
+                        h[sym_col(ss, tt, R)] = v;
+                    }
+                }
+        }
 }
 
-// D[b][x][r][st] (st = s R + t) on FP64 MFMA 16x16x4:
-//   x = 0: sum_i q_r(i) H[b][0][i][st]       (alpha)
-//   x = 1: sum_i q_r(i) H[b][1][i][st]       (d alpha / d phi)
-//   x = 2: sum_i k_i q_r(i) H[b][1][i][st]   (E, the k_i-weighted cos form)
-// One wave per (shape b, H block y, block of 16 columns st): y = 0 makes x =
-// 0, y = 1 makes x = 1 and 2 from the same B loads (each H element is read
-// once); the two r tiles share them too.  K runs over the nodes i, the loads
-// of 4 K-steps issued before their products.
+// D[b][d][r][st] (st a column s <= t) on FP64 MFMA 16x16x4:
+//   d = 0: sum_i q_r(i) H_sin[i][st]       (alpha)
+//   d = 1: sum_i q_r(i) H_cos[i][st]       (d alpha / d phi)
+//   d = 2: sum_i k_i q_r(i) H_cos[i][st]   (E, the k_i-weighted cos form)
+// One workgroup per (shape b, plane of H, block of 16 columns st): the sin
+// plane makes d = 0, the cos plane d = 1 and 2 from the same B loads (each H
+// element is read once); the r tiles share them too.  The four waves take a
+// quarter of the nodes' K-steps each (a chain of N / 64 dependent loads instead
+// of N / 16) and are summed through LDS.  32 shapes, 300 nodes, 30 functions:
+// 70 -> 34 us (half of it from s <= t), one shape of 200 nodes 19 -> 7.9.
 //
 // E gives d alpha / d omega = sum W K cos(omega K + phi) q_r q_s q_t: W and
 // the cos term are symmetric in the three legs, so each of k_j and k_k can
 // be moved onto leg i by relabelling, and d alpha / d omega [r][s][t] =
 // E[r][s][t] + E[s][r][t] + E[t][s][r].
-__global__ __launch_bounds__(64) void proj_stage3(const double* __restrict__ H, const double* __restrict__ q, int ldq,
-                                                  const double* __restrict__ kn, int N, int R, double* __restrict__ D)
+template <int X, int NT>
+__global__ __launch_bounds__(256) void proj_stage3(const double* __restrict__ H, const double* __restrict__ q, int ldq,
+                                                   const double* __restrict__ kn, int N, int R, int PP,
+                                                   double* __restrict__ D)
 {
-    const int lane = threadIdx.x;
-    const int RR = R * R, nblk = (RR + 15) / 16;
-    const int by = blockIdx.x / nblk, st = 16 * (blockIdx.x % nblk) + (lane & 15);
-    const int b = by >> 1, y = by & 1;   // y uniform over the wave
-    const double* const h = H + ((size_t)b * 2 + y) * N * RR + min(st, RR - 1);
-    const int r0 = lane & 15, r1 = 16 + (lane & 15);
-    d4 acc[2][2];   // [w: 0 plain, 1 k-weighted][r tile]
+    constexpr int NX = (X & 1) + (X >> 1), NW = X >> 1, U = 4;
+    __shared__ double red[4][(1 + NW) * NT][256];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, kg = lane >> 4;
+    const int nblk = PP / 16, by = blockIdx.x / nblk, st0 = 16 * (blockIdx.x % nblk);
+    const int b = by / NX, y = X == 2 ? 1 : by % NX;   // y: 0 sin, 1 cos
+    const double* const h = H + (size_t)by * N * PP + st0 + c;
+    d4 acc[1 + NW][NT];   // [0 plain, 1 k-weighted][r tile]
 #pragma unroll
-    for (int w = 0; w < 2; ++w)
+    for (int d = 0; d <= NW; ++d)
 #pragma unroll
-        for (int rt = 0; rt < 2; ++rt) acc[w][rt] = (d4){0.0, 0.0, 0.0, 0.0};
+        for (int a = 0; a < NT; ++a) acc[d][a] = (d4){0.0, 0.0, 0.0, 0.0};
     const int nks = (N + 3) / 4;
-    constexpr int U = 4;
-    for (int k0 = 0; k0 < nks; k0 += U) {
-        double bv[U], a0[U], a1[U], kf[U];
+    for (int k0 = U * w; k0 < nks; k0 += 4 * U) {
+        double bv[U], av[U][NT], kf[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            // K-steps past the last are zero through bv (i >= N)
-            const int i = 4 * (k0 + u) + (lane >> 4);
-            const int ic = min(i, N - 1);
-            bv[u] = i < N ? h[(size_t)ic * RR] : 0.0;
-            a0[u] = r0 < R ? q[(size_t)ic * ldq + r0] : 0.0;
-            a1[u] = r1 < R ? q[(size_t)ic * ldq + r1] : 0.0;
+            const int i = 4 * (k0 + u) + kg, ic = min(i, N - 1);
+            bv[u] = h[(size_t)ic * PP];
             kf[u] = kn[ic];
+#pragma unroll
+            for (int a = 0; a < NT; ++a) av[u][a] = q[(size_t)ic * ldq + min(16 * a + c, R - 1)];
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0[u], bv[u], acc[0][0], 0, 0, 0);
-            acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1[u], bv[u], acc[0][1], 0, 0, 0);
-            if (y) {
-                acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(kf[u] * a0[u], bv[u], acc[1][0], 0, 0, 0);
-                acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(kf[u] * a1[u], bv[u], acc[1][1], 0, 0, 0);
+            const bool in = 4 * (k0 + u) + kg < N;
+#pragma unroll
+            for (int a = 0; a < NT; ++a) {
+                const double qa = in ? av[u][a] : 0.0;
+                acc[0][a] = __builtin_amdgcn_mfma_f64_16x16x4f64(qa, bv[u], acc[0][a], 0, 0, 0);
+                if (NW && y) acc[NW][a] = __builtin_amdgcn_mfma_f64_16x16x4f64(kf[u] * qa, bv[u], acc[NW][a], 0, 0, 0);
             }
         }
     }
-    // element v of tile rt: r = 16 rt + 4 v + lane / 16, column st; x = y + w
-    if (st < RR)
 #pragma unroll
-        for (int w = 0; w < 2; ++w)
-            if (w <= y)
+    for (int d = 0; d <= NW; ++d)
 #pragma unroll
-                for (int rt = 0; rt < 2; ++rt)
+        for (int a = 0; a < NT; ++a)
 #pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int r = 16 * rt + 4 * v + (lane >> 4);
-                        if (r < R) D[(((size_t)b * 3 + y + w) * R + r) * RR + st] = acc[w][rt][v];
-                    }
+            for (int v = 0; v < 4; ++v) red[w][d * NT + a][64 * v + lane] = acc[d][a][v];
+    __syncthreads();
+#pragma unroll
+    for (int d = 0; d <= NW; ++d)
+        if (d <= y)
+#pragma unroll
+            for (int a = 0; a < NT; ++a) {
+                const int r = 16 * a + (tid >> 4), e = d * NT + a;
+                if (r < R)
+                    D[(((size_t)b * 3 + y + d) * R + r) * PP + st0 + (tid & 15)] =
+                        (red[0][e][tid] + red[1][e][tid]) + (red[2][e][tid] + red[3][e][tid]);
+            }
 }
 
-// alpha[b][m] = D[b][0][r][s R + t], d alpha / d omega = E[r][s][t] +
-// E[s][r][t] + E[t][s][r] (E = D[b][2]), d alpha / d phi = D[b][1][r][s R +
-// t], (r, s, t) = order[m], written in the caller's layout: alpha[b][m] and
-// dalpha[b][x][m] (x = 0: omega, 1: phi).
-__global__ void proj_stage3_modes(const double* __restrict__ D, int R, const int* __restrict__ modes, int n, int nb,
-                                  double* __restrict__ alpha, double* __restrict__ dalpha)
+// The sum of a plane of D over the three legs that a mode (r, s, t) may have
+// on the node i: d alpha / d omega from E = D[b][2], and three times alpha and d
+// alpha / d phi from D[b][0] and D[b][1], where the three are equal but for
+// their stage-1 roundings.
+__device__ __forceinline__ double legs(const double* __restrict__ E, int r, int s, int t, int R, int PP)
+{
+    return E[(size_t)r * PP + sym_col(s, t, R)] + E[(size_t)s * PP + sym_col(r, t, R)] +
+           E[(size_t)t * PP + sym_col(s, r, R)];
+}
+
+// alpha[b][m], d alpha / d omega and d alpha / d phi of the modes (r, s, t) =
+// order[m], written in the caller's layout: alpha[b][m] and dalpha[b][x][m] (x =
+// 0: omega, 1: phi); nx = 3, or 1 for alpha alone.
+__global__ void proj_stage3_modes(const double* __restrict__ D, int R, int PP, const int* __restrict__ modes, int n,
+                                  int nb, int nx, double* __restrict__ alpha, double* __restrict__ dalpha)
 {
     const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nb * 3 * n) return;
-    const int m = e % n, x = (e / n) % 3, b = e / (3 * n);
+    if (e >= nb * nx * n) return;
+    const int m = e % n, x = (e / n) % nx, b = e / (nx * n);
     const int pk = modes[m], r = pk & 255, s = (pk >> 8) & 255, t = (pk >> 16) & 255;
-    const int RR = R * R;
-    const double* const Db = D + (size_t)b * 3 * R * RR;
-    if (x == 0) alpha[(size_t)b * n + m] = Db[(size_t)r * RR + s * R + t];
-    else if (x == 1) dalpha[((size_t)b * 2 + 1) * n + m] = Db[(size_t)R * RR + (size_t)r * RR + s * R + t];
-    else {
-        const double* const E = Db + 2 * (size_t)R * RR;
-        dalpha[(size_t)b * 2 * n + m] = E[(size_t)r * RR + s * R + t] + E[(size_t)s * RR + r * R + t] +
-                                        E[(size_t)t * RR + s * R + r];
-    }
+    const double v = legs(D + ((size_t)b * 3 + x) * R * PP, r, s, t, R, PP);
+    if (x == 0) alpha[(size_t)b * n + m] = v / 3.0;
+    else if (x == 1) dalpha[((size_t)b * 2 + 1) * n + m] = v / 3.0;
+    else dalpha[(size_t)b * 2 * n + m] = v;
 }
 
 // ---- adjoint ---------------------------------------------------------------
-// With Gb[r][s][t] = gbar[b][m] at (r, s, t) = order[m] (0 elsewhere) and
-// Gh[r][s][t] = Gb[r][s][t] + Gb[s][r][t] + Gb[t][s][r]:
-//   dL/domega = sum Gb (E[r][s][t] + E[s][r][t] + E[t][s][r]) = sum Gh E,
-//   dL/dphi   = sum Gb Dphi = sum Gh Dphi / 3
-// (Dphi is symmetric in r, s, t, and Gh / 3 has the symmetric part of Gb).
-// Both are then sum_i {k_i, 1/3} P_i with P_i = sum_{j,t} Gbar(i,j,t)
-// G_1(i,j,t), Gbar(i,j,t) = sum_s q_s(j) Hbar[i][s][t], Hbar[i][s][t] =
-// sum_r q_r(i) Gh[r][s][t].
-//
-// Hbar[b][i][s][t]: per shape a product Q (N x R) . Gh (R x R^2) on FP64
-// MFMA 16x16x4, Gh gathered through slot[r][s][t] = m (-1: no mode).  One
-// wave per (shape b, block of 16 columns st): its B operand (Gh, R padded to
-// 32) is gathered once into registers, then the N / 16 row tiles of Q run
-// through 8 K-steps each.
-__global__ __launch_bounds__(64) void proj_hbar(const double* __restrict__ gbar, const int* __restrict__ slot,
-                                                const double* __restrict__ q, int ldq, int N, int R, int n, int nb,
-                                                double* __restrict__ Hb)
+// dtheta[b] = sum_m gbar[b][m] (d alpha_m / d omega, d alpha_m / d phi), one
+// workgroup per shape: thread l sums m = l, l + 512, ..., then the waves and
+// the workgroup are summed in a fixed order.  (32 shapes of 4960 modes: 14 us;
+// the contraction of gbar with the basis that this replaces, 62.)
+__global__ __launch_bounds__(512) void proj_dtheta(const double* __restrict__ D, int R, int PP,
+                                                   const int* __restrict__ modes, int n,
+                                                   const double* __restrict__ gbar, double* __restrict__ out)
 {
-    const int lane = threadIdx.x;
-    const int RR = R * R, nblk = (RR + 15) / 16;
-    const int b = blockIdx.x / nblk, st = 16 * (blockIdx.x % nblk) + (lane & 15);
-    double bv[8];
-    const int s = min(st, RR - 1) / R, t = min(st, RR - 1) % R;
-    auto g = [&](int m) { return m >= 0 ? gbar[(size_t)b * n + m] : 0.0; };
-#pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-        const int r = 4 * ks + (lane >> 4);
-        bv[ks] = 0.0;
-        if (r < R && st < RR)
-            bv[ks] = g(slot[r * RR + s * R + t]) + g(slot[s * RR + r * R + t]) + g(slot[t * RR + s * R + r]);
+    __shared__ double part[8][2];
+    const int b = blockIdx.x, tid = threadIdx.x;
+    const size_t plane = (size_t)R * PP;
+    const double* const P = D + ((size_t)b * 3 + 1) * plane;
+    const double* const E = P + plane;
+    double so = 0.0, sp = 0.0;
+#pragma unroll 4
+    for (int m = tid; m < n; m += 512) {
+        const int pk = modes[m], r = pk & 255, s = (pk >> 8) & 255, t = (pk >> 16) & 255;
+        const double g = gbar[(size_t)b * n + m];
+        so += g * legs(E, r, s, t, R, PP);
+        sp += g * (legs(P, r, s, t, R, PP) / 3.0);
     }
-    for (int i0 = 0; i0 < N; i0 += 16) {
-        const int ia = min(i0 + (lane & 15), N - 1);   // A row (rows past N: the last, not stored)
-        d4 acc = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const int r = 4 * ks + (lane >> 4);
-            const double a = r < R ? q[(size_t)ia * ldq + r] : 0.0;
-            acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a, bv[ks], acc, 0, 0, 0);
-        }
-        // element v: row i0 + 4 v + lane / 16, column st
-        if (st < RR)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int i = i0 + 4 * v + (lane >> 4);
-                if (i < N) Hb[((size_t)b * N + i) * RR + st] = acc[v];
-            }
+    for (int d = 32; d > 0; d >>= 1) {
+        so += __shfl_xor(so, d);
+        sp += __shfl_xor(sp, d);
     }
-}
-
-// dpart[b][i] = (k_i P_i, P_i / 3), P_i = sum_{j,t} Gbar(i,j,t) G_1(i,j,t), for
-// one (b, i) per workgroup
-template <class T>
-__global__ __launch_bounds__(256) void proj_adjoint(const T* __restrict__ Y, int ldy, const int* __restrict__ rowof,
-                                                    const double* __restrict__ kn,
-                                                    const double* __restrict__ q, int ldq, int N, int R,
-                                                    const double* __restrict__ theta, int nb,
-                                                    const double* __restrict__ scb,
-                                                    const double* __restrict__ Hb, double* __restrict__ dpart)
-{
-    // one workgroup per (shape b, node i), over chunks of 32 nodes j:
-    // Gbar[j][t] = sum_s q_s(j) Hbar[s][t] on FP64 MFMA 16x16x4 (A = Q, j x s;
-    // B = Hbar, s x t; wave w owns the j tile w / 2 and the t tile w % 2),
-    // then each lane adds Gbar G_1 at its 4 output elements.  The Y and sin /
-    // cos omega k_j of those elements and the basis entries of Qs in the next
-    // chunk are loaded while the current chunk's products run.
-    __shared__ double Hs[32][32];   // [s][t]
-    __shared__ double Qs[32][32];   // [s][j in chunk]
-    __shared__ double red[256];
-    const int b = blockIdx.x % nb, i = blockIdx.x / nb;
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int jm = 16 * (w >> 1), tn = 16 * (w & 1);
-    const int t = tn + (lane & 15);   // the lane's output column; rows jm + 4 v + lane / 16
-    const double ki = kn[i];
-    double sa, ca;   // sin, cos of omega k_i + phi
-    sincos(theta[2 * b] * ki + theta[2 * b + 1], &sa, &ca);
-    const double* const sc = scb + 2 * (size_t)b * N;
-    for (int e = tid; e < 32 * 32; e += 256) {
-        const int ss = e >> 5, tt = e & 31;
-        Hs[ss][tt] = (ss < R && tt < R) ? Hb[(((size_t)b * N) + i) * R * R + ss * R + tt] : 0.0;
+    if ((tid & 63) == 0) {
+        part[tid >> 6][0] = so;
+        part[tid >> 6][1] = sp;
     }
-    T yv[4][2];
-    double sv[4], cv[4], qn[4];
-    // the lane's elements (j0 + jm + 4 v + lane / 16, t) of a chunk and the
-    // thread's 4 entries of its Qs (nodes past N: the last node; columns past
-    // R: the last column; all unused)
-    auto fetch = [&](int j0) {
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const int j = min(j0 + jm + 4 * v + (lane >> 4), N - 1), tt = min(t, R - 1);
-            const T* y = Y + (size_t)rowof[pair_row(i, j, N)] * ldy + (size_t)b * 2 * R + tt;
-            yv[v][0] = y[0];
-            yv[v][1] = y[R];
-            sv[v] = sc[2 * j];
-            cv[v] = sc[2 * j + 1];
-        }
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = tid + 256 * k, ss = e >> 5, jj = e & 31;
-            qn[k] = q[(size_t)min(j0 + jj, N - 1) * ldq + min(ss, R - 1)];
-        }
-    };
-    double pacc = 0.0;
-    fetch(0);
-    for (int j0 = 0; j0 < N; j0 += 32) {
-        __syncthreads();   // Hs written / the previous chunk is done with Qs
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            const int e = tid + 256 * k, ss = e >> 5, jj = e & 31;
-            Qs[ss][jj] = (ss < R && j0 + jj < N) ? qn[k] : 0.0;
-        }
-        __syncthreads();
-        // this chunk's element data, then the next chunk's loads
-        T yc[4][2];
-        double scs[4], ccs[4];
-#pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            yc[v][0] = yv[v][0];
-            yc[v][1] = yv[v][1];
-            scs[v] = sv[v];
-            ccs[v] = cv[v];
-        }
-        fetch(min(j0 + 32, N - 1));
-        d4 gb = {0.0, 0.0, 0.0, 0.0};
-#pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
-            const int ss = 4 * ks + (lane >> 4);
-            gb = __builtin_amdgcn_mfma_f64_16x16x4f64(Qs[ss][jm + (lane & 15)], Hs[ss][t], gb, 0, 0, 0);
-        }
-        if (t < R)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                if (j0 + jm + 4 * v + (lane >> 4) < N) {
-                    const double sA = sa * ccs[v] + ca * scs[v], cA = ca * ccs[v] - sa * scs[v];
-                    const double yr = (double)yc[v][0], ys = (double)yc[v][1];
-                    pacc += gb[v] * (cA * yr - sA * ys);
-                }
-            }
-    }
-    red[tid] = pacc;
     __syncthreads();
-    for (int wd = 128; wd > 0; wd >>= 1) {
-        if (tid < wd) red[tid] += red[tid + wd];
-        __syncthreads();
-    }
-    if (tid == 0) {
-        dpart[((size_t)b * N + i) * 2] = ki * red[0];
-        dpart[((size_t)b * N + i) * 2 + 1] = red[0] * (1.0 / 3.0);
+    if (tid < 2) {
+        double v = 0.0;
+        for (int w = 0; w < 8; ++w) v += part[w][tid];
+        out[2 * b + tid] = v;
     }
 }
-
-// dtheta[b][x] = sum_i dpart[b][i][x]: one wave per (b, x), lane l summing
-// i = l, l + 64, ..., then a butterfly over the lanes (a fixed order)
-__global__ __launch_bounds__(64) void proj_sum_parts(const double* __restrict__ dpart, int N, int nb,
-                                                     double* __restrict__ out)
-{
-    const int e = blockIdx.x, b = e / 2, x = e % 2, lane = threadIdx.x;
-    double s = 0.0;
-    for (int i = lane; i < N; i += 64) s += dpart[((size_t)b * N + i) * 2 + x];
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
-    if (lane == 0) out[e] = s;
-}
-
-// ---- host side ---------------------------------------------------------------
 
 static int ensure_W(mcmb_ctx* c, int prec)
 {
@@ -576,10 +570,10 @@ static int ensure_W(mcmb_ctx* c, int prec)
     // The pair rows i <= j in an order that groups rows of like nonzero k
     // range: W_ijk is nonzero only for k_k in [k_j - k_i, k_i + k_j] (the
     // triangle), so with the rows sorted by (upper end / PK, lower end) most
-    // K chunks of a PT-row tile are zero throughout, and the GEMMs skip them
+    // K chunks of a WT-row tile are zero throughout, and the GEMMs skip them
     // (43% of the chunks remain at 300 nodes, against 87% in i-major pair
     // order).  Each row's k-sum is unchanged, so Y holds the same values in
-    // W's row order; wrow[pair_row(i, j)] is the row of (i, j).
+    // W's row order; wrow[stage2_row(i, j)] is the row of (i, j) or (j, i).
     const std::vector<double>& kn = K.kn;
     std::vector<int2> rowij;
     std::vector<long> key;
@@ -596,17 +590,37 @@ static int ensure_W(mcmb_ctx* c, int prec)
     for (long r = 0; r < M; ++r) ord[r] = r;
     std::stable_sort(ord.begin(), ord.end(), [&](long a, long b) { return key[a] < key[b]; });
     std::vector<int2> rows(M);
-    std::vector<int> wrow(M);
+    const int Np = stage2_nodes(N);
+    std::vector<int> rowof(M), wrow((size_t)N * Np);
     for (long r = 0; r < M; ++r) {
         rows[r] = rowij[ord[r]];
-        wrow[ord[r]] = (int)r;   // rowij is in pair_row order
+        rowof[ord[r]] = (int)r;   // rowij is in i-major pair order
     }
+    {
+        long m = 0;
+        for (int i = 0; i < N; ++i)
+            for (int j = i; j < N; ++j, ++m)
+                wrow[stage2_row(i, j, Np)] = wrow[stage2_row(j, i, Np)] = rowof[m];
+        for (int i = 0; i < N; ++i)
+            for (int j = N; j < Np; ++j) wrow[stage2_row(i, j, Np)] = wrow[stage2_row(i, N - 1, Np)];
+    }
+    // stage 2's basis operand: (j, c) -> the columns a Rh + c of its NT tiles,
+    // zero past the nodes and the columns
+    const BasisTiles bt = basis_tiles(K.R);
+    std::vector<double> qt((size_t)Np * 16 * bt.NT, 0.0);
+    for (int j = 0; j < N; ++j)
+        for (int c = 0; c < bt.Rh; ++c)
+            for (int a = 0; a < bt.NT; ++a)
+                if (a * bt.Rh + c < K.R)
+                    qt[((size_t)j * 16 + c) * bt.NT + a] = K.q[(size_t)j * K.ldq + a * bt.Rh + c];
+    MCMB_TRY(c->d_pq.alloc(sizeof(double) * qt.size()));
+    MCMB_HIP(hipMemcpyAsync(c->d_pq.p, qt.data(), sizeof(double) * qt.size(), hipMemcpyHostToDevice, c->stream));
     DevBuf d_ij;
     MCMB_TRY(d_ij.alloc(sizeof(int2) * (size_t)M));
     MCMB_HIP(hipMemcpyAsync(d_ij.p, rows.data(), sizeof(int2) * (size_t)M, hipMemcpyHostToDevice, c->stream));
-    MCMB_TRY(c->d_wrow.alloc(sizeof(int) * (size_t)M));
-    MCMB_HIP(hipMemcpyAsync(c->d_wrow.p, wrow.data(), sizeof(int) * (size_t)M, hipMemcpyHostToDevice, c->stream));
-    const unsigned ntile = (unsigned)((M + PT - 1) / PT);
+    MCMB_TRY(c->d_wrow.alloc(sizeof(int) * wrow.size()));
+    MCMB_HIP(hipMemcpyAsync(c->d_wrow.p, wrow.data(), sizeof(int) * wrow.size(), hipMemcpyHostToDevice, c->stream));
+    const unsigned ntile = (unsigned)((M + WT - 1) / WT);
     MCMB_TRY(c->d_wtile.alloc(sizeof(int2) * ntile));
     size_t tot = (size_t)M * Kp;
     MCMB_TRY(launch_guard("projection weight cube", (tot + 255) / 256, 256));
@@ -626,76 +640,85 @@ static int ensure_W(mcmb_ctx* c, int prec)
                            (const float*)c->d_W.as<float>(), M, Kp, c->d_wtile.as<int2>());
     }
     MCMB_HIP(hipGetLastError());
-    MCMB_HIP(hipStreamSynchronize(c->stream));   // the pair table goes out of scope
+    MCMB_HIP(hipStreamSynchronize(c->stream));   // the host tables go out of scope
     c->w_ready = prec + 1;
     return MCMB_OK;
 }
 
-// Leading dimension of stage 1's Z and Y for a batch of nb shapes (4R
-// columns per shape, rounded up to whole GEMM tiles).
+// Leading dimension of stage 1's Z and Y for a batch of nb shapes (whole GEMM
+// tiles).
 static int stage1_ld(int nb, int R)
 {
-    return (nb * 2 * R + PT - 1) / PT * PT;
+    return (nb * basis_tiles(R).cols + WT - 1) / WT * WT;
 }
 
-// FP32 stage-1 GEMM C[m][ldc] = A[m][Kp] B[Kp][ldb] (B zero-padded to ldb
-// columns and Kp rows, A to Kp columns): 128 x 128 tiles, 4 waves of
-// 64 x 64 on v_mfma_f32_16x16x4f32, K chunks of 16 in double-buffered LDS,
-// over the tile's chunks ktiles[tile] = (first, count) only (A is zero in
-// the others).  Operands come in as 16-byte loads two chunks ahead of their
-// use (two register sets), A stored [m][k] and B [k][n] with row strides (20
-// and 144 floats) that keep both the 16-byte stores and the MFMA operand
-// reads free of bank conflicts.  The chunks run in K order.
-constexpr int PF_LDA = PK + 4, PF_LDB = PT + 16;
-__global__ __launch_bounds__(256, 2) void proj_gemm_f32(const float* __restrict__ A, const float* __restrict__ B,
-                                                        int M, int Kp, int ldb, float* __restrict__ C, int ldc,
-                                                        const int2* __restrict__ ktiles)
+// Stage-1 GEMM C[m][ldc] = A[m][Kp] B[Kp][ldb] (B zero-padded to ldb columns
+// and Kp rows, A to Kp columns): 64 x 64 tiles, 4 waves of 32
+// x 32 on v_mfma_{f32,f64}_16x16x4, K chunks of 16 in
+// double-buffered LDS, over the chunks ktiles[row tile] = (first, count)
+// only (A is zero in the others).  Operands come in as 16-byte loads two chunks
+// ahead of their use (two register sets), A stored [m][k] and B [k][n] with row
+// strides that keep both the 16-byte stores and the MFMA operand reads free of
+// bank conflicts.  The chunks run in K order.
+//
+// 64 x 64 tiles were never slower than 128 x 128 (two of those fit a CU): one
+// shape of 200 nodes and 20 functions, 40 columns of which a 128-wide tile
+// pads two thirds, 15.9 against 36.6 us in FP64; 8 shapes 33 against 54; 32
+// shapes 98 against 111; 32 shapes of 300 nodes and 30 functions in FP32 259
+// both.
+template <class T>
+__global__ __launch_bounds__(256, 4) void proj_gemm_w(const T* __restrict__ A, const T* __restrict__ B, int M, int Kp,
+                                                      int ldb, T* __restrict__ C, int ldc,
+                                                      const int2* __restrict__ ktiles)
 {
-    __shared__ __align__(16) float As[2][PT][PF_LDA];
-    __shared__ __align__(16) float Bs[2][PK][PF_LDB];
-    const int m0 = blockIdx.y * PT, n0 = blockIdx.x * PT;
+    constexpr int TL = WT / 32;                                  // 16 x 16 tiles of a wave, each way
+    constexpr int EV = 16 / sizeof(T);                           // elements of a load
+    constexpr int LDA = PK + EV, LDB = WT + 64 / sizeof(T);      // LDS row strides
+    constexpr int NL = WT * PK / EV / 256;                       // loads of A (and of B) a thread and chunk
+    constexpr int QA = PK / EV, QB = WT / EV;                    // loads of an A row, of a B row
+    typedef T TV __attribute__((ext_vector_type(EV)));
+    typedef typename MF<T>::V Acc;
+    __shared__ __align__(16) T As[2][WT][LDA];
+    __shared__ __align__(16) T Bs[2][PK][LDB];
+    const int m0 = blockIdx.y * WT, n0 = blockIdx.x * WT;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
-    f4 acc[4][4];
+    Acc acc[TL][TL];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < TL; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = (f4){0.f, 0.f, 0.f, 0.f};
-    // a chunk is 512 float4 of A (row r = e / 4, k = 4 (e % 4)) and 512 of B
-    // (k = e / 32, n = 4 (e % 32)), e = tid + 256 u
-    const f4 z4 = {0.f, 0.f, 0.f, 0.f};
-    auto gload = [&](int k0, f4 (&ra)[2], f4 (&rb)[2]) {
+        for (int b = 0; b < TL; ++b) acc[a][b] = (Acc){0, 0, 0, 0};
+    // load e = tid + 256 u of a chunk: A row e / QA, k = EV (e % QA); B row k =
+    // e / QB, n = EV (e % QB).  Rows of A past M repeat the last one (not stored).
+    auto gload = [&](int k0, TV (&ra)[NL], TV (&rb)[NL]) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < NL; ++u) {
             const int e = tid + 256 * u;
-            const int r = e >> 2, kq = e & 3, gm = m0 + r;
-            ra[u] = gm < M ? *reinterpret_cast<const f4*>(A + (size_t)gm * Kp + k0 + 4 * kq) : z4;
-            const int kb = e >> 5, c4 = e & 31;
-            rb[u] = *reinterpret_cast<const f4*>(B + (size_t)(k0 + kb) * ldb + n0 + 4 * c4);
+            ra[u] = *reinterpret_cast<const TV*>(A + (size_t)min(m0 + e / QA, M - 1) * Kp + k0 + EV * (e % QA));
+            rb[u] = *reinterpret_cast<const TV*>(B + (size_t)(k0 + e / QB) * ldb + n0 + EV * (e % QB));
         }
     };
-    auto sstore = [&](int buf, const f4 (&ra)[2], const f4 (&rb)[2]) {
+    auto sstore = [&](int buf, const TV (&ra)[NL], const TV (&rb)[NL]) {
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int u = 0; u < NL; ++u) {
             const int e = tid + 256 * u;
-            *reinterpret_cast<f4*>(&As[buf][e >> 2][4 * (e & 3)]) = ra[u];
-            *reinterpret_cast<f4*>(&Bs[buf][e >> 5][4 * (e & 31)]) = rb[u];
+            *reinterpret_cast<TV*>(&As[buf][e / QA][EV * (e % QA)]) = ra[u];
+            *reinterpret_cast<TV*>(&Bs[buf][e / QB][EV * (e % QB)]) = rb[u];
         }
     };
     auto compute = [&](int buf) {
 #pragma unroll
         for (int ks = 0; ks < PK / 4; ++ks) {
             const int kk = ks * 4 + (lane >> 4);
-            float av[4], bv[4];
+            T av[TL], bv[TL];
 #pragma unroll
-            for (int a = 0; a < 4; ++a) av[a] = As[buf][wm * 64 + a * 16 + (lane & 15)][kk];
+            for (int a = 0; a < TL; ++a) av[a] = As[buf][(wm * TL + a) * 16 + (lane & 15)][kk];
 #pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = Bs[buf][kk][wn * 64 + b * 16 + (lane & 15)];
+            for (int b = 0; b < TL; ++b) bv[b] = Bs[buf][kk][(wn * TL + b) * 16 + (lane & 15)];
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < TL; ++a)
 #pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[a], bv[b], acc[a][b], 0, 0, 0);
+                for (int b = 0; b < TL; ++b) acc[a][b] = MF<T>::mma(av[a], bv[b], acc[a][b]);
         }
     };
     // the tile's chunks c0 .. c0 + nk - 1 (the rest of W's rows here are
@@ -704,7 +727,7 @@ __global__ __launch_bounds__(256, 2) void proj_gemm_f32(const float* __restrict_
     // every load is unconditional
     const int2 kr = ktiles[blockIdx.y];
     const int c0 = kr.x, nk = kr.y;
-    f4 ra0[2], rb0[2], ra1[2], rb1[2];
+    TV ra0[NL], rb0[NL], ra1[NL], rb1[NL];
     gload(c0 * PK, ra0, rb0);
     gload((c0 + min(1, nk - 1)) * PK, ra1, rb1);
     sstore(0, ra0, rb0);
@@ -722,102 +745,13 @@ __global__ __launch_bounds__(256, 2) void proj_gemm_f32(const float* __restrict_
         if (kc + 2 >= nk) break;
     }
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < TL; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int gm = m0 + wm * 64 + a * 16 + MF<float>::row(v, lane);
-                const int gn = n0 + wn * 64 + b * 16 + (lane & 15);
-                if (gm < M) C[(size_t)gm * ldc + gn] = acc[a][b][v];
-            }
-}
-
-// FP64 stage-1 GEMM, the same scheme with 16-byte (two-double) operand
-// loads two chunks ahead: a chunk is 1024 double2 of A (row r = e / 8, k = 2
-// (e % 8)) and 1024 of B (k = e / 64, n = 2 (e % 64)), e = tid + 256 u, u <
-// 4.  A is stored [m][k] with a row stride of 18 doubles (16-byte aligned
-// rows), B [k][n] with 136.  It issues the MFMA sequence of proj_gemm<double>
-// (same operands, same K order).
-constexpr int PD_LDA = PK + 2, PD_LDB = PT + 8;
-typedef double d2v __attribute__((ext_vector_type(2)));
-__global__ __launch_bounds__(256, 2) void proj_gemm_f64(const double* __restrict__ A, const double* __restrict__ B,
-                                                        int M, int Kp, int ldb, double* __restrict__ C, int ldc,
-                                                        const int2* __restrict__ ktiles)
-{
-    __shared__ __align__(16) double As[2][PT][PD_LDA];
-    __shared__ __align__(16) double Bs[2][PK][PD_LDB];
-    const int m0 = blockIdx.y * PT, n0 = blockIdx.x * PT;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
-    d4 acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = (d4){0.0, 0.0, 0.0, 0.0};
-    const d2v z2 = {0.0, 0.0};
-    auto gload = [&](int k0, d2v (&ra)[4], d2v (&rb)[4]) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            const int r = e >> 3, kq = e & 7, gm = m0 + r;
-            ra[u] = gm < M ? *reinterpret_cast<const d2v*>(A + (size_t)gm * Kp + k0 + 2 * kq) : z2;
-            const int kb = e >> 6, c2 = e & 63;
-            rb[u] = *reinterpret_cast<const d2v*>(B + (size_t)(k0 + kb) * ldb + n0 + 2 * c2);
-        }
-    };
-    auto sstore = [&](int buf, const d2v (&ra)[4], const d2v (&rb)[4]) {
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-            const int e = tid + 256 * u;
-            *reinterpret_cast<d2v*>(&As[buf][e >> 3][2 * (e & 7)]) = ra[u];
-            *reinterpret_cast<d2v*>(&Bs[buf][e >> 6][2 * (e & 63)]) = rb[u];
-        }
-    };
-    auto compute = [&](int buf) {
-#pragma unroll
-        for (int ks = 0; ks < PK / 4; ++ks) {
-            const int kk = ks * 4 + (lane >> 4);
-            double av[4], bv[4];
-#pragma unroll
-            for (int a = 0; a < 4; ++a) av[a] = As[buf][wm * 64 + a * 16 + (lane & 15)][kk];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) bv[b] = Bs[buf][kk][wn * 64 + b * 16 + (lane & 15)];
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-#pragma unroll
-                for (int b = 0; b < 4; ++b)
-                    acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(av[a], bv[b], acc[a][b], 0, 0, 0);
-        }
-    };
-    // the tile's chunks c0 .. c0 + nk - 1, as proj_gemm_f32
-    const int2 kr = ktiles[blockIdx.y];
-    const int c0 = kr.x, nk = kr.y;
-    d2v ra0[4], rb0[4], ra1[4], rb1[4];
-    gload(c0 * PK, ra0, rb0);
-    gload((c0 + min(1, nk - 1)) * PK, ra1, rb1);
-    sstore(0, ra0, rb0);
-    __syncthreads();
-    for (int kc = 0;; kc += 2) {
-        gload((c0 + min(kc + 2, nk - 1)) * PK, ra0, rb0);
-        compute(0);
-        sstore(1, ra1, rb1);
-        __syncthreads();
-        if (kc + 1 >= nk) break;
-        gload((c0 + min(kc + 3, nk - 1)) * PK, ra1, rb1);
-        compute(1);
-        sstore(0, ra0, rb0);
-        __syncthreads();
-        if (kc + 2 >= nk) break;
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b)
+        for (int b = 0; b < TL; ++b)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int gm = m0 + wm * 64 + a * 16 + MF<double>::row(v, lane);
-                const int gn = n0 + wn * 64 + b * 16 + (lane & 15);
+                const int gm = m0 + (wm * TL + a) * 16 + MF<T>::row(v, lane);
+                const int gn = n0 + (wn * TL + b) * 16 + (lane & 15);
                 if (gm < M) C[(size_t)gm * ldc + gn] = acc[a][b][v];
             }
 }
@@ -836,15 +770,9 @@ static int run_stage1(mcmb_ctx* c, const double* d_theta, int nb, int& ldy, DevB
     size_t ze = (size_t)Kp * ldz;
     hipLaunchKernelGGL(proj_build_Z<T>, dim3((unsigned)((ze + 255) / 256)), dim3(256), 0, c->stream,
                        K.d_kn.as<double>(), K.d_q.as<double>(), K.ldq, N, R, d_theta, nb, Kp, ldz, Zb.as<T>());
-    dim3 grid((unsigned)(ldz / PT), (unsigned)((M + PT - 1) / PT));
-    if (std::is_same<T, float>::value)
-        hipLaunchKernelGGL(proj_gemm_f32, grid, dim3(256), 0, c->stream, (const float*)c->d_W.as<T>(),
-                           (const float*)Zb.as<T>(), (int)M, Kp, ldz, (float*)Yb.as<T>(), ldy,
-                           (const int2*)c->d_wtile.as<int2>());
-    else
-        hipLaunchKernelGGL(proj_gemm_f64, grid, dim3(256), 0, c->stream, (const double*)c->d_W.as<T>(),
-                           (const double*)Zb.as<T>(), (int)M, Kp, ldz, (double*)Yb.as<T>(), ldy,
-                           (const int2*)c->d_wtile.as<int2>());
+    const dim3 grid((unsigned)(ldz / WT), (unsigned)((M + WT - 1) / WT));
+    hipLaunchKernelGGL(proj_gemm_w<T>, grid, dim3(256), 0, c->stream, (const T*)c->d_W.as<T>(), (const T*)Zb.as<T>(),
+                       (int)M, Kp, ldz, Yb.as<T>(), ldy, (const int2*)c->d_wtile.as<int2>());
     MCMB_HIP(hipGetLastError());
     return MCMB_OK;
 }
@@ -852,37 +780,58 @@ static int run_stage1(mcmb_ctx* c, const double* d_theta, int nb, int& ldy, DevB
 // sin / cos of omega_b k_j for the nb shapes of a batch into c->psc
 static int sincos_table(mcmb_ctx* c, const double* d_theta, int nb)
 {
-    const int N = c->ks.lmax + 1;
-    MCMB_TRY(c->psc.alloc(sizeof(double) * 2 * (size_t)PBATCH * N));
-    hipLaunchKernelGGL(proj_sincos_tab, dim3((unsigned)((nb * N + 255) / 256)), dim3(256), 0, c->stream,
-                       c->ks.d_kn.as<double>(), d_theta, N, nb, c->psc.as<double>());
+    const int N = c->ks.lmax + 1, Np = stage2_nodes(N);
+    MCMB_TRY(c->psc.alloc(sizeof(double) * 2 * (size_t)PBATCH * Np));
+    hipLaunchKernelGGL(proj_sincos_tab, dim3((unsigned)((nb * Np + 255) / 256)), dim3(256), 0, c->stream,
+                       c->ks.d_kn.as<double>(), d_theta, N, Np, nb, c->psc.as<double>());
+    MCMB_HIP(hipGetLastError());
+    return MCMB_OK;
+}
+
+// Stages 2 and 3 of a batch from its stage-1 product: D[b][d] (c->pdm) for the
+// planes X (1 sin, 2 cos, 3 both).
+template <class T, int X, int NT>
+static int run_stages23(mcmb_ctx* c, const double* d_theta, int nb, const T* Y, int ldy)
+{
+    PointSet& K = c->ks;
+    constexpr int NX = (X & 1) + (X >> 1);
+    const int N = K.lmax + 1, R = K.R, PP = sym_cols(R);
+    MCMB_TRY(c->ph.alloc(sizeof(double) * (size_t)PBATCH * NX * N * PP));
+    MCMB_TRY(c->pdm.alloc(sizeof(double) * (size_t)PBATCH * 3 * R * PP));
+    MCMB_TRY(sincos_table(c, d_theta, nb));
+    const bool two = X != 3 && (long)nb * N >= S2_PAIR;
+    const int ni = two ? (N + 1) / 2 : N;
+    const dim3 grid((unsigned)((ni + 7) / 8 * 8 * nb));
+    auto* const k2 = two ? proj_stage2<T, X, NT, X != 3 ? 2 : 1> : proj_stage2<T, X, NT, 1>;
+    hipLaunchKernelGGL(k2, grid, dim3(256), 0, c->stream, Y, ldy, (const int*)c->d_wrow.as<int>(), K.d_kn.as<double>(),
+                       (const double*)c->d_pq.as<double>(), N, R, PP, d_theta, nb, (const double*)c->psc.as<double>(),
+                       c->ph.as<double>());
+    hipLaunchKernelGGL((proj_stage3<X, NT>), dim3((unsigned)(nb * NX * (PP / 16))), dim3(256), 0, c->stream,
+                       (const double*)c->ph.as<double>(), K.d_q.as<double>(), K.ldq, K.d_kn.as<double>(), N, R, PP,
+                       c->pdm.as<double>());
     MCMB_HIP(hipGetLastError());
     return MCMB_OK;
 }
 
 // Y is stage 1's product buffer (the context's batch buffer, or a slot of
-// the forward cache).
+// the forward cache).  d_dalpha null: alpha alone.
 template <class T>
 static int project_fwd_batch(mcmb_ctx* c, const double* d_theta, int nb, double* d_alpha /* [nb][n] */,
                              double* d_dalpha /* [nb][2][n] */, DevBuf& Yb)
 {
     PointSet& K = c->ks;
-    const int N = K.lmax + 1, R = K.R, n = K.n;
-    DevBuf& Hb = c->ph;
+    const int R = K.R, n = K.n, nx = d_dalpha ? 3 : 1;
     int ldy = 0;
     MCMB_TRY(run_stage1<T>(c, d_theta, nb, ldy, Yb));
-    MCMB_TRY(Hb.alloc(sizeof(double) * (size_t)PBATCH * 2 * N * R * R));
-    MCMB_TRY(sincos_table(c, d_theta, nb));
-    hipLaunchKernelGGL(proj_stage2<T>, dim3((unsigned)(nb * N)), dim3(256), 0, c->stream, Yb.as<T>(), ldy,
-                       (const int*)c->d_wrow.as<int>(), K.d_kn.as<double>(), K.d_q.as<double>(), K.ldq, N, R, d_theta, nb,
-                       (const double*)c->psc.as<double>(), Hb.as<double>());
-    MCMB_TRY(c->pdm.alloc(sizeof(double) * (size_t)PBATCH * 3 * R * R * R));
-    hipLaunchKernelGGL(proj_stage3, dim3((unsigned)(nb * 2 * ((R * R + 15) / 16))), dim3(64), 0, c->stream,
-                       (const double*)Hb.as<double>(), K.d_q.as<double>(), K.ldq, K.d_kn.as<double>(), N, R,
-                       c->pdm.as<double>());
-    const int ne = nb * 3 * n;
+    const T* const Y = Yb.as<T>();
+    if (d_dalpha)
+        MCMB_TRY(R > 16 ? (run_stages23<T, 3, 2>(c, d_theta, nb, Y, ldy)) : (run_stages23<T, 3, 1>(c, d_theta, nb, Y, ldy)));
+    else
+        MCMB_TRY(R > 16 ? (run_stages23<T, 1, 2>(c, d_theta, nb, Y, ldy)) : (run_stages23<T, 1, 1>(c, d_theta, nb, Y, ldy)));
+    const int ne = nb * nx * n;
     hipLaunchKernelGGL(proj_stage3_modes, dim3((ne + 255) / 256), dim3(256), 0, c->stream,
-                       (const double*)c->pdm.as<double>(), R, K.d_modes.as<int>(), n, nb, d_alpha, d_dalpha);
+                       (const double*)c->pdm.as<double>(), R, sym_cols(R), K.d_modes.as<int>(), n, nb, nx, d_alpha,
+                       d_dalpha);
     MCMB_HIP(hipGetLastError());
     return MCMB_OK;
 }
@@ -890,13 +839,11 @@ static int project_fwd_batch(mcmb_ctx* c, const double* d_theta, int nb, double*
 // Ycached: stage 1's product of this batch from the forward cache, or null to
 // compute it.
 template <class T>
-static int project_bwd_batch(mcmb_ctx* c, const double* d_theta, int nb, const double* d_gbar, const int* d_slot,
-                             double* d_dtheta, DevBuf* Ycached)
+static int project_bwd_batch(mcmb_ctx* c, const double* d_theta, int nb, const double* d_gbar, double* d_dtheta,
+                             DevBuf* Ycached)
 {
     PointSet& K = c->ks;
     const int N = K.lmax + 1, R = K.R, n = K.n;
-    DevBuf& Hb = c->ph;
-    DevBuf& Dp = c->pd;
     // a cached product is this batch's own: same shape count, so the same
     // leading dimension; anything smaller than that is recomputed
     const long M = (long)N * (N + 1) / 2;
@@ -904,17 +851,10 @@ static int project_bwd_batch(mcmb_ctx* c, const double* d_theta, int nb, const d
     if (Ycached && Ycached->bytes < sizeof(T) * (size_t)M * ldy) Ycached = nullptr;
     DevBuf& Yb = Ycached ? *Ycached : c->py;
     if (!Ycached) MCMB_TRY(run_stage1<T>(c, d_theta, nb, ldy, Yb));
-    MCMB_TRY(Hb.alloc(sizeof(double) * (size_t)PBATCH * N * R * R));
-    MCMB_TRY(Dp.alloc(sizeof(double) * (size_t)PBATCH * N * 2));
-    const unsigned hblocks = (unsigned)(nb * ((R * R + 15) / 16));
-    hipLaunchKernelGGL(proj_hbar, dim3(hblocks), dim3(64), 0, c->stream, d_gbar, d_slot, K.d_q.as<double>(), K.ldq,
-                       N, R, n, nb, Hb.as<double>());
-    MCMB_TRY(sincos_table(c, d_theta, nb));
-    hipLaunchKernelGGL(proj_adjoint<T>, dim3((unsigned)(nb * N)), dim3(256), 0, c->stream, Yb.as<T>(), ldy,
-                       (const int*)c->d_wrow.as<int>(), K.d_kn.as<double>(), K.d_q.as<double>(), K.ldq, N, R, d_theta, nb,
-                       (const double*)c->psc.as<double>(), Hb.as<double>(), Dp.as<double>());
-    hipLaunchKernelGGL(proj_sum_parts, dim3((unsigned)(nb * 2)), dim3(64), 0, c->stream, Dp.as<double>(), N, nb,
-                       d_dtheta);
+    const T* const Y = Yb.as<T>();
+    MCMB_TRY(R > 16 ? (run_stages23<T, 2, 2>(c, d_theta, nb, Y, ldy)) : (run_stages23<T, 2, 1>(c, d_theta, nb, Y, ldy)));
+    hipLaunchKernelGGL(proj_dtheta, dim3((unsigned)nb), dim3(512), 0, c->stream, (const double*)c->pdm.as<double>(), R,
+                       sym_cols(R), K.d_modes.as<int>(), n, d_gbar, d_dtheta);
     MCMB_HIP(hipGetLastError());
     return MCMB_OK;
 }
@@ -922,6 +862,13 @@ static int project_bwd_batch(mcmb_ctx* c, const double* d_theta, int nb, const d
 // The forward cache holds every batch's stage-1 product when they fit in
 // PCACHE_BYTES together.
 constexpr size_t PCACHE_BYTES = 24ull << 30;
+
+// Host threads that move a batch's slot: starting one costs more (about 15 us)
+// than it saves below 256 KiB.
+static int transfer_threads(size_t slot_bytes)
+{
+    return (int)std::min<size_t>(std::min(8, host_threads()), 1 + slot_bytes / (256u << 10));
+}
 
 static size_t ybytes(const mcmb_ctx* c, int prec)
 {
@@ -1039,12 +986,12 @@ int mcmb_project_fwd(mcmb_ctx* c, int precision, int ntheta, const double* theta
     // move the slots on to the caller's arrays in batch order, so only the
     // last batch's transfer follows the GPU work.
     const int nout = dalpha ? 3 : 1;
-    const size_t slot_bytes = sizeof(double) * (size_t)PBATCH * n * nout;
+    const size_t slot_bytes = sizeof(double) * (size_t)std::min(PBATCH, ntheta) * n * nout;
     const int nslot = (int)std::min<size_t>(PSLOTS, 2 * STAGE_BYTES / slot_bytes);
     const char* cenv = getenv("MCMB_HOST_COPY");
     const bool staged = nslot >= 1 && !(cenv && !strcmp(cenv, "direct"));
     if (staged) MCMB_TRY(copy_stream_ready(c));
-    const int nth = std::min(8, host_threads());
+    const int nth = transfer_threads(slot_bytes);
     auto drain = [&](int bi) -> int {
         MCMB_HIP(hipEventSynchronize(c->slot_ev[1][bi % nslot]));
         const int b0 = bi * PBATCH, nb = std::min(PBATCH, ntheta - b0);
@@ -1063,7 +1010,7 @@ int mcmb_project_fwd(mcmb_ctx* c, int precision, int ntheta, const double* theta
         const int nb = std::min(PBATCH, ntheta - b0);
         DevBuf& Yb = cache ? c->ycache[bi] : c->py;
         double* d_al = dal + (size_t)b0 * n;
-        double* d_dal = ddal + (size_t)b0 * 2 * n;
+        double* d_dal = dalpha ? ddal + (size_t)b0 * 2 * n : nullptr;
         if (precision == MCMB_FP64)
             MCMB_TRY(project_fwd_batch<double>(c, dth + 2 * b0, nb, d_al, d_dal, Yb));
         else
@@ -1113,34 +1060,31 @@ int mcmb_project_bwd(mcmb_ctx* c, int precision, int ntheta, const double* theta
     PointSet& K = c->ks;
     const int n = K.n, R = K.R;
     MCMB_TRY(ensure_W(c, precision));
-    // slot[r][s][t] = mode index of the canonical triple (r,s,t) = order[m]
-    std::vector<int> slot((size_t)R * R * R, -1);
+    // a triple may be listed once only
+    std::vector<char> seen((size_t)R * R * R, 0);
     for (int m = 0; m < n; ++m) {
         int r = K.order[3 * m], s = K.order[3 * m + 1], t = K.order[3 * m + 2];
-        int& sl = slot[((size_t)r * R + s) * R + t];
-        if (sl >= 0) return fail(MCMB_ERR_ORDER, "mcmb_project_bwd: repeated mode (%d,%d,%d)", r, s, t);
-        sl = m;
+        char& sl = seen[((size_t)r * R + s) * R + t];
+        if (sl) return fail(MCMB_ERR_ORDER, "mcmb_project_bwd: repeated mode (%d,%d,%d)", r, s, t);
+        sl = 1;
     }
-    // device arrays of the call: theta [ntheta][2], gbar [ntheta][n], dtheta
-    // [ntheta][2], then the slot table
-    MCMB_TRY(c->pio.alloc(sizeof(double) * (4 + (size_t)n) * ntheta + sizeof(int) * slot.size()));
+    // device arrays of the call: theta [ntheta][2], gbar [ntheta][n], dtheta [ntheta][2]
+    MCMB_TRY(c->pio.alloc(sizeof(double) * (4 + (size_t)n) * ntheta));
     double* const dth = c->pio.as<double>();
     double* const dg = dth + 2 * (size_t)ntheta;
     double* const dd = dg + (size_t)ntheta * n;
-    int* const dslot = reinterpret_cast<int*>(dd + 2 * (size_t)ntheta);
     // the last forward's stage-1 products, when it ran on exactly these shapes
     const bool cached = c->ycache_gen == K.generation && c->ycache_prec == precision &&
                         c->ycache_theta.size() == 2 * (size_t)ntheta &&
                         !memcmp(c->ycache_theta.data(), theta, sizeof(double) * 2 * (size_t)ntheta);
     // gbar goes up batch by batch through slots of the pinned staging: host
     // threads fill slot bi % nslot while the GPU works on earlier batches
-    const size_t slot_bytes = sizeof(double) * (size_t)PBATCH * n;
+    const size_t slot_bytes = sizeof(double) * (size_t)std::min(PBATCH, ntheta) * n;
     const int nslot = (int)std::min<size_t>(PSLOTS, 2 * STAGE_BYTES / slot_bytes);
     const char* cenv = getenv("MCMB_HOST_COPY");
     const bool staged = nslot >= 1 && !(cenv && !strcmp(cenv, "direct"));
     if (staged) MCMB_TRY(copy_stream_ready(c));
-    const int nth = std::min(8, host_threads());
-    MCMB_HIP(hipMemcpyAsync(dslot, slot.data(), sizeof(int) * slot.size(), hipMemcpyHostToDevice, c->stream));
+    const int nth = transfer_threads(slot_bytes);
     MCMB_HIP(hipEventRecord(c->ev0, c->stream));
     MCMB_HIP(hipMemcpyAsync(dth, theta, sizeof(double) * 2 * (size_t)ntheta, hipMemcpyHostToDevice, c->stream));
     if (!staged)
@@ -1165,9 +1109,9 @@ int mcmb_project_bwd(mcmb_ctx* c, int precision, int ntheta, const double* theta
             MCMB_HIP(hipEventRecord(c->slot_ev[0][k], c->stream));
         }
         if (precision == MCMB_FP64)
-            MCMB_TRY(project_bwd_batch<double>(c, th, nb, gb, dslot, dt, Yc));
+            MCMB_TRY(project_bwd_batch<double>(c, th, nb, gb, dt, Yc));
         else
-            MCMB_TRY(project_bwd_batch<float>(c, th, nb, gb, dslot, dt, Yc));
+            MCMB_TRY(project_bwd_batch<float>(c, th, nb, gb, dt, Yc));
     }
     MCMB_HIP(hipMemcpyAsync(dtheta, dd, sizeof(double) * 2 * (size_t)ntheta, hipMemcpyDeviceToHost, c->stream));
     MCMB_HIP(hipEventRecord(c->ev1, c->stream));

@@ -148,3 +148,33 @@ def test_projection_transfers_over_more_batches_than_slots(ctx, monkeypatch):
         ra, rom, rph = O.project_kgl(ks["kn"], ks["kw"], ks["q"], ks["order"], th[b, 0], th[b, 1])
         assert relmax(a[b], ra) < 1e-12
         assert relmax(d[b, 0], rom) < 1e-12 and relmax(d[b, 1], rph) < 1e-12
+
+
+# (N, R, B): one basis tile filled exactly and by a single column, two tiles
+# with an odd column over, node counts at and next to the 16 nodes of a K-step
+# of the four waves, and enough (shape, node) pairs (from 4800 on) for two nodes
+# a workgroup, with an odd node left over and a last group of fewer shapes
+@pytest.mark.parametrize("N,R,B", [(16, 16, 5), (17, 1, 3), (31, 17, 9), (32, 32, 6), (161, 17, 30), (240, 5, 21)])
+@pytest.mark.parametrize("prec", [modalcmb.FP64, modalcmb.FP32])
+def test_projection_tile_edges(ctx, N, R, B, prec):
+    ks = W.kspace(N, R)
+    ctx.kspace_set(ks["kn"], ks["kw"], ks["q"], ks["order"])
+    th = W.shape_batch(B, seed=31)
+    gbar = np.random.default_rng(3).standard_normal((B, ks["order"].shape[0]))
+    a, d = ctx.project_fwd(th, prec)
+    assert np.array_equal(ctx.project_fwd(th, prec, derivatives=False), a)
+    dt = ctx.project_bwd(th, gbar, prec)
+    # the terms of sum_m gbar_m d_m, rounded once each (FP64) and summed
+    scale = np.einsum("bn,bxn->bx", np.abs(gbar), np.abs(d))
+    assert (np.abs(dt - np.einsum("bn,bxn->bx", gbar, d)) <= 1e-12 * scale).all()
+    for b in (0, B - 1):
+        # a shape alone takes one node a workgroup and gives the same bits
+        a1, d1 = ctx.project_fwd(th[b], prec)
+        assert np.array_equal(a1[0], a[b]) and np.array_equal(d1[0], d[b])
+        assert np.array_equal(ctx.project_bwd(th[b], gbar[b], prec)[0], dt[b])
+        ra, rom, rph = O.project_kgl(ks["kn"], ks["kw"], ks["q"], ks["order"], th[b, 0], th[b, 1])
+        tol = 1e-12 if prec == modalcmb.FP64 else 5e-6
+        # against the size of the terms: one mode alone (R = 1) may cancel
+        size = max(np.abs(ra).max(), np.abs(rph).max())
+        assert np.abs(a[b] - ra).max() < tol * size and np.abs(d[b, 1] - rph).max() < tol * size
+        assert np.abs(d[b, 0] - rom).max() < tol * max(np.abs(rom).max(), size)
