@@ -143,6 +143,24 @@ def test_gamma_gl_compressed_equals_direct_node_sum(ctx, L, R, mod):
     assert np.array_equal(G, ctx.gamma_gl())
 
 
+# rows of the pair products at the most that a factorisation step's 256 threads
+# hold, just past it (1024 threads), an odd count, and the most that can be set
+@pytest.mark.parametrize("L", [37, 3071, 3072, 8190])
+def test_pair_basis_factorisation_rows(ctx, L):
+    R = 7   # the smallest whose rank 2R - 1 is at most half the pairs
+    ws = W.lspace(L, R, False)
+    ctx.lspace_set(2, L, ws["q"], ws["v"], ws["order"])
+    G = ctx.gamma_gl()
+    assert ctx.last_basis_rank() == 2 * R - 1
+    os.environ["MCMB_GL_PATH"] = "direct"
+    try:
+        Gd = ctx.gamma_gl()
+    finally:
+        del os.environ["MCMB_GL_PATH"]
+    # as above; the node sum's cancellation, and with it both roundings, grows as lmax^2
+    assert rel_elem(G, Gd) < 1e-13 * max(1.0, L / 2500) ** 2
+
+
 def test_gamma_gl_full_rank_basis_takes_direct_node_sum(ctx):
     """A random basis has full-rank pair products: no compressed basis, and
     the GL Gram is the direct node sum bit for bit."""
