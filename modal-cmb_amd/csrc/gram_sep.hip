@@ -41,6 +41,14 @@ typedef double fd2 __attribute__((ext_vector_type(2)));
 constexpr int SG_FM = 5, SG_FN = 3;   // 16 x 16 blocks per wave (rows, columns); 2 x 2 waves
 constexpr int SG_TM = 32 * SG_FM;     // GEMM tile rows (160)
 constexpr int SG_TN = 32 * SG_FN;     // GEMM tile columns (96)
+// The same of the expansion's products: their K is one compressed rank (4 to
+// 60), so a tile is mostly its first loads and its stores, and what counts is
+// tiles enough for the chip, several of them on a CU, and little cut off at the
+// triangles.  At 59 functions and 465 pairs 64 x 64 takes 122 us in all, 160 x
+// 96 (the contractions') 165, 128 x 64 147, 96 x 96 137, 128 x 128 155; at 23
+// and 78, 16 against 29.
+constexpr int EX_FM = 2, EX_FN = 2;
+constexpr int EX_TM = 32 * EX_FM, EX_TN = 32 * EX_FN;
 constexpr int SG_SMALL = 64;          // basis widths up to this use 64 x 64 tiles (2 x 2 blocks per wave)
 constexpr int SG_KC = 16;             // K rows per LDS stage
 constexpr int SG_KSPLIT = 16;         // K splits of the l1 contraction over a compressed basis
@@ -609,19 +617,19 @@ __global__ __launch_bounds__(64 * NW, (NW == 1 && CPW == 4) ? 3 : 2) void sep_ro
 }
 
 // Stages 2 and 3:  C_task[m][n] (+)= sum_{kk < K} U[row(kk)][m] * B[boff + kk][n]
-// for m < Md, n < Nd, over a list of 160 x 96 tiles (task, m0, n0); row(kk) =
+// for m < Md, n < Nd, over a list of tiles (task, m0, n0); row(kk) =
 // aoff + kk when the A rows are contiguous (CONTIG), else aidx[aoff + kk].
 // Both operands are K-major with even leading dimensions (16-byte loads; the
 // element past an odd Md or Nd is padding and only feeds outputs that are not
 // stored).  16 K rows per stage, double-buffered in LDS; FP64 MFMA 16x16x4
-// with 4 waves of 80 x 48.  The tile list holds groups of GS consecutive
+// with 4 waves, 2 x 2 over the tile.  The tile list holds groups of GS consecutive
 // tiles that share one B panel (the m tiles of one (task, n0)).  Blocks b,
 // b+8, ... share an XCD (and its L2): the groups are dealt to the 8 XCDs in
 // turn, each group's tiles to consecutive blocks of one XCD, so the tiles of
 // a group meet in the same L2 and the XCDs get alike shares of the work.
 // STAGE (2: l2, 3: l1, 4: expansion) only names the launches apart in
 // profiles.  FM x FN: 16 x 16 blocks per wave (5 x 3: 160 x 96 tiles; 2 x 2:
-// 64 x 64 tiles for narrow bases).  PAIRS: C is symmetric (Md = Nd) and only
+// 64 x 64 tiles for narrow bases and the expansion).  PAIRS: C is symmetric (Md = Nd) and only
 // its upper triangle is stored, at C + coff + pair_index(m, n, Md).
 template <bool CONTIG, int STAGE, int FM = SG_FM, int FN = SG_FN, bool PAIRS = false>
 __global__ __launch_bounds__(256, 2) void sep_gemm(const double* __restrict__ U, int ldu,
@@ -1885,27 +1893,27 @@ static int separable_compress(mcmb_ctx* c, SepComp& S, const BasisRef& Bq, int n
         std::vector<SepTask> t1(1), t2(r), t3(1);
         std::vector<int4> g1, g2, g3;
         t1[0] = SepTask{0, 0, 0, r};
-        for (int n0c = 0; n0c < NP; n0c += SG_TN)
-            for (int m0 = 0; m0 < r * r; m0 += SG_TM) g1.push_back(make_int4(0, m0, n0c, 0));
+        for (int n0c = 0; n0c < NP; n0c += EX_TN)
+            for (int m0 = 0; m0 < r * r; m0 += EX_TM) g1.push_back(make_int4(0, m0, n0c, 0));
         // Y2[a] is symmetric (H is): its upper triangle goes straight to pair
         // order, and tiles wholly below the diagonal are skipped
         const long ldp = NPP + (NPP & 1);
         for (int a = 0; a < r; ++a) {
             t2[a] = SepTask{(long)a * r, (long)a * ldp, 0, r};
-            for (int n0c = 0; n0c < NP; n0c += SG_TN)
-                for (int m0 = 0; m0 < NP && m0 < n0c + SG_TN; m0 += SG_TM) g2.push_back(make_int4(a, m0, n0c, 0));
+            for (int n0c = 0; n0c < NP; n0c += EX_TN)
+                for (int m0 = 0; m0 < NP && m0 < n0c + EX_TN; m0 += EX_TM) g2.push_back(make_int4(a, m0, n0c, 0));
         }
         // G[x][{y,z}] only where x <= y (the assembly reads sorted triples):
         // tiles whose rows all lie above the pair columns' last y are skipped
         t3[0] = SepTask{0, 0, 0, r};
-        std::vector<int> ylast((NPP + SG_TN - 1) / SG_TN);
+        std::vector<int> ylast((NPP + EX_TN - 1) / EX_TN);
         for (int y = 0; y < NP; ++y)
             for (int z = y; z < NP; ++z) {
                 const long pidx = pair_index(y, z, NP);
-                ylast[pidx / SG_TN] = y;
+                ylast[pidx / EX_TN] = y;
             }
-        for (long n0c = 0; n0c < NPP; n0c += SG_TN)
-            for (int m0 = 0; m0 < NP && m0 <= ylast[n0c / SG_TN]; m0 += SG_TM)
+        for (long n0c = 0; n0c < NPP; n0c += EX_TN)
+            for (int m0 = 0; m0 < NP && m0 <= ylast[n0c / EX_TN]; m0 += EX_TM)
                 g3.push_back(make_int4(0, m0, (int)n0c, 0));
         std::vector<int> buf;
         S.o_task[0] = append(buf, t1);
@@ -1917,8 +1925,8 @@ static int separable_compress(mcmb_ctx* c, SepComp& S, const BasisRef& Bq, int n
         S.nt[0] = (int)g1.size();
         S.nt[1] = (int)g2.size();
         S.nt[2] = (int)g3.size();
-        S.gs[0] = (r * r + SG_TM - 1) / SG_TM;
-        S.gs[1] = S.gs[2] = (NP + SG_TM - 1) / SG_TM;
+        S.gs[0] = (r * r + EX_TM - 1) / EX_TM;
+        S.gs[1] = S.gs[2] = (NP + EX_TM - 1) / EX_TM;
         MCMB_TRY(S.tab.alloc(sizeof(int) * buf.size()));
         MCMB_HIP(hipMemcpy(S.tab.p, buf.data(), sizeof(int) * buf.size(), hipMemcpyHostToDevice));
         MCMB_TRY(S.h.alloc(sizeof(double) * (size_t)r * ldh));
@@ -1969,15 +1977,15 @@ static int sep_expand(mcmb_ctx* c, const SepComp& S, int NP, int ld)
     const double* const Ct = S.ct.as<double>();
     double *const T1 = c->sg_M.as<double>(), *const Y2s = c->sg_Ys.as<double>(), *const G = c->sg_G.as<double>();
     for (int k = 0; k < 3; ++k) MCMB_TRY(launch_guard("expansion", sep_blocks(S.nt[k], S.gs[k]), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(S.nt[0], S.gs[0])), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((sep_gemm<true, 4, EX_FM, EX_FN>), dim3(sep_blocks(S.nt[0], S.gs[0])), dim3(256), 0, c->stream,
                        (const double*)S.h.as<double>(), (int)ldh, tb, Ct, (long)ld, T1, (long)ld, r * r, NP,
                        reinterpret_cast<const SepTask*>(tb + S.o_task[0]),
                        reinterpret_cast<const int4*>(tb + S.o_tile[0]), S.nt[0], S.gs[0], 0);
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN, true>), dim3(sep_blocks(S.nt[1], S.gs[1])), dim3(256), 0,
+    hipLaunchKernelGGL((sep_gemm<true, 4, EX_FM, EX_FN, true>), dim3(sep_blocks(S.nt[1], S.gs[1])), dim3(256), 0,
                        c->stream, Ct, ld, tb, (const double*)T1, (long)ld, Y2s, ldp, NP, NP,
                        reinterpret_cast<const SepTask*>(tb + S.o_task[1]),
                        reinterpret_cast<const int4*>(tb + S.o_tile[1]), S.nt[1], S.gs[1], 0);
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(S.nt[2], S.gs[2])), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((sep_gemm<true, 4, EX_FM, EX_FN>), dim3(sep_blocks(S.nt[2], S.gs[2])), dim3(256), 0, c->stream,
                        Ct, ld, tb, (const double*)Y2s, (long)ldp, G, (long)ldp, NP, (int)NPP,
                        reinterpret_cast<const SepTask*>(tb + S.o_task[2]),
                        reinterpret_cast<const int4*>(tb + S.o_tile[2]), S.nt[2], S.gs[2], 0);
@@ -2162,16 +2170,16 @@ int gram_gl_mixed_compressed(mcmb_ctx* c, int pol, int RT, int RE, int npt, cons
     std::vector<SepTask> t1(1), t2(rS), t3(1);
     std::vector<int4> g1, g2, g3;
     t1[0] = SepTask{0, 0, 0, rP};
-    for (int n0 = 0; n0 < NPP_; n0 += SG_TN)
-        for (int m0 = 0; m0 < rS * rP; m0 += SG_TM) g1.push_back(make_int4(0, m0, n0, 0));
+    for (int n0 = 0; n0 < NPP_; n0 += EX_TN)
+        for (int m0 = 0; m0 < rS * rP; m0 += EX_TM) g1.push_back(make_int4(0, m0, n0, 0));
     for (int g = 0; g < rS; ++g) {
         t2[g] = SepTask{(long)g * rP, (long)g * ldq, 0, rP};
-        for (int n0 = 0; n0 < NPP_; n0 += SG_TN)
-            for (int m0 = 0; m0 < NPP_ && m0 < n0 + SG_TN; m0 += SG_TM) g2.push_back(make_int4(g, m0, n0, 0));
+        for (int n0 = 0; n0 < NPP_; n0 += EX_TN)
+            for (int m0 = 0; m0 < NPP_ && m0 < n0 + EX_TN; m0 += EX_TM) g2.push_back(make_int4(g, m0, n0, 0));
     }
     t3[0] = SepTask{0, 0, 0, rS};
-    for (long n0 = 0; n0 < NQ; n0 += SG_TN)
-        for (int m0 = 0; m0 < NPS; m0 += SG_TM) g3.push_back(make_int4(0, m0, (int)n0, 0));
+    for (long n0 = 0; n0 < NQ; n0 += EX_TN)
+        for (int m0 = 0; m0 < NPS; m0 += EX_TM) g3.push_back(make_int4(0, m0, (int)n0, 0));
     std::vector<int> buf;
     const size_t ot1 = append(buf, t1), og1 = append(buf, g1), ot2 = append(buf, t2), og2 = append(buf, g2),
                  ot3 = append(buf, t3), og3 = append(buf, g3);
@@ -2187,20 +2195,20 @@ int gram_gl_mixed_compressed(mcmb_ctx* c, int pol, int RT, int RE, int npt, cons
     double* const T1 = c->sg_M.as<double>();
     double* const Y = c->sg_Ys.as<double>();
     double* const K = c->sg_G.as<double>();
-    const int gs1 = (rS * rP + SG_TM - 1) / SG_TM, gs2 = (NPP_ + SG_TM - 1) / SG_TM, gs3 = (NPS + SG_TM - 1) / SG_TM;
+    const int gs1 = (rS * rP + EX_TM - 1) / EX_TM, gs2 = (NPP_ + EX_TM - 1) / EX_TM, gs3 = (NPS + EX_TM - 1) / EX_TM;
     const int nt1 = (int)g1.size(), nt2 = (int)g2.size(), nt3 = (int)g3.size();
     MCMB_TRY(launch_guard("GL expansion", sep_blocks(nt1, gs1), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(nt1, gs1)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((sep_gemm<true, 4, EX_FM, EX_FN>), dim3(sep_blocks(nt1, gs1)), dim3(256), 0, c->stream,
                        (const double*)H, (int)ldh, tb, (const double*)SP.ct.as<double>(), (long)ldP, T1, (long)ldP,
                        rS * rP, NPP_, reinterpret_cast<const SepTask*>(tb + ot1),
                        reinterpret_cast<const int4*>(tb + og1), nt1, gs1, 0);
     MCMB_TRY(launch_guard("GL expansion", sep_blocks(nt2, gs2), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN, true>), dim3(sep_blocks(nt2, gs2)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((sep_gemm<true, 4, EX_FM, EX_FN, true>), dim3(sep_blocks(nt2, gs2)), dim3(256), 0, c->stream,
                        (const double*)SP.ct.as<double>(), ldP, tb, (const double*)T1, (long)ldP, Y, ldq, NPP_, NPP_,
                        reinterpret_cast<const SepTask*>(tb + ot2), reinterpret_cast<const int4*>(tb + og2), nt2, gs2,
                        0);
     MCMB_TRY(launch_guard("GL expansion", sep_blocks(nt3, gs3), 256));
-    hipLaunchKernelGGL((sep_gemm<true, 4, SG_FM, SG_FN>), dim3(sep_blocks(nt3, gs3)), dim3(256), 0, c->stream,
+    hipLaunchKernelGGL((sep_gemm<true, 4, EX_FM, EX_FN>), dim3(sep_blocks(nt3, gs3)), dim3(256), 0, c->stream,
                        (const double*)SS.ct.as<double>(), ldS, tb, (const double*)Y, (long)ldq, K, (long)ldq, NPS,
                        (int)NQ, reinterpret_cast<const SepTask*>(tb + ot3), reinterpret_cast<const int4*>(tb + og3),
                        nt3, gs3, 0);
