@@ -17,7 +17,7 @@
 // of the rounded T.  gl_gate bounds the error for the weights at hand, and a
 // setup it does not pass takes the tetrapyd contraction.  Measured, core
 // tensor by the tetrapyd contraction -> as a node sum: lmax 2500, r = 59: 2.20
-// -> 0.29 ms; lmax 2000, r = 39: 1.22 -> 0.11 ms.
+// -> 0.20 ms; lmax 2000, r = 39: 1.22 -> 0.07 ms.
 //
 // Both parities of l are summed apart (P_l(-x) = (-1)^l P_l(x)), so the table
 // holds the nodes x >= 0 only, and the columns at +x and -x are E + O and
@@ -132,9 +132,11 @@ __global__ __launch_bounds__(64) void gl_ptab(int lmax, int half, int SH, const 
 
 // T[l][a] = (2l + 1) v_l P[l][a] for a < r, and the gate's column a = r, (2l +
 // 1) |v_l| max_a |P[l][a]|; 0 for lmin > l and for r < a < ldt.  One workgroup
-// per 32 l (Pc is stored by columns, T by rows).
+// per 32 l (Pc is stored by columns, T by rows), which leaves the sum of its
+// part of the gate's column in Sp (if given).
 __global__ __launch_bounds__(256) void gl_ttab(const double* __restrict__ Pc, int nlp, int nl, int r, int lmin,
-                                               const double* __restrict__ v, int ldt, double* __restrict__ T)
+                                               const double* __restrict__ v, int ldt, double* __restrict__ T,
+                                               double* __restrict__ Sp)
 {
     __shared__ double S[GN_RMAX + 1][33];
     const int l0 = blockIdx.x * 32, tl = threadIdx.x & 31;
@@ -144,6 +146,10 @@ __global__ __launch_bounds__(256) void gl_ttab(const double* __restrict__ Pc, in
         double m = 0.0;
         for (int a = 0; a < r; ++a) m = fmax(m, fabs(S[a][tl]));
         S[r][tl] = m;
+        const int l = l0 + tl;
+        double g = l < nl && l >= lmin ? m * fabs((2.0 * l + 1.0) * v[l]) : 0.0;
+        for (int o = 16; o >= 1; o >>= 1) g += __shfl_xor(g, o);
+        if (Sp && tl == 0) Sp[blockIdx.x] = g;
     }
     __syncthreads();
     for (int e = threadIdx.x; e < 32 * ldt; e += 256) {
@@ -154,18 +160,27 @@ __global__ __launch_bounds__(256) void gl_ttab(const double* __restrict__ Pc, in
     }
 }
 
+// S = sum_l T[l][r] from gl_ttab's parts, alike in every lane of every wave:
+// no column's sum of |T[l][a] P_l| exceeds it (|P_l| <= 1).
+__device__ __forceinline__ double gl_sbound(const double* __restrict__ Sp, int nsp, int lane)
+{
+    double s = 0.0;
+    for (int b = lane; b < nsp; b += 64) s += Sp[b];
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
+    return s;
+}
+
 // Phi[a][k] for CA columns from a0 on at 64 nodes: k = s is +x_s, k = SH + s
 // is -x_s.  16 waves: waves 0..7 take the even l, 8..15 the odd ones, l =
 // parity + 2 wave' + 16 i, and their sums are added pairwise in LDS in a fixed
-// order.  Lane = node; the T row is uniform (scalar loads).  11 FP64 operations
-// per (l, node, column), so it is bound by FP64 issue: 0.157 ms at 2501 l,
-// 1876 nodes, 60 columns is 20e12 operations/s, where a loop of additions or
-// fused multiply-adds alone reaches 29e12 to 32e12 on this card.  CA columns
-// share a P load.
+// order.  Lane = node; the T row is uniform (scalar loads).  5 FP64 operations
+// per (l, node, column): at 2501 l, 1876 nodes, 60 columns 0.101 ms, 0.157
+// with the 11 of an error-free running sum.  CA columns share a P load.
 constexpr int GN_W = 16;
 template <int CA>
 __global__ __launch_bounds__(64 * GN_W) void gl_phi(const dd* __restrict__ P, int SH, const double* __restrict__ T,
-                                                    int ldt, int nl, int nc, dd* __restrict__ Phi)
+                                                    int ldt, int nl, int nc, const double* __restrict__ Sp, int nsp,
+                                                    dd* __restrict__ Phi)
 {
     __shared__ dd R[GN_W / 2][CA][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -177,19 +192,20 @@ __global__ __launch_bounds__(64 * GN_W) void gl_phi(const dd* __restrict__ P, in
     if (64 * nb >= SH) return;
     const int s = 64 * nb + lane;
     const int par = wave >> 3, ww = wave & 7;
+    const double B = dd_bias(gl_sbound(Sp, nsp, lane));
     dd acc[CA];
 #pragma unroll
-    for (int k = 0; k < CA; ++k) acc[k] = dd{0.0, 0.0};
+    for (int k = 0; k < CA; ++k) acc[k] = dd{B, 0.0};
     const dd* const p = P + s;
 #pragma unroll 4
     for (int l = par + 2 * ww; l < nl; l += GN_W) {
         const dd pl = p[(long)l * SH];
         const double* const t = T + (long)l * ldt + a0;
 #pragma unroll
-        for (int k = 0; k < CA; ++k) dd_mac(acc[k], t[k], pl);
+        for (int k = 0; k < CA; ++k) dd_bmac(acc[k], t[k], pl);
     }
 #pragma unroll
-    for (int k = 0; k < CA; ++k) acc[k] = dd_renorm(acc[k]);
+    for (int k = 0; k < CA; ++k) acc[k] = dd_unbias(acc[k], B);
     // 8 -> 4 -> 2 -> 1 waves per parity
 #pragma unroll
     for (int h = 4; h >= 1; h >>= 1) {
@@ -238,9 +254,10 @@ __device__ __forceinline__ dd wave_totals(dd (&acc)[32], int lane)
 // One workgroup per job: a in a tile of four columns ta, two b of tile tb >=
 // ta, c in tile tc >= tb (a <= b <= c covers every entry; the entry is written
 // at all its orders).  Wave q takes a quarter of the 64-node steps, lane =
-// node: per step 10 columns are read for 32 products (12 operations each plus
-// the pair products: FP64 issue bounds it, the reads come from L2).  The last
-// workgroup forms the gate's two sums.
+// node: per step 10 columns are read for 32 products (6 operations each plus
+// the pair products; the reads come from L2): 0.088 ms at 3752 nodes and 59
+// columns, 0.120 with 12 operations each.  The last workgroup forms the gate's
+// two sums.
 __device__ __forceinline__ void core_job(int job, int NT, int* ta, int* tb, int* tc, int* h)
 {
     int t = 0;
@@ -254,44 +271,39 @@ __device__ __forceinline__ void core_job(int job, int NT, int* ta, int* tb, int*
 
 __global__ __launch_bounds__(256, 2) void gl_core_dd(const dd* __restrict__ Phi, int SH, const dd* __restrict__ w,
                                                      int r, double scale, double* __restrict__ H, long ldh, int njobs,
-                                                     const double* __restrict__ T, int ldt, int nl,
+                                                     const double* __restrict__ Sp, int nsp,
                                                      double* __restrict__ gate)
 {
     __shared__ dd R[4][32];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, K = 2 * SH;
+    const double S = gl_sbound(Sp, nsp, lane);
     if (blockIdx.x == (unsigned)njobs) {
-        // gate[0] = sum_k w_k Phi_r^3, gate[1] = sum_l T[l][r]; H's padding
+        // gate[0] = sum_k w_k Phi_r^3, gate[1] = S; H's padding
         // (r^2 odd) is zeroed
         if (ldh > (long)r * r)
             for (int g = threadIdx.x; g < r; g += 256) H[(long)g * ldh + (long)r * r] = 0.0;
         dd A{0.0, 0.0};
-        double S = 0.0;
         for (int k = threadIdx.x; k < K; k += 256) {
             const dd f = Phi[(long)r * K + k];
             A = A + w[k < SH ? k : k - SH] * f * (f * f);
         }
-        for (int l = threadIdx.x; l < nl; l += 256) S += T[(long)l * ldt + r];
-        for (int o = 32; o >= 1; o >>= 1) {
-            A = A + dd_shfl_xor(A, o);
-            S += __shfl_xor(S, o);
-        }
-        if (lane == 0) {
-            R[wave][0] = A;
-            R[wave][1].hi = S;
-        }
+        for (int o = 32; o >= 1; o >>= 1) A = A + dd_shfl_xor(A, o);
+        if (lane == 0) R[wave][0] = A;
         __syncthreads();
         if (threadIdx.x == 0) {
             const dd a = (R[0][0] + R[1][0]) + (R[2][0] + R[3][0]);
             gate[0] = a.hi + a.lo;
-            gate[1] = (R[0][1].hi + R[1][1].hi) + (R[2][1].hi + R[3][1].hi);
+            gate[1] = S;
         }
         return;
     }
     int ta, tb, tc, h;
     core_job(blockIdx.x, (r + 3) / 4, &ta, &tb, &tc, &h);
+    // |Phi| <= S and sum w = 2
+    const double B = dd_bias(2.0 * S * S * S);
     dd acc[32];
 #pragma unroll
-    for (int i = 0; i < 32; ++i) acc[i] = dd{0.0, 0.0};
+    for (int i = 0; i < 32; ++i) acc[i] = dd{B, 0.0};
     // columns past r repeat the last one (their products are not stored);
     // uniform row bases and one lane offset, the next step's columns loaded
     // before this step's products
@@ -333,13 +345,13 @@ __global__ __launch_bounds__(256, 2) void gl_core_dd(const dd* __restrict__ Phi,
             for (int i = 0; i < 4; ++i) {
                 const dd t = u * cur.a[i];
 #pragma unroll
-                for (int q = 0; q < 4; ++q) dd_mac(acc[16 * j + 4 * i + q], t, cur.c[q]);
+                for (int q = 0; q < 4; ++q) dd_bmac(acc[16 * j + 4 * i + q], t, cur.c[q]);
             }
         }
         cur = nxt;
     }
 #pragma unroll
-    for (int i = 0; i < 32; ++i) acc[i] = dd_renorm(acc[i]);
+    for (int i = 0; i < 32; ++i) acc[i] = dd_unbias(acc[i], B);
     const dd tot = wave_totals(acc, lane);
     if (!(lane & 1)) R[wave][lane >> 1] = tot;
     __syncthreads();
@@ -384,7 +396,7 @@ int gl_table(mcmb_ctx* c, int npt, int lmax)
 
 // Whether the node form takes this setup's whole Gram (see the header comment;
 // the gate is checked after the sums).  Below GN_LMIN the tetrapyd contraction
-// stays the default: it takes 0.17 ms there, most of it launches, and its
+// stays the default: it takes 0.16 ms there, most of it launches, and its
 // results are the same bits for all its kernel variants.  Above GN_TABMAX the
 // table of P_l would be kept at the expense of the caller's memory.
 bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool any_lmax)
@@ -411,15 +423,19 @@ int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, i
     const int nbx = G.SH / 64;
     while (ca > 2 && nbx * ((nc + ca - 1) / ca) < 200) ca >>= 1;
     const int ldt = (nc + 7) & ~7;
-    MCMB_TRY(c->gn_ws.alloc(sizeof(dd) * (size_t)nc * K + sizeof(double) * (size_t)nl * ldt));
+    const int nsp = (nl + 31) / 32;
+    MCMB_TRY(c->gn_ws.alloc(sizeof(dd) * (size_t)nc * K + sizeof(double) * ((size_t)nl * ldt + nsp)));
     dd* const Phi = c->gn_ws.as<dd>();
     double* const T = reinterpret_cast<double*>(Phi + (size_t)nc * K);
+    double* const Sp = T + (size_t)nl * ldt;
     if (!c->gn_gate) MCMB_HIP(hipHostMalloc((void**)&c->gn_gate, 2 * sizeof(double), hipHostMallocDefault));
     MCMB_TRY(phase("basis at the nodes"));
     hipLaunchKernelGGL(gl_ttab, dim3((nl + 31) / 32), dim3(256), 0, c->stream, Pc, nlp, nl, r, L.lmin,
-                       (const double*)L.d_v.as<double>(), ldt, T);
+                       (const double*)L.d_v.as<double>(), ldt, T, Sp);
     const dim3 grid(8 * ((nbx + 7) / 8) * ((nc + ca - 1) / ca)), block(64 * GN_W);
-#define GN_PHI(CA) hipLaunchKernelGGL(gl_phi<CA>, grid, block, 0, c->stream, (const dd*)G.P, G.SH, (const double*)T, ldt, nl, nc, Phi)
+#define GN_PHI(CA)                                                                                                       \
+    hipLaunchKernelGGL(gl_phi<CA>, grid, block, 0, c->stream, (const dd*)G.P, G.SH, (const double*)T, ldt, nl, nc, \
+                       (const double*)Sp, nsp, Phi)
     if (ca == 8) GN_PHI(8);
     else if (ca == 4) GN_PHI(4);
     else GN_PHI(2);
@@ -430,7 +446,7 @@ int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, i
     int njobs = 0;
     for (int t = 0; t < NT; ++t) njobs += 2 * (t + 1) * (NT - t);
     hipLaunchKernelGGL(gl_core_dd, dim3(njobs + 1), dim3(256), 0, c->stream, (const dd*)Phi, G.SH, (const dd*)G.w, r,
-                       3.0 / (4.0 * M_PI), H, ldh, njobs, (const double*)T, ldt, nl, c->gn_gate);
+                       3.0 / (4.0 * M_PI), H, ldh, njobs, (const double*)Sp, nsp, c->gn_gate);
     MCMB_HIP(hipGetLastError());
     return MCMB_OK;
 }
@@ -440,11 +456,16 @@ int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, i
 // sum w Phi_m^3 formed with absolute values, at most 2 S^3 (|P_l| <= 1, sum w
 // = 2); A = sum w Phi_m^3 is the tetrapyd sum of the same bound over the
 // allowed terms, the scale of H that FP64 resolves to 2^-53.  Each term
-// carries about 2^-104 times a growth of the recurrence linear in l.
+// carries about 2^-104 times a growth of the recurrence linear in l, and the
+// biased sums of Phi and of H each add 2^-104 of their bound (at most 4 S, 8
+// S^3 and so 4 times the terms') a term: 2^-101 covers them.  (The workloads'
+// spectra pass with 3 decades to spare at lmax 2500, 5 at 520.)
 bool gl_gate(const mcmb_ctx* c, int lmax)
 {
-    const double A = c->gn_gate[0], S = c->gn_gate[1];
-    return 2.0 * S * S * S * 0x1p-104 * (lmax + 64.0) <= 0x1p-54 * A;
+    const double A = c->gn_gate[0], S = c->gn_gate[1], b = 2.0 * S * S * S;
+    // (within reach of overflow or of subnormal rests the bias does not hold)
+    if (S != 0.0 && !(b > 1e-250 && b < 1e300)) return false;
+    return b * 0x1p-101 * (lmax + 64.0) <= 0x1p-54 * A;
 }
 
 // ---- the FP64 node sum (mcmb_gamma_gl, mcmb_gamma_gl_pol) over compressed bases ----
@@ -604,7 +625,8 @@ int gl_phi64_launch(mcmb_ctx* c, const double* Pc, int nlp, int nl, int r, int l
     const GlHalf& G = c->glh;
     const int ldt = gl_ldt(r);
     *phi = ws + (size_t)nl * ldt;
-    hipLaunchKernelGGL(gl_ttab, dim3((nl + 31) / 32), dim3(256), 0, c->stream, Pc, nlp, nl, r, lmin, v, ldt, ws);
+    hipLaunchKernelGGL(gl_ttab, dim3((nl + 31) / 32), dim3(256), 0, c->stream, Pc, nlp, nl, r, lmin, v, ldt, ws,
+                       (double*)nullptr);
     hipLaunchKernelGGL(gl_phi64, dim3(G.SH / 16), dim3(1024), 0, c->stream, (const double*)G.P, G.SH, (const double*)ws,
                        ldt, nl, r, *phi);
     MCMB_HIP(hipGetLastError());

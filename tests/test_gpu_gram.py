@@ -613,6 +613,28 @@ def test_node_form_gate(ctx):
     assert "node sum" in [p for p, _ in ctx.last_phases()]
 
 
+# The node form's sums carry a bias of a power of two above sum |T|: scales at
+# and next to a power (v times 2^k only moves the exponents, so Gamma is 2^3k
+# times the same bits), and far from one; scales at which the cube nears the
+# ends of the exponent range take the tetrapyd contraction
+def test_node_form_scales(ctx):
+    L, R = 600, 8
+    ws = W.lspace(L, R)
+    ctx.lspace_set(2, L, ws["q"], ws["v"], ws["order"])
+    G = ctx.gamma_tet(modalcmb.FP64)
+    for k in (-200, -1, 1, 2, 150):
+        ctx.lspace_set(2, L, ws["q"], ws["v"] * 2.0**k, ws["order"])
+        assert np.array_equal(ctx.gamma_tet(modalcmb.FP64), np.ldexp(G, 3 * k))
+        assert "node sum" in [p for p, _ in ctx.last_phases()]
+    ctx.lspace_set(2, L, ws["q"], ws["v"] * 1.37, ws["order"])
+    assert rel_elem(ctx.gamma_tet(modalcmb.FP64), G * 1.37**3) < 1e-13
+    for k in (-330, 330):
+        ctx.lspace_set(2, L, ws["q"], ws["v"] * 2.0**k, ws["order"])
+        D = ctx.gamma_tet(modalcmb.FP64)
+        assert "node sum" not in [p for p, _ in ctx.last_phases()]
+        assert np.array_equal(D, _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"], equal_nan=True)
+
+
 def test_separable_device_row_groups_equal_host_lmax2500(ctx):
     """As test_separable_device_row_groups_equal_host at a size where the
     default is the node form, which reads no row groups: the tetrapyd
