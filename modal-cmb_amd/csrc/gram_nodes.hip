@@ -475,7 +475,8 @@ bool gl_gate(const mcmb_ctx* c, int lmax)
 // on (npt, lmax) alone and is kept with the context; Phi is then a GEMM on the
 // matrix cores instead of a recurrence per column group (lmax 2000, r = 39:
 // 0.356 -> 0.035 ms, bound by its loads' latency: 94 workgroups), and the core
-// tensor is cx_core's (0.072 -> 0.038 ms with gl_hsum).
+// tensor is cx_core's (0.072 -> 0.030 ms with gl_hsum, whose sums over the units
+// wait for memory once per 16 of them).
 
 // P[l][s] = P_l(x_s) by the three-term recurrence of the direct node sum, l <=
 // lmax; 0 past half.  One thread per node, a serial chain.
@@ -555,14 +556,14 @@ __global__ __launch_bounds__(1024) void gl_phi64(const double* __restrict__ P, i
 // The core H from the units' tile tensors (cx_core), added in order: H[g][a r
 // + b] of one field, or H[b][g rP + a] with (a, b) of the pair's field.
 template <bool SAME>
-__global__ __launch_bounds__(256) void gl_hsum(const double* __restrict__ Hu, long us, int nu, int rP, int rS,
+__global__ __launch_bounds__(64) void gl_hsum(const double* __restrict__ Hu, long us, int nu, int rP, int rS,
                                                double scale, double* __restrict__ H, long ldh)
 {
     __shared__ long base[8];
     const int NTC = (rS + 15) >> 4, NTB = (rP + 15) >> 4;
     if (threadIdx.x < NTB) base[threadIdx.x] = cx_base(threadIdx.x, NTC, SAME);
     __syncthreads();
-    const long e = (long)blockIdx.x * 256 + threadIdx.x;
+    const long e = (long)blockIdx.x * 64 + threadIdx.x;
     if (e >= (long)rP * ldh) return;
     const int x = (int)(e / ldh), rem = (int)(e % ldh), y = rem / rP, z = rem % rP;
     if (rem >= (SAME ? rP : rS) * rP) {
@@ -581,7 +582,13 @@ __global__ __launch_bounds__(256) void gl_hsum(const double* __restrict__ Hu, lo
     }
     const double* const h = Hu + cx_tile(base[b >> 4], a >> 4, b, c >> 4, NTC, SAME) * 256 + 16 * (a & 15) + (c & 15);
     double t = 0.0;
-    for (int u = 0; u < nu; ++u) t += h[(long)u * us];
+    for (int u0 = 0; u0 < nu; u0 += 16) {   // 16 loads in flight, added in order
+        double v[16];
+#pragma unroll
+        for (int k = 0; k < 16; ++k) v[k] = u0 + k < nu ? h[(long)(u0 + k) * us] : 0.0;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) t += v[k];
+    }
     H[e] = scale * t;
 }
 
@@ -662,12 +669,12 @@ int gl_core64_launch(mcmb_ctx* c, const double* phP, int rP, const double* phS, 
     int g, ng;
     gl_units(c, rP, rS, same, &jobs, &g, &ng, &us);
     const int nch = 2 * c->glh.SH / 64;
-    const dim3 grid((unsigned)jobs, ng), hgrid((unsigned)(((long)rP * ldh + 255) / 256));
+    const dim3 grid((unsigned)jobs, ng), hgrid((unsigned)(((long)rP * ldh + 63) / 64));
 #define GL_CORE64(SAME)                                                                                          \
     do {                                                                                                         \
         hipLaunchKernelGGL(cx_core<SAME>, grid, dim3(256), 0, c->stream, phP, rP, phS, rS, 64,                   \
                            (const double*)c->glh.w, 64l, (const double*)nullptr, 0, ng, g, nch, 0, ws, us);      \
-        hipLaunchKernelGGL(gl_hsum<SAME>, hgrid, dim3(256), 0, c->stream, (const double*)ws, us, ng, rP, rS, scale, H, \
+        hipLaunchKernelGGL(gl_hsum<SAME>, hgrid, dim3(64), 0, c->stream, (const double*)ws, us, ng, rP, rS, scale, H, \
                            ldh);                                                                                 \
     } while (0)
     if (same) GL_CORE64(true);

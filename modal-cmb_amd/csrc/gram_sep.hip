@@ -997,8 +997,9 @@ __global__ void sep_ptab(const double* __restrict__ Pc, int nlp, int nl, int r, 
 // G2[y][{x,z}] + G2[z][{x,y}] (x <= y <= z, pairs over r), each G2 entry the
 // sum of the ns partial sums G2 + s lds in order of s: every entry of the
 // fully symmetrised tensor over the compressed basis, equal for all orders of
-// (g, a, b); the padding entry of each row (r^2 odd) is zeroed.
-__global__ void sep_hfull(const double* __restrict__ G2, long ldg, long lds, int ns, int r, double* __restrict__ H,
+// (g, a, b); the padding entry of each row (r^2 odd) is zeroed.  Bound by the
+// latency of its loads (19 columns: 15.8 us with one at a time, 4.2; 39 columns 17.3, 10.9).
+__global__ __launch_bounds__(64) void sep_hfull(const double* __restrict__ G2, long ldg, long lds, int ns, int r, double* __restrict__ H,
                           long ldh)
 {
     const long e = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -1011,12 +1012,21 @@ __global__ void sep_hfull(const double* __restrict__ G2, long ldg, long lds, int
     }
     const int a = (int)(ab / r), b = (int)(ab % r);
     const int x = min(g, min(a, b)), z = max(g, max(a, b)), y = g + a + b - x - z;
-    auto g2 = [&](int u, int p) {
-        double t = 0.0;
-        for (int sp = 0; sp < ns; ++sp) t += G2[sp * lds + (long)u * ldg + p];
-        return t;
-    };
-    H[e] = g2(x, pair_index(y, z, r)) + g2(y, pair_index(x, z, r)) + g2(z, pair_index(x, y, r));
+    const double* const g2[3] = {G2 + (long)x * ldg + pair_index(y, z, r), G2 + (long)y * ldg + pair_index(x, z, r),
+                                 G2 + (long)z * ldg + pair_index(x, y, r)};
+    double t[3] = {0.0, 0.0, 0.0};
+    for (int s0 = 0; s0 < ns; s0 += 8) {   // 24 loads in flight
+        double v[3][8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int u = 0; u < 3; ++u) v[u][k] = s0 + k < ns ? g2[u][(s0 + k) * lds] : 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+#pragma unroll
+            for (int u = 0; u < 3; ++u) t[u] += v[u][k];
+    }
+    H[e] = t[0] + t[1] + t[2];
 }
 
 // Gamma[m][n] = Gamma[n][m] = (1/36) sum over the 6 matchings sigma of the
@@ -2572,8 +2582,8 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
         MCMB_TRY(phase("expansion to pairs"));
         const int r = NB;
         const long eh = (long)r * ldh;
-        MCMB_TRY(launch_guard("expansion", (unsigned long long)((eh + 255) / 256), 256));
-        hipLaunchKernelGGL(sep_hfull, dim3((unsigned)((eh + 255) / 256)), dim3(256), 0, c->stream,
+        MCMB_TRY(launch_guard("expansion", (unsigned long long)((eh + 63) / 64), 64));
+        hipLaunchKernelGGL(sep_hfull, dim3((unsigned)((eh + 63) / 64)), dim3(64), 0, c->stream,
                            (const double*)c->sg_G.as<double>(), ldq2, (long)NB * ldq2,
                            ksplit, r, S.h.as<double>(), ldh);
         MCMB_TRY(sep_expand(c, S, NP, ld));
