@@ -17,7 +17,7 @@
 // of the rounded T.  gl_gate bounds the error for the weights at hand, and a
 // setup it does not pass takes the tetrapyd contraction.  Measured, core
 // tensor by the tetrapyd contraction -> as a node sum: lmax 2500, r = 59: 2.20
-// -> 0.20 ms; lmax 2000, r = 39: 1.22 -> 0.07 ms.
+// -> 0.18 ms; lmax 2000, r = 39: 1.22 -> 0.07 ms.
 //
 // Both parities of l are summed apart (P_l(-x) = (-1)^l P_l(x)), so the table
 // holds the nodes x >= 0 only, and the columns at +x and -x are E + O and
@@ -174,7 +174,7 @@ __device__ __forceinline__ double gl_sbound(const double* __restrict__ Sp, int n
 // is -x_s.  16 waves: waves 0..7 take the even l, 8..15 the odd ones, l =
 // parity + 2 wave' + 16 i, and their sums are added pairwise in LDS in a fixed
 // order.  Lane = node; the T row is uniform (scalar loads).  5 FP64 operations
-// per (l, node, column): at 2501 l, 1876 nodes, 60 columns 0.101 ms, 0.157
+// per (l, node, column): at 2501 l, 1876 nodes, 60 columns 0.081 ms, 0.157
 // with the 11 of an error-free running sum.  CA columns share a P load.
 constexpr int GN_W = 16;
 template <int CA>
@@ -418,8 +418,11 @@ int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, i
     MCMB_TRY(gl_table(c, npt, L.lmax));
     const GlTable& G = c->glt;
     const int nc = r + 1, K = 2 * G.SH;
-    // columns per thread: the most that still give about one workgroup per CU
-    int ca = 8;
+    // columns per thread: four (eight share a P load among more, but leave one
+    // workgroup a CU at lmax 2500: 100 us against 81), or two where four give
+    // fewer than about one workgroup per CU (lmax 2000, 40 columns, 240
+    // workgroups: 38 us with four, 53 with two)
+    int ca = 4;
     const int nbx = G.SH / 64;
     while (ca > 2 && nbx * ((nc + ca - 1) / ca) < 200) ca >>= 1;
     const int ldt = (nc + 7) & ~7;
@@ -436,8 +439,7 @@ int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, i
 #define GN_PHI(CA)                                                                                                       \
     hipLaunchKernelGGL(gl_phi<CA>, grid, block, 0, c->stream, (const dd*)G.P, G.SH, (const double*)T, ldt, nl, nc, \
                        (const double*)Sp, nsp, Phi)
-    if (ca == 8) GN_PHI(8);
-    else if (ca == 4) GN_PHI(4);
+    if (ca == 4) GN_PHI(4);
     else GN_PHI(2);
 #undef GN_PHI
     MCMB_HIP(hipGetLastError());
