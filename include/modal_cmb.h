@@ -417,7 +417,9 @@ int mcmb_device_copy(mcmb_ctx* ctx, void* dst, const void* src, size_t bytes);
 
 /* Per-phase milliseconds of the last call that records phases (the FP64
  * separable Gram: basis compression on the first call of a setup, pair
- * products or weights, l3 / l2 / l1 contractions, expansion, assembly),
+ * products or weights, l3 / l2 / l1 contractions, expansion, assembly; or, as
+ * a node sum: Legendre table when it is built, basis at the nodes, node sum,
+ * expansion to pairs, assembly),
  * each between HIP events on the context stream.  Writes up to cap entries of
  * ms[] and names[] (static strings) and returns the phase count (0 if the last
  * such call recorded none; with MCMB_PHASES=0 in the environment no call
