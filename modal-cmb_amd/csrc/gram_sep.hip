@@ -23,6 +23,7 @@
 // point-by-point contraction; the summation is FP64 throughout and in a
 // fixed order (no atomics), so repeated calls are bit-identical.
 #include "mcmb_internal.h"
+#include "step_status.h"
 #include "weights.h"
 #include <algorithm>
 #include <chrono>
@@ -848,14 +849,14 @@ __global__ __launch_bounds__(256) void sep_mgs_norms(const double* __restrict__ 
 // in place).  nin[f] is the squared residual norm of column f after step a - 1
 // (-1 once f has been a pivot); the pivot p is the largest (the smallest f on
 // ties), and its squared norm is recorded in piv[a].  The factorisation stops
-// (rank[0] = a) when the pivot's squared norm is at most tol2 times the first
-// pivot's (kept in n0[0]), and gives up (rank[0] = -2) at a = amax.  Otherwise, with v = Uc[p] / |Uc[p]|: Pc[a] = v;
+// (status a) when the pivot's squared norm is at most tol2 times the first
+// pivot's (kept in n0[0]), and gives up (status -2) at a = amax.  Otherwise, with v = Uc[p] / |Uc[p]|: Pc[a] = v;
 // for every column that has not been a pivot Ct[a][f] = v . Uc[f], Uc[f] -=
 // Ct[a][f] v and nout[f] = |Uc[f]|^2; Ct[a][p] = |Uc[p]| and Ct[a][f] = 0 for
 // earlier pivots.  Every workgroup takes the same decisions from the same nin
 // and the pivot column is only read, so the in-place update is race-free.
-// Launched for a = 0, 1, ... in stream order; after rank[0] is set the later
-// launches return at once.
+// Launched for a = 0, 1, ... in stream order (status words: step_status.h);
+// once the chain has stopped the later launches only pass the status on.
 //
 // A launch per step, bound by its chain of dependent memory round trips: one
 // workgroup per column of 256 V threads (V = 1 or 4) keeps the column in
@@ -869,7 +870,7 @@ template <int V>
 __global__ __launch_bounds__(256 * V) void sep_mgs_step(double* __restrict__ Uc, int nlp, int NP,
                                                         const double* __restrict__ nin, double* __restrict__ nout,
                                                         int a, int amax, double tol2, double* __restrict__ n0,
-                                                        int* __restrict__ rank, double* __restrict__ piv,
+                                                        int* __restrict__ st, double* __restrict__ piv,
                                                         double* __restrict__ Pc, double* __restrict__ Ct, int ldct)
 {
     constexpr int T = 256 * V, NW = T / 64, NV = MGS_NV;
@@ -883,7 +884,11 @@ __global__ __launch_bounds__(256 * V) void sep_mgs_step(double* __restrict__ Uc,
     for (int k = 0; k < NV; ++k) ur[k] = tid + T * k < nlp ? u[tid + T * k] : 0.0;
     const double nf = nin[f];
     const double ref0 = a == 0 ? 0.0 : n0[0];
-    if (*rank != -1) return;
+    const int status = step_status(st, a);
+    if (status != STEP_RUNNING) {
+        if (f == 0 && tid == 0) step_stop(st, a, status);
+        return;
+    }
     double best = -2.0;
     int bi = NP;
     for (int g = tid; g < NP; g += T) {
@@ -915,11 +920,11 @@ __global__ __launch_bounds__(256 * V) void sep_mgs_step(double* __restrict__ Uc,
     const double ref = a == 0 ? n2 : ref0;
     if (f == 0 && tid == 0) piv[a] = n2;
     if (!(n2 > tol2 * ref)) {
-        if (f == 0 && tid == 0) *rank = a;
+        if (f == 0 && tid == 0) step_stop(st, a, a);
         return;
     }
     if (a >= amax) {
-        if (f == 0 && tid == 0) *rank = -2;
+        if (f == 0 && tid == 0) step_stop(st, a, -2);
         return;
     }
     if (a == 0 && f == 0 && tid == 0) n0[0] = n2;
@@ -1851,16 +1856,16 @@ static int separable_compress(mcmb_ctx* c, SepComp& S, const BasisRef& Bq, int n
     DevBuf uc, nrm, dpxy, dpiv;
     MCMB_TRY(uc.alloc(sizeof(double) * (size_t)NP * nlp));
     MCMB_TRY(dpiv.alloc(sizeof(double) * ((size_t)amax + 2)));
-    MCMB_TRY(nrm.alloc(sizeof(double) * (2 * (size_t)NP + 2)));
+    MCMB_TRY(nrm.alloc(sizeof(double) * (2 * (size_t)NP + 1) + sizeof(int) * step_words(amax)));
     MCMB_TRY(dpxy.alloc(sizeof(int2) * (size_t)NP));
     MCMB_TRY(S.pc.alloc(sizeof(double) * (size_t)std::max(1, amax) * nlp));
     MCMB_TRY(S.ct.alloc(sizeof(double) * (size_t)std::max(1, amax) * ld));
     double* const dn = nrm.as<double>();
     double* const n0 = dn + 2 * NP;
-    int* const rank = reinterpret_cast<int*>(n0 + 1);
+    int* const st = reinterpret_cast<int*>(n0 + 1);
     MCMB_HIP(hipMemcpyAsync(dpxy.p, pxy.data(), sizeof(int2) * (size_t)NP, hipMemcpyHostToDevice, c->stream));
     MCMB_HIP(hipMemsetAsync(S.ct.p, 0, S.ct.bytes, c->stream));
-    MCMB_HIP(hipMemsetAsync(rank, 0xff, sizeof(int), c->stream));   // -1: running
+    MCMB_HIP(hipMemsetAsync(st, 0xff, sizeof(int) * step_words(amax), c->stream));   // STEP_RUNNING
     const long e = (long)NP * nlp;
     MCMB_TRY(launch_guard("pair columns", (unsigned long long)((e + 255) / 256), 256));
     hipLaunchKernelGGL(sep_ucols, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, c->stream, Bq.q, Bq.ldq, nl, nlp,
@@ -1873,14 +1878,15 @@ static int separable_compress(mcmb_ctx* c, SepComp& S, const BasisRef& Bq, int n
     const bool wide = nlp > 256 * MGS_NV;
     if (nlp > 1024 * MGS_NV) return fail(MCMB_ERR_ARG, "pair basis: %d rows are more than %d", nlp, 1024 * MGS_NV);
     for (int a0 = 0; a0 <= amax && hr == -1; a0 += 8) {
-        for (int a = a0; a < a0 + 8 && a <= amax; ++a)
+        const int a1 = std::min(a0 + 8, amax + 1);
+        for (int a = a0; a < a1; ++a)
             hipLaunchKernelGGL(wide ? sep_mgs_step<4> : sep_mgs_step<1>, dim3((unsigned)NP), dim3(wide ? 1024 : 256), 0,
                                c->stream, uc.as<double>(), nlp, NP,
                                (const double*)(dn + (a & 1) * NP), dn + ((a + 1) & 1) * NP, a, amax,
-                               SEP_RANK_TOL * SEP_RANK_TOL, n0, rank, dpiv.as<double>(), S.pc.as<double>(),
+                               SEP_RANK_TOL * SEP_RANK_TOL, n0, st, dpiv.as<double>(), S.pc.as<double>(),
                                S.ct.as<double>(), ld);
         MCMB_HIP(hipGetLastError());
-        MCMB_HIP(hipMemcpyAsync(&hr, rank, sizeof(int), hipMemcpyDeviceToHost, c->stream));
+        MCMB_HIP(hipMemcpyAsync(&hr, st + a1, sizeof(int), hipMemcpyDeviceToHost, c->stream));
         MCMB_HIP(hipStreamSynchronize(c->stream));
     }
     int r = hr > 0 ? hr : 0;

@@ -161,6 +161,27 @@ def test_pair_basis_factorisation_rows(ctx, L):
     assert rel_elem(G, Gd) < 1e-13 * max(1.0, L / 2500) ** 2
 
 
+# the widest basis (528 pair products, so workgroups of a step start after others
+# have ended), at both workgroup sizes: a factorisation that stops at its rank
+# and one that gives up at half the pairs
+@pytest.mark.parametrize("L,full", [(3071, False), (3072, False), (3071, True), (3072, True)])
+def test_pair_basis_factorisation_stops_wide(ctx, L, full):
+    R = 32
+    ws = W.lspace(L, R, False)
+    if full:
+        ws["q"] = np.random.default_rng(L).standard_normal((L + 1, R))
+    order = ws["order"][np.random.default_rng(1).choice(len(ws["order"]), 60, replace=False)]
+    ctx.lspace_set(2, L, ws["q"], ws["v"], order)
+    G = ctx.gamma_gl()
+    assert ctx.last_basis_rank() == (0 if full else 2 * R - 1)
+    os.environ["MCMB_GL_PATH"] = "direct"
+    try:
+        Gd = ctx.gamma_gl()
+    finally:
+        del os.environ["MCMB_GL_PATH"]
+    assert rel_elem(G, Gd) < 1e-13 * (L / 2500) ** 2   # as above
+
+
 def test_gamma_gl_full_rank_basis_takes_direct_node_sum(ctx):
     """A random basis has full-rank pair products: no compressed basis, and
     the GL Gram is the direct node sum bit for bit."""
