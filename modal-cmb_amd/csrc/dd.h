@@ -64,8 +64,10 @@ __device__ __forceinline__ dd operator/(dd a, dd b)
 // 2^(k-51)) throughout.  acc.hi + a b.hi rounded to u differs from acc.hi by an
 // exact multiple of u, which the next operation recovers, and the term's rest,
 // at most u / 2, goes to acc.lo with b's low part: five operations a term (six
-// for two dd), against eleven with an error-free sum of the running value, at
-// an error of about 2^-104 of 2^k a term in place of the partial sum's.
+// for two dd), against eleven with an error-free sum of the running value.  A
+// term rounds at 2^-53 of acc.lo: of rests of random sign that is about 2^-104
+// of 2^k a term, but acc.lo is not folded back, and after n rests of one sign it
+// is n u / 2 and the sum's error up to n^2 2^-104 of 2^k.
 __device__ __forceinline__ double dd_bias(double bound)
 {
     return bound > 0.0 && bound < INFINITY ? ldexp(3.0, ilogb(bound) + 1) : 3.0;

@@ -13,11 +13,13 @@
 // L^2 times the result, which is why the FP64 node sum (mcmb_gamma_gl) keeps
 // only ten digits.  So the nodes, P_l, Phi and the node sum are carried in
 // double-double (T, as in the tetrapyd order, is rounded once), and H is
-// rounded once at the end: at lmax 2500 it is within 2^-53 of the exact sum
-// of the rounded T.  gl_gate bounds the error for the weights at hand, and a
-// setup it does not pass takes the tetrapyd contraction.  Measured, core
-// tensor by the tetrapyd contraction -> as a node sum: lmax 2500, r = 59: 2.20
-// -> 0.18 ms; lmax 2000, r = 39: 1.22 -> 0.07 ms.
+// rounded once at the end.  What double-double leaves of the forbidden terms is
+// alike for all entries, so an entry that the rules make small (columns of
+// local support or of one parity) or zero would be lost in it: gl_gate
+// compares it with what the rules allow, entry by entry, on the first call of a
+// setup, and a setup with an entry that does not pass takes the tetrapyd
+// contraction.  Measured, core tensor by the tetrapyd contraction -> as a node
+// sum: lmax 2500, r = 59: 2.20 -> 0.18 ms; lmax 2000, r = 39: 1.22 -> 0.07 ms.
 //
 // Both parities of l are summed apart (P_l(-x) = (-1)^l P_l(x)), so the table
 // holds the nodes x >= 0 only, and the columns at +x and -x are E + O and
@@ -130,37 +132,33 @@ __global__ __launch_bounds__(64) void gl_ptab(int lmax, int half, int SH, const 
     }
 }
 
-// T[l][a] = (2l + 1) v_l P[l][a] for a < r, and the gate's column a = r, (2l +
-// 1) |v_l| max_a |P[l][a]|; 0 for lmin > l and for r < a < ldt.  One workgroup
-// per 32 l (Pc is stored by columns, T by rows), which leaves the sum of its
-// part of the gate's column in Sp (if given).
+// T[l][a] = (2l + 1) v_l P[l][a] for a < r; 0 for lmin > l and for r <= a <
+// ldt.  One workgroup per 32 l (Pc is stored by columns, T by rows), which
+// leaves the sum over its l of (2l + 1) |v_l| max_a |P[l][a]| in Sp (if given).
 __global__ __launch_bounds__(256) void gl_ttab(const double* __restrict__ Pc, int nlp, int nl, int r, int lmin,
                                                const double* __restrict__ v, int ldt, double* __restrict__ T,
                                                double* __restrict__ Sp)
 {
-    __shared__ double S[GN_RMAX + 1][33];
+    __shared__ double S[GN_RMAX][33];
     const int l0 = blockIdx.x * 32, tl = threadIdx.x & 31;
     for (int a = threadIdx.x >> 5; a < r; a += 8) S[a][tl] = l0 + tl < nl ? Pc[(long)a * nlp + l0 + tl] : 0.0;
     __syncthreads();
     if (threadIdx.x < 32) {
         double m = 0.0;
         for (int a = 0; a < r; ++a) m = fmax(m, fabs(S[a][tl]));
-        S[r][tl] = m;
         const int l = l0 + tl;
         double g = l < nl && l >= lmin ? m * fabs((2.0 * l + 1.0) * v[l]) : 0.0;
         for (int o = 16; o >= 1; o >>= 1) g += __shfl_xor(g, o);
         if (Sp && tl == 0) Sp[blockIdx.x] = g;
     }
-    __syncthreads();
     for (int e = threadIdx.x; e < 32 * ldt; e += 256) {
         const int l = l0 + e / ldt, a = e % ldt;
         if (l >= nl) break;
-        const double f = (2.0 * l + 1.0) * v[l];
-        T[(long)l * ldt + a] = (l < lmin || a > r) ? 0.0 : S[a][l - l0] * (a < r ? f : fabs(f));
+        T[(long)l * ldt + a] = (l < lmin || a >= r) ? 0.0 : S[a][l - l0] * ((2.0 * l + 1.0) * v[l]);
     }
 }
 
-// S = sum_l T[l][r] from gl_ttab's parts, alike in every lane of every wave:
+// S = sum_l max_a |T[l][a]| from gl_ttab's parts, alike in every lane of every wave:
 // no column's sum of |T[l][a] P_l| exceeds it (|P_l| <= 1).
 __device__ __forceinline__ double gl_sbound(const double* __restrict__ Sp, int nsp, int lane)
 {
@@ -176,13 +174,15 @@ __device__ __forceinline__ double gl_sbound(const double* __restrict__ Sp, int n
 // order.  Lane = node; the T row is uniform (scalar loads).  5 FP64 operations
 // per (l, node, column): at 2501 l, 1876 nodes, 60 columns 0.081 ms, 0.157
 // with the 11 of an error-free running sum.  CA columns share a P load.
+// GATE: PhiA[a][k] = sum_l |T[l][a]| P_l(x_k) in FP64 beside them.
 constexpr int GN_W = 16;
-template <int CA>
+template <int CA, bool GATE>
 __global__ __launch_bounds__(64 * GN_W) void gl_phi(const dd* __restrict__ P, int SH, const double* __restrict__ T,
                                                     int ldt, int nl, int nc, const double* __restrict__ Sp, int nsp,
-                                                    dd* __restrict__ Phi)
+                                                    dd* __restrict__ Phi, double* __restrict__ PhiA)
 {
     __shared__ dd R[GN_W / 2][CA][64];
+    __shared__ double RA[GATE ? GN_W : 1][CA][64];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // block b: node block nb and column group cg with b = 8 (ncg (nb / 8) + cg)
     // + nb % 8, so the column groups of a node block share an XCD (b % 8) and
@@ -196,14 +196,21 @@ __global__ __launch_bounds__(64 * GN_W) void gl_phi(const dd* __restrict__ P, in
     dd acc[CA];
 #pragma unroll
     for (int k = 0; k < CA; ++k) acc[k] = dd{B, 0.0};
+    double aa[CA] = {};
     const dd* const p = P + s;
 #pragma unroll 4
     for (int l = par + 2 * ww; l < nl; l += GN_W) {
         const dd pl = p[(long)l * SH];
         const double* const t = T + (long)l * ldt + a0;
 #pragma unroll
-        for (int k = 0; k < CA; ++k) dd_bmac(acc[k], t[k], pl);
+        for (int k = 0; k < CA; ++k) {
+            dd_bmac(acc[k], t[k], pl);
+            if (GATE) aa[k] = __builtin_fma(fabs(t[k]), pl.hi, aa[k]);
+        }
     }
+    if (GATE)
+#pragma unroll
+        for (int k = 0; k < CA; ++k) RA[wave][k][lane] = aa[k];
 #pragma unroll
     for (int k = 0; k < CA; ++k) acc[k] = dd_unbias(acc[k], B);
     // 8 -> 4 -> 2 -> 1 waves per parity
@@ -231,6 +238,17 @@ __global__ __launch_bounds__(64 * GN_W) void gl_phi(const dd* __restrict__ P, in
                 out[s] = acc[k] + o;
                 out[SH + s] = acc[k] - o;
             }
+    if (GATE && wave < CA && a0 + wave < nc) {
+        double e = 0.0, o = 0.0;
+#pragma unroll
+        for (int w = 0; w < GN_W / 2; ++w) {
+            e += RA[w][wave][lane];
+            o += RA[GN_W / 2 + w][wave][lane];
+        }
+        double* const out = PhiA + (long)(a0 + wave) * 2 * SH;
+        out[s] = e + o;
+        out[SH + s] = e - o;
+    }
 }
 
 // Sum the 32 accumulators of a wave over its lanes, halving their number with
@@ -256,8 +274,7 @@ __device__ __forceinline__ dd wave_totals(dd (&acc)[32], int lane)
 // at all its orders).  Wave q takes a quarter of the 64-node steps, lane =
 // node: per step 10 columns are read for 32 products (6 operations each plus
 // the pair products; the reads come from L2): 0.088 ms at 3752 nodes and 59
-// columns, 0.120 with 12 operations each.  The last workgroup forms the gate's
-// two sums.
+// columns, 0.120 with 12 operations each.
 __device__ __forceinline__ void core_job(int job, int NT, int* ta, int* tb, int* tc, int* h)
 {
     int t = 0;
@@ -270,33 +287,14 @@ __device__ __forceinline__ void core_job(int job, int NT, int* ta, int* tb, int*
 }
 
 __global__ __launch_bounds__(256, 2) void gl_core_dd(const dd* __restrict__ Phi, int SH, const dd* __restrict__ w,
-                                                     int r, double scale, double* __restrict__ H, long ldh, int njobs,
-                                                     const double* __restrict__ Sp, int nsp,
-                                                     double* __restrict__ gate)
+                                                     int r, double scale, double* __restrict__ H, long ldh,
+                                                     const double* __restrict__ Sp, int nsp)
 {
     __shared__ dd R[4][32];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, K = 2 * SH;
     const double S = gl_sbound(Sp, nsp, lane);
-    if (blockIdx.x == (unsigned)njobs) {
-        // gate[0] = sum_k w_k Phi_r^3, gate[1] = S; H's padding
-        // (r^2 odd) is zeroed
-        if (ldh > (long)r * r)
-            for (int g = threadIdx.x; g < r; g += 256) H[(long)g * ldh + (long)r * r] = 0.0;
-        dd A{0.0, 0.0};
-        for (int k = threadIdx.x; k < K; k += 256) {
-            const dd f = Phi[(long)r * K + k];
-            A = A + w[k < SH ? k : k - SH] * f * (f * f);
-        }
-        for (int o = 32; o >= 1; o >>= 1) A = A + dd_shfl_xor(A, o);
-        if (lane == 0) R[wave][0] = A;
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const dd a = (R[0][0] + R[1][0]) + (R[2][0] + R[3][0]);
-            gate[0] = a.hi + a.lo;
-            gate[1] = S;
-        }
-        return;
-    }
+    if (blockIdx.x == 0 && ldh > (long)r * r)   // H's padding (r^2 odd)
+        for (int g = threadIdx.x; g < r; g += 256) H[(long)g * ldh + (long)r * r] = 0.0;
     int ta, tb, tc, h;
     core_job(blockIdx.x, (r + 3) / 4, &ta, &tb, &tc, &h);
     // |Phi| <= S and sum w = 2
@@ -368,6 +366,69 @@ __global__ __launch_bounds__(256, 2) void gl_core_dd(const dd* __restrict__ Phi,
     }
 }
 
+// The gate of every entry a <= b <= c (gl_gate): A = sum_k w_k PhiA_a PhiA_b
+// PhiA_c is, but for H's factor, the sum over the allowed multipole triples of
+// the magnitudes of the entry's terms; gate[0] is set where margin S^3 exceeds
+// it (or either is not a number), and gate[1] = S.  FP64: A cancels as H does,
+// and keeps 1e-14 of S^3, a hundredth and less of what it is compared with.
+// Jobs as gl_core_dd's; 256 nodes a stage in LDS, 32 threads for four entries (one
+// entry to eight threads, with three LDS reads a product, took twice as long).
+// On the first call of a setup alone: 3752 nodes and 59 columns 51 us, 1856 and
+// 25 12.
+__global__ __launch_bounds__(256) void gl_core_gate(const double* __restrict__ PhiA, int SH, const dd* __restrict__ w,
+                                                    int r, double margin, const double* __restrict__ Sp, int nsp,
+                                                    double* __restrict__ gate)
+{
+    __shared__ double F[10][256];   // 4 a, 4 c, 2 b with the node's weight
+    const int tid = threadIdx.x, K = 2 * SH;
+    int ta, tb, tc, h;
+    core_job(blockIdx.x, (r + 3) / 4, &ta, &tb, &tc, &h);
+    // columns past r repeat the last one (their entries are not looked at)
+    const double* row[10];
+#pragma unroll
+    for (int u = 0; u < 10; ++u) {
+        const int f = u < 4 ? 4 * ta + u : u < 8 ? 4 * tc + u - 4 : 4 * tb + 2 * h + u - 8;
+        row[u] = PhiA + (long)min(f, r - 1) * K;
+    }
+    double v[10];
+    auto load = [&](int k) {   // node k, of weight 0 past the last
+        const double wk = k < K ? w[k < SH ? k : k - SH].hi : 0.0;
+        const int kc = min(k, K - 1);
+#pragma unroll
+        for (int u = 0; u < 10; ++u) v[u] = row[u][kc];
+        v[8] *= wk;
+        v[9] *= wk;
+    };
+    const int n = tid & 31, i = (tid >> 5) & 3, q = 2 * (tid >> 7);   // a = i; b = 0, 1; c = q, q + 1
+    double t[4] = {0.0, 0.0, 0.0, 0.0};
+    load(tid);
+    for (int k0 = 0; k0 < K; k0 += 256) {
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 10; ++u) F[u][tid] = v[u];
+        __syncthreads();
+        load(k0 + 256 + tid);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const double fa = F[i][32 * u + n], c0 = F[4 + q][32 * u + n], c1 = F[5 + q][32 * u + n];
+#pragma unroll
+            for (int z = 0; z < 2; ++z) {
+                const double p = F[8 + z][32 * u + n] * fa;
+                t[2 * z] = __builtin_fma(p, c0, t[2 * z]);
+                t[2 * z + 1] = __builtin_fma(p, c1, t[2 * z + 1]);
+            }
+        }
+    }
+    const double S = gl_sbound(Sp, nsp, tid & 63);
+    if (blockIdx.x == 0 && tid == 0) gate[1] = S;
+#pragma unroll
+    for (int z = 0; z < 4; ++z) {
+        for (int o = 16; o >= 1; o >>= 1) t[z] += __shfl_xor(t[z], o);
+        const int a = 4 * ta + i, b = 4 * tb + 2 * h + (z >> 1), c = 4 * tc + q + (z & 1);
+        if (n == 0 && a <= b && b <= c && c < r && !(margin * (S * S * S) <= t[z])) gate[0] = 1.0;
+    }
+}
+
 // The double-double rule of order npt and P_l at its nodes up to lmax, kept by
 // the context for the last (npt, lmax): they depend on nothing else.
 int gl_table(mcmb_ctx* c, int npt, int lmax)
@@ -394,8 +455,8 @@ int gl_table(mcmb_ctx* c, int npt, int lmax)
     return MCMB_OK;
 }
 
-// Whether the node form takes this setup's whole Gram (see the header comment;
-// the gate is checked after the sums).  Below GN_LMIN the tetrapyd contraction
+// Whether the node form may take this setup's whole Gram (see the header
+// comment; then gl_gate decides).  Below GN_LMIN the tetrapyd contraction
 // stays the default: it takes 0.16 ms there, most of it launches, and its
 // results are the same bits for all its kernel variants.  Above GN_TABMAX the
 // table of P_l would be kept at the expense of the caller's memory.
@@ -403,71 +464,82 @@ bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool
 {
     if (L.kspace || L.uniform || L.h2mode != MCMB_H2_EXACT || L.kstep != 2) return false;
     if (row_lo != 0 || row_hi != (int)L.rows.size()) return false;
-    if (r < 1 || r + 1 > GN_RMAX || (L.lmax <= GN_LMIN && !any_lmax)) return false;
+    if (r < 1 || r >= GN_RMAX || (L.lmax <= GN_LMIN && !any_lmax)) return false;
     const size_t half = (3 * (size_t)L.lmax / 2 + 2) / 2 + 64;
     return sizeof(dd) * half * (L.lmax + 1) <= GN_TABMAX;
 }
 
+// The gate.  The terms of an entry of H are at most 2 S^3 in sum, S = sum_l max_a
+// |T[l][a]| (|P_l| <= 1, sum w = 2), and the roundings of the node form are
+// shares of that whatever the entry.  The sums A of gl_core_gate, over the
+// magnitudes of the terms that the rules allow, must be at least margin S^3: an
+// error of 2^-101 (lmax + 64) 2 S^3 is then within 2^-54 of A, where FP64
+// itself rounds.  That error is an estimate with room, no bound: against 113
+// bits the entries of six Legendre columns are off by 2^-98.3 of 2 S^3 at most at
+// lmax 2500 (2^-99.3 at 600, 2^-98.6 at 6000; the estimate is 2^-89.7, 2^-91.6
+// and 2^-88.4), while rests of a biased sum that were all of one sign would grow
+// as the square of a wave's terms (dd_bmac), to 2^-83.  The benchmark's
+// spectra pass with a factor 140 to spare at lmax 2500 with 59 columns, 3e4 at
+// 600 with 19; bins, hat functions, Gaussians of a width of lmax / 20 and bases
+// of one parity do not pass.
+static double gl_margin(int lmax) { return 0x1p-46 * (lmax + 64.0); }
+
+// After the stream has been waited for.
+bool gl_gate(const mcmb_ctx* c)
+{
+    const double S = c->gn_gate[1], b = 2.0 * S * S * S;
+    // (within reach of overflow or of subnormal rests the bias does not hold)
+    return c->gn_gate[0] == 0.0 && (S == 0.0 || (b > 1e-250 && b < 1e300));
+}
+
 // H (r x ldh) of the exact tetrapyd Gram over the r columns Pc (by columns,
-// leading dimension nlp).  phase: called with the name of each part.
+// leading dimension nlp).  phase: called with the name of each part.  gate: the
+// sums of gl_gate too.
 int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, int nl, int r, double* H, long ldh,
-                    const std::function<int(const char*)>& phase)
+                    bool gate, const std::function<int(const char*)>& phase)
 {
     const int npt = 3 * L.lmax / 2 + 1;
     if (!(c->glt.npt == npt && c->glt.lmax >= L.lmax)) MCMB_TRY(phase("Legendre table"));
     MCMB_TRY(gl_table(c, npt, L.lmax));
     const GlTable& G = c->glt;
-    const int nc = r + 1, K = 2 * G.SH;
+    const int K = 2 * G.SH;
     // columns per thread: four (eight share a P load among more, but leave one
     // workgroup a CU at lmax 2500: 100 us against 81), or two where four give
     // fewer than about one workgroup per CU (lmax 2000, 40 columns, 240
     // workgroups: 38 us with four, 53 with two)
     int ca = 4;
     const int nbx = G.SH / 64;
-    while (ca > 2 && nbx * ((nc + ca - 1) / ca) < 200) ca >>= 1;
-    const int ldt = (nc + 7) & ~7;
+    while (ca > 2 && nbx * ((r + ca - 1) / ca) < 200) ca >>= 1;
+    const int ldt = (r + 7) & ~7;
     const int nsp = (nl + 31) / 32;
-    MCMB_TRY(c->gn_ws.alloc(sizeof(dd) * (size_t)nc * K + sizeof(double) * ((size_t)nl * ldt + nsp)));
+    MCMB_TRY(c->gn_ws.alloc(sizeof(dd) * (size_t)r * K +
+                            sizeof(double) * ((size_t)nl * ldt + nsp + (gate ? (size_t)r * K : 0))));
     dd* const Phi = c->gn_ws.as<dd>();
-    double* const T = reinterpret_cast<double*>(Phi + (size_t)nc * K);
+    double* const T = reinterpret_cast<double*>(Phi + (size_t)r * K);
     double* const Sp = T + (size_t)nl * ldt;
+    double* const PhiA = Sp + nsp;
     if (!c->gn_gate) MCMB_HIP(hipHostMalloc((void**)&c->gn_gate, 2 * sizeof(double), hipHostMallocDefault));
     MCMB_TRY(phase("basis at the nodes"));
     hipLaunchKernelGGL(gl_ttab, dim3((nl + 31) / 32), dim3(256), 0, c->stream, Pc, nlp, nl, r, L.lmin,
                        (const double*)L.d_v.as<double>(), ldt, T, Sp);
-    const dim3 grid(8 * ((nbx + 7) / 8) * ((nc + ca - 1) / ca)), block(64 * GN_W);
-#define GN_PHI(CA)                                                                                                       \
-    hipLaunchKernelGGL(gl_phi<CA>, grid, block, 0, c->stream, (const dd*)G.P, G.SH, (const double*)T, ldt, nl, nc, \
-                       (const double*)Sp, nsp, Phi)
-    if (ca == 4) GN_PHI(4);
-    else GN_PHI(2);
-#undef GN_PHI
+    const dim3 grid(8 * ((nbx + 7) / 8) * ((r + ca - 1) / ca)), block(64 * GN_W);
+    auto* const phi = ca == 4 ? (gate ? gl_phi<4, true> : gl_phi<4, false>) : (gate ? gl_phi<2, true> : gl_phi<2, false>);
+    hipLaunchKernelGGL(phi, grid, block, 0, c->stream, (const dd*)G.P, G.SH, (const double*)T, ldt, nl, r,
+                       (const double*)Sp, nsp, Phi, PhiA);
     MCMB_HIP(hipGetLastError());
     MCMB_TRY(phase("node sum"));
     const int NT = (r + 3) / 4;
     int njobs = 0;
     for (int t = 0; t < NT; ++t) njobs += 2 * (t + 1) * (NT - t);
-    hipLaunchKernelGGL(gl_core_dd, dim3(njobs + 1), dim3(256), 0, c->stream, (const dd*)Phi, G.SH, (const dd*)G.w, r,
-                       3.0 / (4.0 * M_PI), H, ldh, njobs, (const double*)Sp, nsp, c->gn_gate);
+    if (gate) {
+        c->gn_gate[0] = 0.0;   // (the stream has been waited for since a kernel last wrote it)
+        hipLaunchKernelGGL(gl_core_gate, dim3(njobs), dim3(256), 0, c->stream, (const double*)PhiA, G.SH,
+                           (const dd*)G.w, r, gl_margin(L.lmax), (const double*)Sp, nsp, c->gn_gate);
+    }
+    hipLaunchKernelGGL(gl_core_dd, dim3(njobs), dim3(256), 0, c->stream, (const dd*)Phi, G.SH, (const dd*)G.w, r,
+                       3.0 / (4.0 * M_PI), H, ldh, (const double*)Sp, nsp);
     MCMB_HIP(hipGetLastError());
     return MCMB_OK;
-}
-
-// After the stream has been synchronised: whether the sums are good to FP64.
-// With m_l = max_a |P[l][a]|, every term of every entry is bounded by those of
-// sum w Phi_m^3 formed with absolute values, at most 2 S^3 (|P_l| <= 1, sum w
-// = 2); A = sum w Phi_m^3 is the tetrapyd sum of the same bound over the
-// allowed terms, the scale of H that FP64 resolves to 2^-53.  Each term
-// carries about 2^-104 times a growth of the recurrence linear in l, and the
-// biased sums of Phi and of H each add 2^-104 of their bound (at most 4 S, 8
-// S^3 and so 4 times the terms') a term: 2^-101 covers them.  (The workloads'
-// spectra pass with 3 decades to spare at lmax 2500, 5 at 520.)
-bool gl_gate(const mcmb_ctx* c, int lmax)
-{
-    const double A = c->gn_gate[0], S = c->gn_gate[1], b = 2.0 * S * S * S;
-    // (within reach of overflow or of subnormal rests the bias does not hold)
-    if (S != 0.0 && !(b > 1e-250 && b < 1e300)) return false;
-    return b * 0x1p-101 * (lmax + 64.0) <= 0x1p-54 * A;
 }
 
 // ---- the FP64 node sum (mcmb_gamma_gl, mcmb_gamma_gl_pol) over compressed bases ----

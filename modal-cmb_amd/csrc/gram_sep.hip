@@ -2335,7 +2335,8 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
     bool rowptr_ready = false;
     auto plan = [&]() { return separable_plan(c, L, row_lo, row_hi, NB, ldB, gsz, tm, tn, ksplit, rowptr_ready); };
     // The core as a node sum (gram_nodes.hip), unless a switch of the tetrapyd
-    // contraction is set or the error bound failed on this setup before.
+    // contraction is set or an entry of this setup's core is not resolved by it
+    // (gl_gate, on the first call of the setup: its basis and weights decide).
     // (MCMB_SEP_TABLES asks for the contraction's tables, which the node form
     // does not read: they are built all the same, for last_setup.)
     const char* gpath = getenv("MCMB_GRAM_PATH");
@@ -2349,19 +2350,33 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
         const int r = S.r;
         MCMB_TRY(sep_expand_alloc(c, r, NP, ld));
         setup_done("buffers");
+        // the rest is queued before the verdict is known (waiting for it leaves
+        // the device idle for 15 us), unless the setup before this one failed
+        const bool gate = c->gn_passed != L.generation, wait = gate && c->gn_refused > c->gn_passed;
+        auto verdict = [&]() {
+            nodes = gl_gate(c);
+            (nodes ? c->gn_passed : c->gn_refused) = L.generation;
+        };
         MCMB_TRY(gram_nodes_core(c, L, S.pc.as<double>(), S.nlp, nl, r, S.h.as<double>(),
-                                 (long)r * r + ((r * r) & 1), phase));
-        MCMB_TRY(phase("expansion to pairs"));
-        MCMB_TRY(sep_expand(c, S, NP, ld));
-        MCMB_TRY(phase("assembly"));
-        MCMB_TRY(sep_assemble_launch(c, R, n, L.d_modes.as<int>(), d_gamma));
-        launches += 7;
-        MCMB_TRY(finish(r));
-        if (gl_gate(c, L.lmax)) return MCMB_OK;
-        c->gn_refused = L.generation;   // the tetrapyd contraction, here and from now on
+                                 (long)r * r + ((r * r) & 1), gate, phase));
+        if (wait) {
+            MCMB_HIP(hipStreamSynchronize(c->stream));
+            verdict();
+        }
+        if (nodes) {
+            MCMB_TRY(phase("expansion to pairs"));
+            MCMB_TRY(sep_expand(c, S, NP, ld));
+            MCMB_TRY(phase("assembly"));
+            MCMB_TRY(sep_assemble_launch(c, R, n, L.d_modes.as<int>(), d_gamma));
+            launches += 7 + gate;
+            MCMB_TRY(finish(r));
+            if (gate && !wait) verdict();
+            if (nodes) return MCMB_OK;
+        }
+        // the tetrapyd contraction, here and from now on
+        setup_begin(c);
         np = 0;
         launches = 0;
-        setup_begin(c);
         MCMB_HIP(hipEventRecord(c->ev0, c->stream));
         MCMB_TRY(plan());
     }

@@ -227,7 +227,7 @@ struct GlHalf {
     DevBuf buf;
     double *w = nullptr, *P = nullptr;
 };
-constexpr int GN_RMAX = 64;                    // columns of the node form, the gate's included
+constexpr int GN_RMAX = 64;                    // columns of the node form, and one
 constexpr int GN_LMIN = 512;                   // the node form takes lmax above this
 constexpr size_t GN_TABMAX = (size_t)1 << 30;  // bytes of the table of P_l
 
@@ -331,12 +331,13 @@ struct mcmb_ctx {
     // the GL Gram over compressed bases: T, Phi and the core's units
     mcmb::DevBuf gl_ws;
     // the node form of the tetrapyd Gram: rule and Legendre table, work space,
-    // the gate's two sums (pinned), and the setup that did not pass it
+    // the gate's verdict and scale (pinned), and the setups (generations) that
+    // last passed and last failed it
     mcmb::GlTable glt;
     mcmb::GlHalf glh;
     mcmb::DevBuf gn_ws;
     double* gn_gate = nullptr;
-    long gn_refused = -1;
+    long gn_passed = -1, gn_refused = -1;
     // work buffers of the Cholesky orthonormalisation and solve
     mcmb::DevBuf la_ws;
     // the GL cross-Gamma: node tables, M and the core tensor
@@ -444,13 +445,13 @@ int gram_factored_launch(mcmb_ctx* ctx, PointSet& P, int precision, double* d_ga
 // Separable Gram (contractions over l3, then l2, then l1 of the pair products):
 // whether it handles this basis width and precision, and the launch.
 // The node form of the exact l-space Gram over a compressed basis
-// (gram_nodes.hip): whether it takes the setup, the core tensor H, and after
-// the stream is synchronised whether its error bound holds.
-// (any_lmax: also up to GN_LMIN)
+// (gram_nodes.hip): whether it may take the setup (any_lmax: also up to
+// GN_LMIN), the core tensor H, and, after a call with gate set and once the
+// stream has been waited for, whether every entry of it is resolved to FP64.
 bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool any_lmax);
 int gram_nodes_core(mcmb_ctx* c, const PointSet& L, const double* Pc, int nlp, int nl, int r, double* H, long ldh,
-                    const std::function<int(const char*)>& phase);
-bool gl_gate(const mcmb_ctx* c, int lmax);
+                    bool gate, const std::function<int(const char*)>& phase);
+bool gl_gate(const mcmb_ctx* c);
 // The FP64 node sum over compressed bases (gram_nodes.hip): the half rule's
 // table, Phi of a basis, the core tensor, and their work sizes in doubles.
 int gl_half_table(mcmb_ctx* c, int npt, int lmax, const double* x, const double* w);

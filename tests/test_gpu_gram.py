@@ -634,6 +634,46 @@ def test_node_form_gate(ctx):
     assert "node sum" in [p for p, _ in ctx.last_phases()]
 
 
+def _local_basis(kind, L, R):
+    ls = np.arange(L + 1.0)
+    mid = np.linspace(0.0, L, R)
+    if kind == "bins":
+        return ((ls[:, None] * R / (L + 1)).astype(int) == np.arange(R)[None]).astype(float)
+    if kind == "hats":
+        return np.maximum(0.0, 1.0 - np.abs(ls[:, None] - mid) / (L / (R - 1)))
+    if kind == "gauss":
+        return np.exp(-0.5 * ((ls[:, None] - mid) / (L / 20.0)) ** 2)
+    # every other l: products that live on the even l only, and on the odd l only
+    q = W.legendre_table(ls / L, R // 2 - 1)
+    return np.concatenate([q * (ls[:, None] % 2 == 0), q * (ls[:, None] % 2 == 1)], 1)
+
+
+@pytest.mark.parametrize("L", [600, 2500])
+@pytest.mark.parametrize("kind", ["bins", "hats", "gauss", "parity"])
+def test_local_support_keeps_the_selection_rules(ctx, kind, L):
+    """Modes of local support or of one parity: most of their products violate
+    the triangle or the parity rule, or meet it only in the tails.  The exact
+    walk gives zero (or the tails' value) there, and a node sum the rounding of
+    terms that cancel: the default is the tetrapyd contraction, bit for bit."""
+    R = 10
+    ws = W.lspace(L, R, True)
+    q = _local_basis(kind, L, R)
+    ctx.lspace_set(2, L, q, ws["v"], ws["order"])
+    D = ctx.gamma_tet(modalcmb.FP64)
+    S = _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"]
+    if kind == "bins":
+        m = [i for i, o in enumerate(ws["order"]) if o[2] == 9 and o[1] < 4]   # l3 past l1 + l2
+        assert m and not S[m].any() and not D[m].any()
+    assert np.array_equal(D, S)
+    # a second call, and another setup between two calls
+    assert np.array_equal(ctx.gamma_tet(modalcmb.FP64), S)
+    ctx.lspace_set(2, L, ws["q"], ws["v"], ws["order"])
+    ctx.gamma_tet(modalcmb.FP64)
+    assert "node sum" in [p for p, _ in ctx.last_phases()]
+    ctx.lspace_set(2, L, q, ws["v"], ws["order"])
+    assert np.array_equal(ctx.gamma_tet(modalcmb.FP64), S)
+
+
 # The node form's sums carry a bias of a power of two above sum |T|: scales at
 # and next to a power (v times 2^k only moves the exponents, so Gamma is 2^3k
 # times the same bits), and far from one; scales at which the cube nears the
