@@ -2337,15 +2337,13 @@ int gram_separable_launch(mcmb_ctx* c, PointSet& L, int precision, double* d_gam
     // The core as a node sum (gram_nodes.hip), unless a switch of the tetrapyd
     // contraction is set or an entry of this setup's core is not resolved by it
     // (gl_gate, on the first call of the setup: its basis and weights decide).
-    // (MCMB_SEP_TABLES asks for the contraction's tables, which the node form
-    // does not read: they are built all the same, for last_setup.)
     const char* gpath = getenv("MCMB_GRAM_PATH");
     const bool asked = gpath && !strcmp(gpath, "nodes");
     bool nodes = comp && (!gpath || !*gpath || asked) && c->gn_refused != L.generation &&
                  gram_nodes_supported(L, S.r, row_lo, row_hi, asked);
     for (const char* k : {"MCMB_SEP_L3", "MCMB_SEP_WEIGHTS", "MCMB_SEP_GROUPS", "MCMB_SEP_BLOCK_ROWS"})
         if (getenv(k)) nodes = false;
-    if (!nodes || getenv("MCMB_SEP_TABLES")) MCMB_TRY(plan());
+    if (!nodes) MCMB_TRY(plan());
     if (nodes) {
         const int r = S.r;
         MCMB_TRY(sep_expand_alloc(c, r, NP, ld));

@@ -567,9 +567,10 @@ def test_separable_device_row_groups_equal_host(ctx, lmax, R, block_rows, weight
     # row groups sharing l2 formed on the device (one wave per l2 and parity)
     # are the host walk's groups, l3 ranges and weight offsets: the same Gram
     # bit for bit, with fused weights and with staged ones (which read the
-    # offsets), in one block and in several
+    # offsets), in one block and in several; by name, since the node form that
+    # is the default above lmax 512 reads no row groups
     ws = W.lspace(lmax, R, True)
-    env = {}
+    env = {"MCMB_GRAM_PATH": "separable"}
     if block_rows:
         env["MCMB_SEP_BLOCK_ROWS"] = block_rows
     if weights:
@@ -696,17 +697,21 @@ def test_node_form_scales(ctx):
         assert np.array_equal(D, _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"], equal_nan=True)
 
 
-def test_separable_device_row_groups_equal_host_lmax2500(ctx):
-    """As test_separable_device_row_groups_equal_host at a size where the
-    default is the node form, which reads no row groups: the tetrapyd
-    contraction by name."""
+def test_node_form_at_lmax2500(ctx):
+    """The default at lmax 2500 and 4960 modes against the tetrapyd contraction:
+    both are FP64 roundings of one sum (1e-13, as test_node_form_vs_separable),
+    and the node form builds none of the contraction's tables."""
     ws = W.lspace(2500, 30, True)
     ctx.lspace_set(2, 2500, ws["q"], ws["v"], ws["order"])
-    Gd = _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"]
     os.environ["MCMB_SEP_TABLES"] = "host"
     try:
-        ctx.lspace_set(2, 2500, ws["q"], ws["v"], ws["order"])      # a new setup: tables rebuilt on the host
-        Gh = _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"]
+        D = ctx.gamma_tet(modalcmb.FP64)
+        assert "node sum" in [p for p, _ in ctx.last_phases()]
+        assert "row groups and tables (host)" not in [p for p, _ in ctx.last_setup()]
     finally:
         del os.environ["MCMB_SEP_TABLES"]
-    assert np.array_equal(Gd, Gh)
+    assert ctx.last_basis_rank() == 59
+    S = _gram_paths(ctx, modalcmb.FP64, ("separable",))["separable"]
+    assert rel_elem(D, S) < 1e-13
+    assert np.array_equal(D, D.T)
+    assert np.array_equal(ctx.gamma_tet(modalcmb.FP64), D)
