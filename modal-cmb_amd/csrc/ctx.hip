@@ -1,7 +1,7 @@
 // Context, error reporting and l-space setup of libmodalcmb.
+#include "chunk_crew.h"
 #include "mcmb_internal.h"
 #include <algorithm>
-#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -75,8 +75,7 @@ int copy_stream_ready(mcmb_ctx* c)
 
 // The staged copies cut the bytes into chunks that go round CSLOTS slots of
 // pinned memory of their own: the DMA of a chunk and the host threads' move of the
-// others overlap.  The threads live for the whole copy, each moving its stripe
-// of every chunk; progress is two counters, so no thread waits for a lock.
+// others overlap (chunk_crew.h: a thread moves its stripe of every chunk).
 // Copying a fresh 19 MB array out (its pages are touched for the first time
 // here, by all threads): 1.1 -> 0.6 ms against one pageable hipMemcpy; 1 MB
 // took 0.06 ms longer (starting the threads), hence COPY_MIN.  Below COPY_BIG
@@ -85,48 +84,6 @@ int copy_stream_ready(mcmb_ctx* c)
 // ms, 31 ms through slots of 1 MiB).
 constexpr size_t COPY_BIG = 2 * STAGE_BYTES, CSTAGE_BYTES = (size_t)8 << 20;
 constexpr size_t COPY_MIN_OUT = (size_t)8 << 20, COPY_MIN_IN = (size_t)4 << 20;
-
-namespace {
-struct ChunkCrew {
-    const int nth;
-    std::vector<std::atomic<int>> done;   // threads that have moved chunk k
-    std::atomic<long> ready{0};           // chunks the threads may move
-    std::atomic<bool> stop{false};
-    std::vector<std::thread> th;
-
-    template <class F> ChunkCrew(int n, size_t nk, F move) : nth(n), done(nk)
-    {
-        for (auto& d : done) d.store(0, std::memory_order_relaxed);
-        th.reserve(n);
-        try {
-            for (int t = 0; t < n; ++t)
-                th.emplace_back([this, t, nk, move] {
-                    for (size_t k = 0; k < nk; ++k) {
-                        while (ready.load(std::memory_order_acquire) <= (long)k) {
-                            if (stop.load(std::memory_order_relaxed)) return;
-                            std::this_thread::yield();
-                        }
-                        move(t, k);
-                        done[k].fetch_add(1, std::memory_order_release);
-                    }
-                });
-        } catch (...) {   // no further thread to be had
-            join();
-            throw;
-        }
-    }
-    void join()
-    {
-        stop.store(true);
-        for (auto& x : th) x.join();
-    }
-    void wait(size_t k) const
-    {
-        while (done[k].load(std::memory_order_acquire) < nth) std::this_thread::yield();
-    }
-    ~ChunkCrew() { join(); }
-};
-}  // namespace
 
 static int staged_copy(mcmb_ctx* c, char* host, char* dev, size_t bytes, bool to_host)
 {
