@@ -85,11 +85,20 @@ int copy_stream_ready(mcmb_ctx* c)
 constexpr size_t COPY_BIG = 2 * STAGE_BYTES, CSTAGE_BYTES = (size_t)8 << 20;
 constexpr size_t COPY_MIN_OUT = (size_t)8 << 20, COPY_MIN_IN = (size_t)4 << 20;
 
+// The pinned memory of a staged copy, or null where none is to be had.
+static void* copy_staging(mcmb_ctx* c, bool big)
+{
+    void*& p = big ? c->stage : c->copy_stage;
+    if (!p && hipHostMalloc(&p, big ? 2 * STAGE_BYTES : CSTAGE_BYTES, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError();
+        p = nullptr;
+    }
+    return p;
+}
+
 static int staged_copy(mcmb_ctx* c, char* host, char* dev, size_t bytes, bool to_host)
 {
     const bool big = bytes >= COPY_BIG;
-    if (big) MCMB_TRY(stage_ready(c));
-    else if (!c->copy_stage) MCMB_HIP(hipHostMalloc(&c->copy_stage, CSTAGE_BYTES, hipHostMallocDefault));
     for (hipEvent_t& e : c->copy_ev)
         if (!e) MCMB_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     char* const stage = static_cast<char*>(big ? c->stage : c->copy_stage);
@@ -153,16 +162,16 @@ static int plain_copy(mcmb_ctx* c, void* dst, const void* src, size_t bytes, hip
     return MCMB_OK;
 }
 
-static bool copy_staged(size_t bytes, size_t least)
+static bool copy_staged(mcmb_ctx* c, size_t bytes, size_t least)
 {
     const char* env = getenv("MCMB_HOST_COPY");
-    return bytes >= least && !(env && !strcmp(env, "direct"));
+    return bytes >= least && !(env && !strcmp(env, "direct")) && copy_staging(c, bytes >= COPY_BIG);
 }
 
 int copy_to_device(mcmb_ctx* c, void* dev, const void* host, size_t bytes)
 {
     if (!bytes) return MCMB_OK;
-    if (copy_staged(bytes, COPY_MIN_IN)) {
+    if (copy_staged(c, bytes, COPY_MIN_IN)) {
         try {
             return staged_copy(c, const_cast<char*>(static_cast<const char*>(host)), static_cast<char*>(dev), bytes, false);
         } catch (const std::exception&) {   // no thread or memory to be had: copy without them
@@ -175,7 +184,7 @@ int copy_to_device(mcmb_ctx* c, void* dev, const void* host, size_t bytes)
 int copy_to_host(mcmb_ctx* c, void* host, const void* dev, size_t bytes)
 {
     if (!bytes) return MCMB_OK;
-    if (copy_staged(bytes, COPY_MIN_OUT)) {
+    if (copy_staged(c, bytes, COPY_MIN_OUT)) {
         try {
             return staged_copy(c, static_cast<char*>(host), const_cast<char*>(static_cast<const char*>(dev)), bytes, true);
         } catch (const std::exception&) {
