@@ -56,6 +56,31 @@ print("ok")
 """
 
 
+# bytes at and next to the sizes from which copies are staged in (4 MiB) and out
+# (8 MiB) and from which they take the larger staging (32 MiB): chunks of 2 MiB
+# in four slots, of 4 MiB in eight; a short last chunk, fewer chunks than slots
+@pytest.mark.parametrize("nbytes", [4 * MIB - 8, 4 * MIB, 4 * MIB + 8, 6 * MIB, 8 * MIB - 8, 8 * MIB, 8 * MIB + 8,
+                                    10 * MIB + 520, 32 * MIB - 8, 32 * MIB, 32 * MIB + 8, 45 * MIB + 136])
+def test_bytes_in_and_out(ctx, nbytes):
+    # a solve with the unit matrix returns its right-hand sides: in and out again
+    rhs = np.random.default_rng(nbytes).standard_normal((nbytes // 8, 1))
+    got = ctx.cholesky_solve(np.eye(1), rhs.T)
+    assert np.array_equal(got.ravel(), rhs.ravel())
+    # out alone, to an offset address
+    dev = ctx.device_alloc(nbytes)
+    try:
+        out = [np.zeros(nbytes // 8 + 1) for _ in range(2)]
+        ctx.device_to_host(dev, out[0][1:])
+        os.environ["MCMB_HOST_COPY"] = "direct"
+        try:
+            ctx.device_to_host(dev, out[1][1:])
+        finally:
+            del os.environ["MCMB_HOST_COPY"]
+    finally:
+        ctx.device_free(dev)
+    assert np.array_equal(out[0].view(np.int64), out[1].view(np.int64))
+
+
 def test_copies_without_pinned_memory(tmp_path):
     (tmp_path / "shim.c").write_text(SHIM)
     so = str(tmp_path / "shim.so")

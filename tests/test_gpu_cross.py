@@ -120,6 +120,23 @@ def test_cross_gl_core_tensor_edges(ctx, R, npb, nx, tlmax, late, prim):
     assert np.array_equal(G, ctx.gamma_cross_gl(modalcmb.SPLINE_NATURAL))
 
 
+def test_cross_gl_core_tensor_in_parts(ctx):
+    """640 functions: one unit of the core tensor takes 376 MB, so the units are
+    held two at a time (1 GiB) and gathered onto the sums of the parts before.
+    Two linear samples and the ten single ones; every 40th late mode.  1e-12 as
+    above."""
+    c = case(tlmax=20, Lq=24, R=20, npb=32, nx=12, seed=5)
+    c["order_late"] = np.concatenate([c["order_late"][::2], [[19, 19, 19]]]).astype(np.int32)
+    c["order_prim"] = np.concatenate([c["order_prim"][:60], [[31, 31, 31]]]).astype(np.int32)
+    setup(ctx, c)
+    G = ctx.gamma_cross_gl(modalcmb.SPLINE_NATURAL)
+    assert ctx.last_kernel_ms()[1] > 10   # launches: a table, M, and two for each part
+    ref = O.gamma_cross_gl(c["tlmin"], c["tlmax"], c["b"], c["order_late"], c["qt"], c["xvec"], c["order_prim"],
+                           c["cl"], c["nl"], c["bl"], c["dphi"], spline=modalcmb.SPLINE_NATURAL)
+    assert relmax(G, ref) < 1e-12
+    assert np.array_equal(G, ctx.gamma_cross_gl(modalcmb.SPLINE_NATURAL))
+
+
 def test_legacy_cross_entry_points(ctx):
     lib = modalcmb.load_library()
     c = case()

@@ -102,6 +102,28 @@ def test_eigen_sym_large_against_lapack(ctx, n):
     assert np.abs(V.T @ Y - X).max() < 1e-12 * np.sqrt(n) * 8
 
 
+def test_eigen_sym_rows_per_wave(ctx):
+    """Order 4100: the first columns' products take four rows a wave and the
+    others two.  A Householder reflection of a given spectrum, so the checks
+    stay O(n^2); tolerances as above."""
+    n = 4100
+    rng = np.random.default_rng(n)
+    d = np.sort(rng.standard_normal(n))[::-1].copy()
+    u = rng.standard_normal(n)
+    u /= np.linalg.norm(u)
+    w = d * u   # (I - 2 u u^T) D (I - 2 u u^T)
+    A = np.diag(d) - 2 * np.outer(u, w) - 2 * np.outer(w, u) + 4 * (u @ w) * np.outer(u, u)
+    A = 0.5 * (A + A.T)
+    ev, V, sweeps = ctx.eigen_sym(A)
+    assert sweeps == 0
+    nrm = np.abs(d).max()
+    assert np.abs(ev - d).max() < 1e-13 * nrm * 8
+    X = rng.standard_normal((n, 16))
+    Y = V @ X
+    assert np.abs(A @ Y - V @ (ev[:, None] * X)).max() < 1e-12 * nrm * np.sqrt(n) * 8
+    assert np.abs(V.T @ Y - X).max() < 1e-12 * np.sqrt(n) * 8
+
+
 def _wilkinson(m):
     """W_{2m+1}^+: diagonal |m - i|, unit off-diagonal (pairs of eigenvalues
     that agree to many digits)."""

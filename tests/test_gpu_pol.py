@@ -236,7 +236,11 @@ def cross_setup(ctx, c):
     return ttt, tte, tee, eee
 
 
-@pytest.mark.parametrize("kw", [{}, dict(T=(5, 33), E=(2, 40), RT=5, RE=3, npb=3, seed=3)])
+# (the last two: pairs of 72 and of 27 functions with third functions of 27 and
+# of 72, five and two tiles of 16 either way and a group of c tiles not full)
+@pytest.mark.parametrize("kw", [{}, dict(T=(5, 33), E=(2, 40), RT=5, RE=3, npb=3, seed=3),
+                                dict(T=(2, 37), E=(2, 40), RT=8, RE=3, npb=9, nx=13, seed=4),
+                                dict(T=(2, 40), E=(3, 31), RT=3, RE=8, npb=9, nx=31, seed=5)])
 @pytest.mark.parametrize("spline", [modalcmb.SPLINE_FMM, modalcmb.SPLINE_NATURAL])
 def test_cross_gl_pol_vs_oracle(ctx, kw, spline):
     c = cross_case(**kw)
