@@ -831,10 +831,13 @@ __global__ void sep_ucols(const double* __restrict__ q, int ldq, int nl, int nlp
     Uc[e] = l < nl ? q[(long)l * ldq + xy.x] * q[(long)l * ldq + xy.y] : 0.0;
 }
 
-// nrm[f] = |Uc[f]|^2, one wave per column
+// nrm[f] = |Uc[f]|^2, one wave per column; and the nst status words of the
+// steps (a fill of their own takes two launches more).
 __global__ __launch_bounds__(256) void sep_mgs_norms(const double* __restrict__ Uc, int nlp, int NP,
-                                                     double* __restrict__ nrm)
+                                                     double* __restrict__ nrm, int* __restrict__ st, int nst)
 {
+    if (blockIdx.x == 0)
+        for (int k = threadIdx.x; k < nst; k += 256) st[k] = STEP_RUNNING;
     const int lane = threadIdx.x & 63;
     const int f = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (f >= NP) return;
@@ -1865,14 +1868,13 @@ static int separable_compress(mcmb_ctx* c, SepComp& S, const BasisRef& Bq, int n
     int* const st = reinterpret_cast<int*>(n0 + 1);
     MCMB_HIP(hipMemcpyAsync(dpxy.p, pxy.data(), sizeof(int2) * (size_t)NP, hipMemcpyHostToDevice, c->stream));
     MCMB_HIP(hipMemsetAsync(S.ct.p, 0, S.ct.bytes, c->stream));
-    MCMB_HIP(hipMemsetAsync(st, 0xff, sizeof(int) * step_words(amax), c->stream));   // STEP_RUNNING
     const long e = (long)NP * nlp;
     MCMB_TRY(launch_guard("pair columns", (unsigned long long)((e + 255) / 256), 256));
     hipLaunchKernelGGL(sep_ucols, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, c->stream, Bq.q, Bq.ldq, nl, nlp,
                        dpxy.as<int2>(), NP, uc.as<double>());
     const unsigned ncb = (unsigned)((NP + 3) / 4);
     hipLaunchKernelGGL(sep_mgs_norms, dim3(ncb), dim3(256), 0, c->stream, (const double*)uc.as<double>(), nlp, NP,
-                       dn);
+                       dn, st, step_words(amax));
     MCMB_HIP(hipGetLastError());
     int hr = -1;
     const bool wide = nlp > 256 * MGS_NV;
