@@ -339,7 +339,7 @@ def gamma_roofline(phases, npts, L, nb, workload):
     or the l3 contraction on FP64 MFMA where the tetrapyd contraction runs."""
     ms = phases.get("basis at the nodes")
     if ms:
-        ops = 5.0 * (nb + 1) * (L + 1) * ((3 * L // 2 + 2) // 2)
+        ops = 5.0 * nb * (L + 1) * ((3 * L // 2 + 2) // 2)
         achieved = ops / (ms * 1e-3) / 1e12
         return {"bound": "fp64 valu", "achieved": round(achieved, 2), "peak": PEAK_FP64_TFLOPS / 2,
                 "unit": "T FP64 operations/s", "frac": round(achieved / (PEAK_FP64_TFLOPS / 2), 4), "traffic": None,

@@ -456,10 +456,13 @@ int gl_table(mcmb_ctx* c, int npt, int lmax)
 }
 
 // Whether the node form may take this setup's whole Gram (see the header
-// comment; then gl_gate decides).  Below GN_LMIN the tetrapyd contraction
-// stays the default: it takes 0.16 ms there, most of it launches, and its
-// results are the same bits for all its kernel variants.  Above GN_TABMAX the
-// table of P_l would be kept at the expense of the caller's memory.
+// comment; then gl_gate decides).  Up to GN_LMIN the tetrapyd contraction
+// stays the default not for its time (a repeated call takes 150 us at lmax 500
+// with 10 functions against 82, 184 against 114 with 20, 435 against 335 with
+// 30, 101 against 78 at lmax 200 with 10) but for its bits, which are the same
+// for all its kernel variants and on which callers of those sizes may rely.
+// Above GN_TABMAX the table of P_l would be kept at the expense of the caller's
+// memory.
 bool gram_nodes_supported(const PointSet& L, int r, int row_lo, int row_hi, bool any_lmax)
 {
     if (L.kspace || L.uniform || L.h2mode != MCMB_H2_EXACT || L.kstep != 2) return false;

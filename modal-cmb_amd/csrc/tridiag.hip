@@ -206,9 +206,8 @@ __global__ __launch_bounds__(TRD_ROWT) void trd_row(const double* __restrict__ A
 }
 
 // y = A v on rows j+1.. (the trailing matrix as of the panel's start; v in
-// LDS; four rows per wave at a time, 16-byte loads kept four steps ahead in
-// registers: lda is even, so the
-// columns j+1+peel, j+2+peel of every row (peel = (j+1) & 1) are one aligned
+// LDS; RW rows a wave, 16-byte loads kept four steps ahead in registers: lda
+// is even, so the columns j+1+peel, j+2+peel of every row (peel = (j+1) & 1) are one aligned
 // pair), stored in W_i, v stored as V_j; and the sums c1[p] = V_p^T v,
 // c2[p] = W_p^T v (p < i, lane p of each wave) and y^T v over the
 // workgroups (w = tau (y - V c2 - W c1) + alpha2 v is made final by the next
