@@ -576,14 +576,22 @@ __global__ __launch_bounds__(256) void la_solve_step(const double* __restrict__ 
     load_block<false>(L, n, rb, nb, S);
     __syncthreads();
     if (wave < ng) {
-        double x = lane < nb ? X[(size_t)(g0 + wave) * n + rb + lane] : 0.0;
-        const double inv = 1.0 / S[lane][lane];
-        for (int t = 0; t < OB; ++t) {
-            const int j = UP ? OB - 1 - t : t;
-            const double y = lane_value(x * inv, j);
-            if (UP ? lane < j : lane > j) x -= (UP ? S[j][lane] : S[lane][j]) * y;
-        }
-        const double y = x * inv;
+        const double x0 = lane < nb ? X[(size_t)(g0 + wave) * n + rb + lane] : 0.0;
+        // Quotients by the pivot, rounded once (a product with the reciprocal
+        // alone rounds twice); by the division itself where a pivot is near the
+        // ends of the exponent range or a result is not finite.
+        const double d = S[lane][lane], inv = 1.0 / d;
+        auto solve = [&](double x, auto quotient) {
+            for (int t = 0; t < OB; ++t) {
+                const int j = UP ? OB - 1 - t : t;
+                const double y = lane_value(quotient(x), j);
+                if (UP ? lane < j : lane > j) x -= (UP ? S[j][lane] : S[lane][j]) * y;
+            }
+            return quotient(x);
+        };
+        double y = solve(x0, [&](double a) { return div_by(a, d, inv); });
+        if (!__all(fabs(d) > 1e-280 && fabs(d) < 1e280 && fabs(y) < INFINITY))
+            y = solve(x0, [&](double a) { return a / d; });
         ys[wave][lane] = y;
         if (blockIdx.x == 0 && lane < nb) Y[(size_t)(g0 + wave) * n + rb + lane] = y;
     } else {

@@ -113,6 +113,20 @@ def test_cholesky_solve_block_steps(ctx, n, nrhs):
     assert np.abs(ctx.cholesky_solve(ortho, G @ C) - C).max() < 1e-11
 
 
+@pytest.mark.parametrize("nrhs", [1, 4, 128, 129])
+def test_cholesky_solve_rounds_as_a_division(ctx, nrhs):
+    """With a diagonal factor a solve is two quotients an entry, each rounded
+    once however many right-hand sides there are, also at the ends of the
+    exponent range."""
+    n = 130
+    rng = np.random.default_rng(nrhs)
+    d = rng.uniform(0.5, 2.0, n)
+    d[[3, 70, 100, 129]] = 4e-309, 1.3e-200, 6e307, 1.7e150
+    C = rng.standard_normal((n, nrhs))
+    C[[3, 70, 100, 129]] *= np.array([1e-310, 1e-200, 1e300, 1e120])[:, None]
+    assert np.array_equal(ctx.cholesky_solve(np.diag(d), C), C / d[:, None] / d[:, None])
+
+
 def test_lmax500_gram_orthonormalisation_status(ctx):
     # The lmax-500 Gram (r<=s<=t<10 Legendre modes, weight h^2/C^3) has
     # kappa(D^-1 G D^-1) ~ 1e17 > 1/eps: whether FP64 Cholesky meets a
